@@ -99,6 +99,7 @@ struct WaveLds {
   uint32_t fr_n[kLevels];
   uint32_t fr_cur[kLevels];
   uint32_t own[kWave];          // lane -> owning range, via prefix max
+  unsigned long long tot[2];    // interactions of the wavefront's units so far
   V4 pp[kBuf];                  // x, y, z (relative to the target centre), m
   PcRing<Real> pc;
 };
@@ -764,14 +765,6 @@ __device__ bool traverse(const WalkArgs& a, Lds& L, uint32_t* gfr, const Box6& b
   return true;
 }
 
-// The unit's interaction totals, one atomic pair per wavefront.
-__device__ inline void add_totals(const WalkArgs& a, unsigned long long pp, unsigned long long pc) {
-  if (__lane_id() == 0) {
-    atomicAdd(&a.totals[0], pp);
-    atomicAdd(&a.totals[1], pc);
-  }
-}
-
 __device__ inline double wave_min(double v) {
   for (int o = 32; o > 0; o >>= 1) v = fmin(v, __shfl_xor(v, o));
   return v;
@@ -1095,7 +1088,10 @@ __device__ void walk_group(const WalkArgs& a, Lds& L, uint32_t slot, uint32_t g)
       tot_pc += static_cast<unsigned long long>(n_pc) * size;
     }
   }
-  add_totals(a, tot_pp, tot_pc);
+  if (lane == 0) {
+    L.tot[0] += tot_pp;
+    L.tot[1] += tot_pc;
+  }
 }
 
 // A fixed grid of workgroups (one wavefront each) takes the walk units from
@@ -1106,6 +1102,15 @@ __device__ void walk_group(const WalkArgs& a, Lds& L, uint32_t slot, uint32_t g)
 // free. A wavefront leaves once its queue is past its end, so every
 // wavefront exits. The unit count and the queue heads are on the device
 // (counted and cleared by the step), so the launch needs no host read.
+//
+// Device-scope atomics on one address from many wavefronts queue up behind
+// each other (measured inside this kernel at 65,536 particles: a claim 27,000
+// cycles while all wavefronts start, the unit's two total counters 44,000 to
+// 115,000 cycles when a few thousand small units end in a row, a unit itself
+// 160,000). So a wavefront's first unit is its own place in the queue (the
+// head counts the units after those), and its interaction totals are summed
+// in LDS and added once, when it leaves. Many small systems gain most: 2,000
+// of 1,000 particles in 16-particle units, walk 4.14 -> 2.00 ms.
 template <typename Real, int kWaves, bool kMask, bool kDeep>
 __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(4))) void k_walk(WalkArgs a) {
   __shared__ WaveLds<Real, kShallowFrames, kDeep> lds[kWaves];
@@ -1115,16 +1120,23 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(4))
   const uint32_t x = blockIdx.x & 7u;
   const uint32_t lo = static_cast<uint32_t>(uint64_t(units) * x / 8);
   const uint32_t hi = static_cast<uint32_t>(uint64_t(units) * (x + 1) / 8);
-  for (;;) {
+  auto& L = lds[0];
+  if (__lane_id() == 0) L.tot[0] = L.tot[1] = 0ull;
+  __builtin_amdgcn_wave_barrier();
+  const uint32_t first = gridDim.x >> 3;
+  for (uint32_t k = blockIdx.x >> 3; k < hi - lo;) {
+    walk_group<Real, kMask>(a, L, blockIdx.x, uniform(a.groups[lo + k]));
     // Every lane takes part in the claim (adding 1 for lane 0, 0 for the
     // others) and the unit is read from lane 0's result: no branch on the
     // lane id inside the loop, so all 64 lanes stay together in it (a
     // lane-0-only claim lets the compiler keep the other lanes looping on
     // their own, with a stale claim).
     const uint32_t mine = atomicAdd(&a.misc[kMiscQueue + x], __lane_id() == 0 ? 1u : 0u);
-    const uint32_t k = uniform(__builtin_amdgcn_readlane(mine, 0));
-    if (k >= hi - lo) break;
-    walk_group<Real, kMask>(a, lds[0], blockIdx.x, uniform(a.groups[lo + k]));
+    k = first + uniform(__builtin_amdgcn_readlane(mine, 0));
+  }
+  if (__lane_id() == 0 && (L.tot[0] | L.tot[1]) != 0ull) {
+    atomicAdd(&a.totals[0], L.tot[0]);
+    atomicAdd(&a.totals[1], L.tot[1]);
   }
 }
 
