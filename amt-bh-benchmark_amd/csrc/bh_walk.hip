@@ -52,10 +52,9 @@ namespace bhk {
 
 namespace {
 
-constexpr int kBatch = 48;  // entries evaluated per batch (at most)
+constexpr int kBatch = 48;  // staged entries that make a batch (a batch takes all that are staged)
 constexpr int kBuf = 112;   // staging capacity: kBatch - 1 left over + 64 staged at once
 constexpr int kGroupChunks = kGroupCap / kWave;  // a group's particle slots per lane
-static_assert(kBatch == 48, "the group layouts assume 48-entry batches");
 
 template <typename Real>
 struct Vec4T;
@@ -96,9 +95,6 @@ struct WaveLds {
   static constexpr bool kDeepFrames = kDeep;
   using V4 = typename Vec4T<Real>::T;
   uint32_t fr[F][kWave];  // child ranges: (first << 3) | (count - 1)
-  uint32_t fr_n[kLevels];
-  uint32_t fr_cur[kLevels];
-  uint32_t own[kWave];          // lane -> owning range, via prefix max
   unsigned long long tot[2];    // interactions of the wavefront's units so far
   V4 pp[kBuf];                  // x, y, z (relative to the target centre), m
   PcRing<Real> pc;
@@ -181,39 +177,17 @@ __device__ inline typename Vec4T<Real>::T make_entry(double x, double y, double 
   return v;
 }
 
-// Padding entry: zero mass far away, contributes exactly 0 without NaNs.
-template <typename Real>
-__device__ inline typename Vec4T<Real>::T pad_entry() {
-  return make_entry<Real>(1e18, 1e18, 1e18, 0.0);
-}
-
-// P2P over this lane's C consecutive entries (grouped_ttg.h:137-153),
-// added to the plain partial sums bx, by, bz.
-template <typename Real, bool kMask>
-__device__ inline void eval_pp_part(const typename Vec4T<Real>::T* e, int C, Real tx, Real ty, Real tz, Real eps2,
-                                    Real& bx, Real& by, Real& bz) {
-  using V4 = typename Vec4T<Real>::T;
-#pragma unroll 4
-  for (int k = 0; k < C; ++k) {
-    const V4 q = e[k];
-    const Real dx = q.x - tx, dy = q.y - ty, dz = q.z - tz;
-    const Real r2 = fmaR(dx, dx, fmaR(dy, dy, fmaR(dz, dz, eps2)));
-    Real inv = rsq(r2);
-    if (kMask) inv = r2 > Real(0) ? inv : Real(0);
-    const Real s3 = q.w * inv * inv * inv;
-    bx = fmaR(s3, dx, bx);
-    by = fmaR(s3, dy, by);
-    bz = fmaR(s3, dz, bz);
-  }
-}
-
-// The same, added to the lane's accumulator.
-template <typename Real, bool kMask>
-__device__ inline void eval_pp(const typename Vec4T<Real>::T* e, int C, Real tx, Real ty, Real tz, Real eps2,
-                               Acc<Real>& acc) {
-  Real bx = 0, by = 0, bz = 0;
-  eval_pp_part<Real, kMask>(e, C, tx, ty, tz, eps2, bx, by, bz);
-  acc.add(bx, by, bz);
+// One particle (or monopole) interaction (grouped_ttg.h:137-153).
+template <typename Real, bool kMask, typename V4>
+__device__ inline void pp_term(const V4& q, Real tx, Real ty, Real tz, Real eps2, Real& bx, Real& by, Real& bz) {
+  const Real dx = q.x - tx, dy = q.y - ty, dz = q.z - tz;
+  const Real r2 = fmaR(dx, dx, fmaR(dy, dy, fmaR(dz, dz, eps2)));
+  Real inv = rsq(r2);
+  if (kMask) inv = r2 > Real(0) ? inv : Real(0);
+  const Real s3 = q.w * inv * inv * inv;
+  bx = fmaR(s3, dx, bx);
+  by = fmaR(s3, dy, by);
+  bz = fmaR(s3, dz, bz);
 }
 
 // Monopole + traceless quadrupole of one cell (multipole.h:171-200):
@@ -238,86 +212,72 @@ __device__ inline void p2c_term(const V4& e0, const V4& e1, const V2& e2, Real t
   bz = fmaR(inv5, fmaR(g, dz, -qz), bz);
 }
 
-// P2C over this lane's C consecutive cells from j0, added to the plain
-// partial sums bx, by, bz.
-template <typename Real>
-__device__ inline void eval_pc_part(const PcRing<Real>& r, int j0, int C, Real tx, Real ty, Real tz, Real eps2, Real& bx,
-                                    Real& by, Real& bz) {
-#pragma unroll 2
-  for (int k = 0; k < C; ++k) p2c_term(r.a[j0 + k], r.b[j0 + k], r.c[j0 + k], tx, ty, tz, eps2, bx, by, bz);
-}
-
-// The same, added to the lane's accumulator.
-template <typename Real>
-__device__ inline void eval_pc(const PcRing<Real>& r, int j0, int C, Real tx, Real ty, Real tz, Real eps2,
-                               Acc<Real>& acc) {
-  Real bx = 0, by = 0, bz = 0;
-  eval_pc_part<Real>(r, j0, C, tx, ty, tz, eps2, bx, by, bz);
-  acc.add(bx, by, bz);
-}
-
-// Group-phase P2P / P2C: every lane holds NC (<= 2) particles of the group
-// and takes the C entries at e (the same entries for both).
-template <typename Real, bool kMask, int NC>
-__device__ inline void eval_pp_group(const typename Vec4T<Real>::T* e, int C, const Real* gx, const Real* gy,
-                                     const Real* gz, Real eps2, Acc<Real>* acc) {
-  using V4 = typename Vec4T<Real>::T;
-  Real bx[NC], by[NC], bz[NC];
-#pragma unroll
-  for (int k = 0; k < NC; ++k) bx[k] = by[k] = bz[k] = 0;
-#pragma unroll 2
-  for (int j = 0; j < C; ++j) {
-    const V4 q = e[j];
-#pragma unroll
-    for (int k = 0; k < NC; ++k) {
-      const Real dx = q.x - gx[k], dy = q.y - gy[k], dz = q.z - gz[k];
-      const Real r2 = fmaR(dx, dx, fmaR(dy, dy, fmaR(dz, dz, eps2)));
-      Real inv = rsq(r2);
-      if (kMask) inv = r2 > Real(0) ? inv : Real(0);
-      const Real s3 = q.w * inv * inv * inv;
-      bx[k] = fmaR(s3, dx, bx[k]);
-      by[k] = fmaR(s3, dy, by[k]);
-      bz[k] = fmaR(s3, dz, bz[k]);
-    }
+// How a batch of n entries is shared by S slices: slice s takes q or q + 1
+// consecutive entries, the first n - q S slices the longer share. No entry
+// is padding, and only the last round of the longer shares is divergent.
+struct Share {
+  uint32_t slices, inv;  // inv = ceil(2^16 / slices): n * inv >> 16 = n / slices for n <= kBuf
+  uint32_t s;            // this lane's slice
+  __device__ inline void setup(uint32_t S, uint32_t slice) {
+    slices = S;
+    inv = (65536u + S - 1) / S;
+    s = slice;
   }
-#pragma unroll
-  for (int k = 0; k < NC; ++k) acc[k].add(bx[k], by[k], bz[k]);
-}
+  __device__ inline void of(uint32_t n, int* q, int* first, bool* more) const {
+    const uint32_t w = (n * inv) >> 16, r = n - w * slices;
+    *q = static_cast<int>(w);
+    *first = static_cast<int>(s * w + (s < r ? s : r));
+    *more = s < r;
+  }
+};
 
-template <typename Real, int NC>
-__device__ inline void eval_pc_group(const PcRing<Real>& r, int j0, int C, const Real* gx, const Real* gy,
-                                     const Real* gz, Real eps2, Acc<Real>* acc) {
-  using V4 = typename Vec4T<Real>::T;
-  using V2 = typename Vec2T<Real>::T;
-  Real bx[NC], by[NC], bz[NC];
+// Entries [j0, j0 + n) of a batch for the NC particles of this lane, added to
+// the plain partial sums.
+template <typename Real, bool kMask, int NC>
+__device__ inline void eval_pp(const typename Vec4T<Real>::T* e, int n, const Real* gx, const Real* gy, const Real* gz,
+                               Real eps2, Real* bx, Real* by, Real* bz) {
+  constexpr int kU = NC == 1 ? 4 : 2;
+#pragma unroll kU
+  for (int j = 0; j < n; ++j) {
+    const auto q = e[j];
 #pragma unroll
-  for (int k = 0; k < NC; ++k) bx[k] = by[k] = bz[k] = 0;
-  for (int k2 = 0; k2 < C; ++k2) {
-    const V4 e0 = r.a[j0 + k2];
-    const V4 e1 = r.b[j0 + k2];
-    const V2 e2 = r.c[j0 + k2];
+    for (int k = 0; k < NC; ++k) pp_term<Real, kMask>(q, gx[k], gy[k], gz[k], eps2, bx[k], by[k], bz[k]);
+  }
+}
+template <typename Real, int NC>
+__device__ inline void eval_pc(const PcRing<Real>& r, int j0, int n, const Real* gx, const Real* gy, const Real* gz,
+                               Real eps2, Real* bx, Real* by, Real* bz) {
+  constexpr int kU = NC == 1 && sizeof(Real) == 4 ? 2 : 1;
+#pragma unroll kU
+  for (int j = 0; j < n; ++j) {
+    const auto e0 = r.a[j0 + j];
+    const auto e1 = r.b[j0 + j];
+    const auto e2 = r.c[j0 + j];
 #pragma unroll
     for (int k = 0; k < NC; ++k) p2c_term(e0, e1, e2, gx[k], gy[k], gz[k], eps2, bx[k], by[k], bz[k]);
   }
-#pragma unroll
-  for (int k = 0; k < NC; ++k) acc[k].add(bx[k], by[k], bz[k]);
 }
 
-// Evaluator of a target's particles: lane = (particle p, slice s), batches
-// of B = S * C entries, slice s takes entries [s*C, (s+1)*C). Batches are
-// summed in plain FP32 and folded into the lane's FP64 accumulator once it
-// has summed kFoldEntries entries since the last fold (two full
-// single-slice batches; small targets have many slices and short per-lane
-// batches, so they fold after more batches).
+// Evaluator of a target's particles: lane = (particle p, slice s). Batches
+// are summed in walk precision and folded into the lane's FP64 accumulator
+// before it has summed more than kFoldEntries entries.
+//
+// Small targets are bound by latency, not by issue: with 9 particles and 7
+// slices a 48-entry batch is 7 entries per lane, and moving the left-over
+// entries of the ring to its front took as long as evaluating them. So a
+// batch takes everything that is staged (48 to 111 entries: fewer batches,
+// no move), at any split into slices (Share). 65,536 particles in
+// 16-particle units, walk 0.282 -> 0.268 ms; 1M uniform 1.58 -> 1.50.
 template <typename Real, bool kMask>
 struct TargetEval {
   using V4 = typename Vec4T<Real>::T;
   static constexpr int kFoldEntries = 2 * kBatch;
+  // a batch takes all that is staged
+  static constexpr bool kTakesAll = true;
+  __device__ static inline uint32_t take(uint32_t n) { return n; }
   Real tx, ty, tz, eps2;
-  int S, C, s;  // slices, entries per slice and batch, this lane's slice
+  Share sh;
   bool active;
-  uint32_t B;
-  int fold_every = 1;  // batches between folds: max(1, kFoldEntries / C)
   int pending = 0;
   Real px = 0, py = 0, pz = 0;
   Acc<Real> acc;
@@ -326,152 +286,171 @@ struct TargetEval {
     px = py = pz = 0;
     pending = 0;
   }
-  // The last, partial batch of n entries (padded to B): each slice takes
-  // ceil(n / S) entries; restore() returns to full batches.
-  __device__ inline void last_batch(uint32_t n) { C = (static_cast<int>(n) + S - 1) / S; }
-  __device__ inline void restore() { C = static_cast<int>(B) / S; }
-  __device__ inline void pp(const V4* ring) {
-    if (active) eval_pp_part<Real, kMask>(&ring[s * C], C, tx, ty, tz, eps2, px, py, pz);
-    if (++pending >= fold_every) fold();
+  __device__ inline void count(int q) {
+    pending += q + 1;
+    if (pending > kFoldEntries) {
+      fold();
+      pending = q + 1;
+    }
   }
-  __device__ inline void pc(const PcRing<Real>& ring) {
-    if (active) eval_pc_part<Real>(ring, s * C, C, tx, ty, tz, eps2, px, py, pz);
-    if (++pending >= fold_every) fold();
+  __device__ inline void pp(const V4* ring, uint32_t n) {
+    int q, j0;
+    bool more;
+    sh.of(n, &q, &j0, &more);
+    count(q);
+    if (active) {
+      eval_pp<Real, kMask, 1>(ring + j0, q, &tx, &ty, &tz, eps2, &px, &py, &pz);
+      if (more) pp_term<Real, kMask>(ring[j0 + q], tx, ty, tz, eps2, px, py, pz);
+    }
+  }
+  __device__ inline void pc(const PcRing<Real>& r, uint32_t n) {
+    int q, j0;
+    bool more;
+    sh.of(n, &q, &j0, &more);
+    count(q);
+    if (active) {
+      eval_pc<Real, 1>(r, j0, q, &tx, &ty, &tz, eps2, &px, &py, &pz);
+      if (more) p2c_term(r.a[j0 + q], r.b[j0 + q], r.c[j0 + q], tx, ty, tz, eps2, px, py, pz);
+    }
   }
 };
 
-// Evaluator of a whole group (G <= 128 particles, batches of kBatch
-// entries). Each lane has two particle slots; slot k of lane l holds
-// particle base_k + l % P_k and takes slice l / P_k of S_k slices (C_k =
-// kBatch / S_k consecutive entries of each batch). Layouts, by G:
-//   G <= 42      two slots, P = ceil(G / 2), S = the largest divisor of
-//                kBatch with P S <= 64 (one fused loop)
+// Evaluator of a whole group (G <= 128 particles). Each lane has two
+// particle slots; slot k of lane l holds particle base_k + l % P_k and takes
+// slice l / P_k of S_k slices of each batch. Layouts, by G:
+//   G <= 42      two slots, P = ceil(G / 2), S = 64 / P (one fused loop)
 //   43 .. 53     slot 0: particles 0..31 in 2 slices; slot 1: the r = G - 32
-//                others, S_1 = the largest divisor of kBatch with r S_1 <= 64
+//                others, S_1 = 64 / r
 //   54 .. 64     one slot, P = 64, S = 1
 //   65 .. 96     slot 0: particles 0..63, every entry; slot 1: the r = G - 64
-//                others, S_1 = the largest divisor of kBatch with r S_1 <= 64
+//                others, S_1 = 64 / r
 //   97 .. 128    two slots, P = 64, S = 1 (one fused loop)
-// Slices are summed in FP64 at the end.
+// A lane's sum of a batch is folded into FP64 after at most kBatch entries;
+// slices are summed in FP64 at the end. A batch takes whole folds and the
+// rest of the ring moves to its front: the move is small beside 48 entries
+// for up to 128 particles, and odd batches would cost a second, short fold
+// each (64 systems of 65,536 at target size 96: 8.42 ms against 8.11).
 template <typename Real, bool kMask>
 struct GroupEval {
   using V4 = typename Vec4T<Real>::T;
+  // a batch takes whole folds
+  static constexpr bool kTakesAll = false;
+  __device__ static inline uint32_t take(uint32_t n) { return n / kBatch * kBatch; }
   Real gx[kGroupChunks], gy[kGroupChunks], gz[kGroupChunks], eps2;
   int nc;          // slots in the fused loop (1 or 2)
-  int c0, o0;      // fused loop: entries [o0, o0 + c0) of each batch
-  int c1, o1;      // tail slot 1 (c1 > 0): entries [o1, o1 + c1)
-  uint32_t sl0 = 0, sl1 = 0;  // this lane's slices
-  bool tail_on;    // this lane's tail slot holds a particle
-  uint32_t base[kGroupChunks], rows[kGroupChunks], slices[kGroupChunks];
-  uint32_t B;
+  bool tail;       // slot 1 has a loop of its own
+  bool on0, on1;   // this lane's slots hold a slice
+  Share sh0, sh1;
+  uint32_t base1, rows0, rows1;
   Acc<Real> acc[kGroupChunks];
 
   __device__ inline void setup(uint32_t G, int lane) {
     const uint32_t l = static_cast<uint32_t>(lane);
-    c1 = 0;
-    o1 = 0;
-    tail_on = false;
-    constexpr uint32_t kDiv[9] = {48u, 24u, 16u, 12u, 8u, 6u, 4u, 3u, 2u};  // divisors of kBatch
+    tail = false;
+    uint32_t S0 = 1, S1 = 1;
     if (G <= 42) {
-      const uint32_t P = (G + 1) / 2;
-      uint32_t S = 1;
-#pragma unroll
-      for (int q = 0; q < 9; ++q)
-        if (S == 1 && kDiv[q] * P <= static_cast<uint32_t>(kWave)) S = kDiv[q];
+      rows0 = rows1 = base1 = (G + 1) / 2;
+      S0 = S1 = kWave / rows0;
       nc = 2;
-      base[0] = 0;
-      base[1] = P;
-      rows[0] = rows[1] = P;
-      slices[0] = slices[1] = S;
     } else if (G <= 53) {
-      // particles 0..31 in two slices, the other r = G - 32 in S1 slices
-      const uint32_t r = G - 32;
-      uint32_t S1 = 1;
-#pragma unroll
-      for (int q = 0; q < 9; ++q)
-        if (S1 == 1 && kDiv[q] * r <= static_cast<uint32_t>(kWave)) S1 = kDiv[q];
       nc = 1;
-      base[0] = 0;
-      base[1] = 32;
-      rows[0] = 32;
-      rows[1] = r;
-      slices[0] = 2;
-      slices[1] = S1;
-      c1 = kBatch / static_cast<int>(S1);
-      sl1 = l / r < S1 ? l / r : S1 - 1;
-      o1 = static_cast<int>(sl1) * c1;
-      tail_on = l < r * S1;
+      tail = true;
+      rows0 = base1 = 32;
+      S0 = 2;
+      rows1 = G - 32;
+      S1 = kWave / rows1;
     } else if (G <= 64) {
       nc = 1;
-      base[0] = base[1] = 0;
-      rows[0] = rows[1] = kWave;
-      slices[0] = slices[1] = 1;
+      rows0 = rows1 = kWave;
+      base1 = 0;
     } else if (G <= 96) {
-      const uint32_t r = G - kWave;
-      uint32_t S1 = 1;
-#pragma unroll
-      for (int q = 0; q < 9; ++q)
-        if (S1 == 1 && kDiv[q] * r <= static_cast<uint32_t>(kWave)) S1 = kDiv[q];
       nc = 1;
-      base[0] = 0;
-      base[1] = kWave;
-      rows[0] = kWave;
-      rows[1] = r;
-      slices[0] = 1;
-      slices[1] = S1;
-      c1 = kBatch / static_cast<int>(S1);
-      sl1 = l / r < S1 ? l / r : S1 - 1;
-      o1 = static_cast<int>(sl1) * c1;
-      tail_on = l < r * S1;
+      tail = true;
+      rows0 = base1 = kWave;
+      rows1 = G - kWave;
+      S1 = kWave / rows1;
     } else {
       nc = 2;
-      base[0] = 0;
-      base[1] = kWave;
-      rows[0] = rows[1] = kWave;
-      slices[0] = slices[1] = 1;
+      rows0 = rows1 = base1 = kWave;
     }
-    c0 = kBatch / static_cast<int>(slices[0]);
-    sl0 = l / rows[0] < slices[0] ? l / rows[0] : slices[0] - 1;
-    o0 = static_cast<int>(sl0) * c0;
-    B = kBatch;
-  }
-  // The last, partial batch of n entries (padded to B): each slice takes
-  // ceil(n / S) entries; restore() returns to full batches.
-  __device__ inline void last_batch(uint32_t n) {
-    c0 = static_cast<int>((n + slices[0] - 1) / slices[0]);
-    o0 = static_cast<int>(sl0) * c0;
-    if (c1 > 0) {
-      c1 = static_cast<int>((n + slices[1] - 1) / slices[1]);
-      o1 = static_cast<int>(sl1) * c1;
-    }
-  }
-  __device__ inline void restore() {
-    c0 = kBatch / static_cast<int>(slices[0]);
-    o0 = static_cast<int>(sl0) * c0;
-    if (c1 > 0) {
-      c1 = kBatch / static_cast<int>(slices[1]);
-      o1 = static_cast<int>(sl1) * c1;
-    }
+    sh0.setup(S0, l / rows0);
+    sh1.setup(S1, l / rows1);
+    on0 = sh0.s < S0;
+    on1 = sh1.s < S1;
   }
   // the particle (index within the group, clamped to it) of slot k
   __device__ inline uint32_t particle(int k, int lane, uint32_t G) const {
-    const uint32_t i = base[k] + static_cast<uint32_t>(lane) % rows[k];
+    const uint32_t i = (k ? base1 : 0u) + static_cast<uint32_t>(lane) % (k ? rows1 : rows0);
     return i < G ? i : G - 1;
   }
-  __device__ inline void pp(const V4* ring) {
+  template <int NC, int K0>
+  __device__ inline void pp_slots(const V4* ring, const Share& sh, uint32_t n) {
+    int q, j0;
+    bool more;
+    sh.of(n, &q, &j0, &more);
+    Real bx[NC], by[NC], bz[NC];
+    for (;;) {
+      const int c = q < kBatch ? q : kBatch;
+#pragma unroll
+      for (int k = 0; k < NC; ++k) bx[k] = by[k] = bz[k] = 0;
+      eval_pp<Real, kMask, NC>(ring + j0, c, gx + K0, gy + K0, gz + K0, eps2, bx, by, bz);
+      q -= c;
+      j0 += c;
+      if (q == 0) break;
+#pragma unroll
+      for (int k = 0; k < NC; ++k) acc[K0 + k].add(bx[k], by[k], bz[k]);
+    }
+    if (more) {
+      const V4 e = ring[j0];
+#pragma unroll
+      for (int k = 0; k < NC; ++k)
+        pp_term<Real, kMask>(e, gx[K0 + k], gy[K0 + k], gz[K0 + k], eps2, bx[k], by[k], bz[k]);
+    }
+#pragma unroll
+    for (int k = 0; k < NC; ++k) acc[K0 + k].add(bx[k], by[k], bz[k]);
+  }
+  template <int NC, int K0>
+  __device__ inline void pc_slots(const PcRing<Real>& r, const Share& sh, uint32_t n) {
+    int q, j0;
+    bool more;
+    sh.of(n, &q, &j0, &more);
+    Real bx[NC], by[NC], bz[NC];
+    for (;;) {
+      const int c = q < kBatch ? q : kBatch;
+#pragma unroll
+      for (int k = 0; k < NC; ++k) bx[k] = by[k] = bz[k] = 0;
+      eval_pc<Real, NC>(r, j0, c, gx + K0, gy + K0, gz + K0, eps2, bx, by, bz);
+      q -= c;
+      j0 += c;
+      if (q == 0) break;
+#pragma unroll
+      for (int k = 0; k < NC; ++k) acc[K0 + k].add(bx[k], by[k], bz[k]);
+    }
+    if (more) {
+      const auto e0 = r.a[j0];
+      const auto e1 = r.b[j0];
+      const auto e2 = r.c[j0];
+#pragma unroll
+      for (int k = 0; k < NC; ++k)
+        p2c_term(e0, e1, e2, gx[K0 + k], gy[K0 + k], gz[K0 + k], eps2, bx[k], by[k], bz[k]);
+    }
+#pragma unroll
+    for (int k = 0; k < NC; ++k) acc[K0 + k].add(bx[k], by[k], bz[k]);
+  }
+  __device__ inline void pp(const V4* ring, uint32_t n) {
     if (nc == 2) {
-      eval_pp_group<Real, kMask, 2>(ring + o0, c0, gx, gy, gz, eps2, acc);
+      if (on0) pp_slots<2, 0>(ring, sh0, n);
     } else {
-      eval_pp_group<Real, kMask, 1>(ring + o0, c0, gx, gy, gz, eps2, acc);
-      if (c1 > 0 && tail_on) eval_pp<Real, kMask>(ring + o1, c1, gx[1], gy[1], gz[1], eps2, acc[1]);
+      if (on0) pp_slots<1, 0>(ring, sh0, n);
+      if (tail && on1) pp_slots<1, 1>(ring, sh1, n);
     }
   }
-  __device__ inline void pc(const PcRing<Real>& ring) {
+  __device__ inline void pc(const PcRing<Real>& r, uint32_t n) {
     if (nc == 2) {
-      eval_pc_group<Real, 2>(ring, o0, c0, gx, gy, gz, eps2, acc);
+      if (on0) pc_slots<2, 0>(r, sh0, n);
     } else {
-      eval_pc_group<Real, 1>(ring, o0, c0, gx, gy, gz, eps2, acc);
-      if (c1 > 0 && tail_on) eval_pc<Real>(ring, o1, c1, gx[1], gy[1], gz[1], eps2, acc[1]);
+      if (on0) pc_slots<1, 0>(r, sh0, n);
+      if (tail && on1) pc_slots<1, 1>(r, sh1, n);
     }
   }
 };
@@ -480,7 +459,8 @@ struct GroupEval {
 // the node ranges `start` (global, packed (first << 3) | (count - 1)), or
 // from the system's root when start is null. Accepted nodes and the
 // particles of opened leaves are staged in the rings relative to (cx, cy,
-// cz) and handed to ev in batches of ev.B; the last partial batch is padded.
+// cz) and handed to ev in batches of kBatch to kBuf - 1 entries (fewer at the
+// end).
 //
 // kGroup: a group's walk (grouped_ttg.h:259-276 at the group node): a node
 // that is neither accepted nor rejected for every box inside
@@ -492,11 +472,9 @@ __device__ bool traverse(const WalkArgs& a, Lds& L, uint32_t* gfr, const Box6& b
                          Eval& ev, uint32_t& n_pp, uint32_t& n_pc, uint32_t* dl, uint32_t& n_def) {
   constexpr int F = Lds::kFrames;
   constexpr int kStack = Lds::kDeepFrames ? kLevels : F;
-  using V4 = typename Vec4T<Real>::T;
   const int lane = __lane_id();
   const uint64_t lt = lanemask_lt();
   const uint32_t last_node = a.n_nodes - 1, last_part = a.n_parts - 1;
-  const uint32_t B = ev.B;
   const double blo0 = uniform_d(box.v[0]), blo1 = uniform_d(box.v[1]), blo2 = uniform_d(box.v[2]);
   const double bhi0 = uniform_d(box.v[3]), bhi1 = uniform_d(box.v[4]), bhi2 = uniform_d(box.v[5]);
   cx = uniform_d(cx);
@@ -506,52 +484,50 @@ __device__ bool traverse(const WalkArgs& a, Lds& L, uint32_t* gfr, const Box6& b
   uint32_t pp_cnt = 0, pc_cnt = 0;
   bool ok = true;
 
-  // Evaluate the first B staged entries, then move the rest (< 64: at most
-  // B - 1 + 64 were staged) to the front; callers repeat while >= B remain.
-  auto flush_pp = [&]() {
+  // Evaluate the first n staged entries and move the rest (fewer than
+  // kBatch) to the front.
+  auto flush_pp = [&](uint32_t n) {
     __builtin_amdgcn_wave_barrier();
-    ev.pp(L.pp);
-    __builtin_amdgcn_wave_barrier();
-    const uint32_t rest = pp_cnt - B;
-    V4 v;
-    if (static_cast<uint32_t>(lane) < rest) v = L.pp[B + lane];
-    __builtin_amdgcn_wave_barrier();
-    if (static_cast<uint32_t>(lane) < rest) L.pp[lane] = v;
-    pp_cnt = rest;
+    ev.pp(L.pp, n);
+    pp_cnt -= n;
+    if (!Eval::kTakesAll && pp_cnt) {
+      typename Vec4T<Real>::T v;
+      if (static_cast<uint32_t>(lane) < pp_cnt) v = L.pp[n + lane];
+      __builtin_amdgcn_wave_barrier();
+      if (static_cast<uint32_t>(lane) < pp_cnt) L.pp[lane] = v;
+    }
     __builtin_amdgcn_wave_barrier();
   };
-  auto flush_pc = [&]() {
+  auto flush_pc = [&](uint32_t n) {
     __builtin_amdgcn_wave_barrier();
-    ev.pc(L.pc);
-    __builtin_amdgcn_wave_barrier();
-    const uint32_t rest = pc_cnt - B;
-    V4 v0, v1;
-    typename Vec2T<Real>::T v2;
-    if (static_cast<uint32_t>(lane) < rest) {
-      v0 = L.pc.a[B + lane];
-      v1 = L.pc.b[B + lane];
-      v2 = L.pc.c[B + lane];
+    ev.pc(L.pc, n);
+    pc_cnt -= n;
+    if (!Eval::kTakesAll && pc_cnt) {
+      typename Vec4T<Real>::T v0, v1;
+      typename Vec2T<Real>::T v2;
+      if (static_cast<uint32_t>(lane) < pc_cnt) {
+        v0 = L.pc.a[n + lane];
+        v1 = L.pc.b[n + lane];
+        v2 = L.pc.c[n + lane];
+      }
+      __builtin_amdgcn_wave_barrier();
+      if (static_cast<uint32_t>(lane) < pc_cnt) {
+        L.pc.a[lane] = v0;
+        L.pc.b[lane] = v1;
+        L.pc.c[lane] = v2;
+      }
     }
-    __builtin_amdgcn_wave_barrier();
-    if (static_cast<uint32_t>(lane) < rest) {
-      L.pc.a[lane] = v0;
-      L.pc.b[lane] = v1;
-      L.pc.c[lane] = v2;
-    }
-    pc_cnt = rest;
     __builtin_amdgcn_wave_barrier();
   };
 
-  if (lane == 0) {
-    L.fr[0][0] = sys_id << 3;  // the system's root: node sys_id, one node
-    L.fr_n[0] = start ? n_start : 1u;
-    L.fr_cur[0] = 0;
-  }
+  // lane d: ranges of frame d, and the next of them to pop
+  uint32_t fr_n = start ? n_start : 1u, fr_cur = 0;
+  if (lane == 0) L.fr[0][0] = sys_id << 3;  // the system's root: node sys_id, one node
   __builtin_amdgcn_wave_barrier();
   int depth = 0;
   while (depth >= 0) {
-    const uint32_t nr = uniform(L.fr_n[depth]);
-    const uint32_t cur = uniform(L.fr_cur[depth]);
+    const uint32_t nr = __builtin_amdgcn_readlane(fr_n, depth);
+    const uint32_t cur = __builtin_amdgcn_readlane(fr_cur, depth);
     if (cur >= nr) {
       --depth;
       continue;
@@ -568,8 +544,7 @@ __device__ bool traverse(const WalkArgs& a, Lds& L, uint32_t* gfr, const Box6& b
       // a deferred list: single nodes in walk order, one per lane
       node = rv ? (start[rr] >> 3) : 0u;
       total = nr - cur < kWave ? nr - cur : kWave;
-      if (lane == 0) L.fr_cur[0] = cur + total;
-      __builtin_amdgcn_wave_barrier();
+      if (lane == 0) fr_cur = cur + total;
     } else {
       uint32_t packed = 0u;
       if constexpr (Lds::kDeepFrames) {
@@ -584,14 +559,12 @@ __device__ bool traverse(const WalkArgs& a, Lds& L, uint32_t* gfr, const Box6& b
       const int k = __popcll(__ballot(taken));
       total = uniform(__builtin_amdgcn_readlane(incl, k - 1));
       const uint32_t excl = incl - rcnt;
-      L.own[lane] = 0u;
-      __builtin_amdgcn_wave_barrier();
-      if (taken) L.own[excl] = static_cast<uint32_t>(lane);
-      if (lane == 0) L.fr_cur[depth] = cur + k;
-      __builtin_amdgcn_wave_barrier();
-      const int j = static_cast<int>(wave_incl_max(L.own[lane]));
-      node = static_cast<uint32_t>(__shfl(static_cast<int>(rfirst), j)) +
-             (static_cast<uint32_t>(lane) - static_cast<uint32_t>(__shfl(static_cast<int>(excl), j)));
+      // each taken range sends its index to its first slot; the other lanes
+      // send range 0's, 0, to slot 0
+      const int own = __builtin_amdgcn_ds_permute(taken ? static_cast<int>(excl << 2) : 0, taken ? lane : 0);
+      if (lane == depth) fr_cur = cur + k;
+      const int j = static_cast<int>(wave_incl_max(static_cast<uint32_t>(own)));
+      node = static_cast<uint32_t>(__shfl(static_cast<int>(rfirst - excl), j)) + static_cast<uint32_t>(lane);
     }
     const bool nv = static_cast<uint32_t>(lane) < total;
     // MAC in FP64, reference operation order (multipole.h:130-160). Every
@@ -667,9 +640,9 @@ __device__ bool traverse(const WalkArgs& a, Lds& L, uint32_t* gfr, const Box6& b
       } else {
         if (openf) L.fr[depth + 1][pos] = (lfirst << 3) | (lcnt - 1u);
       }
-      if (lane == 0) {
-        L.fr_n[depth + 1] = __popcll(om);
-        L.fr_cur[depth + 1] = 0;
+      if (lane == depth + 1) {
+        fr_n = __popcll(om);
+        fr_cur = 0;
       }
     }
     // accepted nodes
@@ -694,7 +667,7 @@ __device__ bool traverse(const WalkArgs& a, Lds& L, uint32_t* gfr, const Box6& b
         }
         pc_cnt += nc;
         n_pc += nc;
-        while (pc_cnt >= B) flush_pc();
+        if (pc_cnt >= kBatch) flush_pc(Eval::take(pc_cnt));
       } else {
         if (cellf) {
           const double m = sizeof(Real) == 4 ? static_cast<double>(__uint_as_float(rw2.z)) : a.q64[8 * nd];
@@ -702,7 +675,7 @@ __device__ bool traverse(const WalkArgs& a, Lds& L, uint32_t* gfr, const Box6& b
         }
         pp_cnt += nc;
         n_pp += nc;
-        while (pp_cnt >= B) flush_pp();
+        if (pp_cnt >= kBatch) flush_pp(Eval::take(pp_cnt));
       }
     }
     // particles of opened leaves, mapped to slots like the nodes: the lane
@@ -717,14 +690,13 @@ __device__ bool traverse(const WalkArgs& a, Lds& L, uint32_t* gfr, const Box6& b
         // the leaf holding slot b: the last leaf lane starting at or before it
         const uint64_t before = __ballot(leaff && lexcl <= b);
         const int j0 = 63 - __clzll(static_cast<long long>(before));
-        L.own[lane] = static_cast<uint32_t>(j0);
-        __builtin_amdgcn_wave_barrier();
-        if (leaff && lexcl > b && lexcl < b + kWave) L.own[lexcl - b] = static_cast<uint32_t>(lane);
-        __builtin_amdgcn_wave_barrier();
         const uint32_t e = b + lane;
-        const int jj = static_cast<int>(wave_incl_max(L.own[lane]));
-        uint32_t q = static_cast<uint32_t>(__shfl(static_cast<int>(lfirst), jj)) +
-                     (e - static_cast<uint32_t>(__shfl(static_cast<int>(lexcl), jj)));
+        // each leaf that starts in this chunk sends its lane to its first
+        // slot; the other lanes send j0 to slot 0
+        const bool here = leaff && lexcl > b && lexcl < b + kWave;
+        const int own = __builtin_amdgcn_ds_permute(here ? static_cast<int>((lexcl - b) << 2) : 0, here ? lane : j0);
+        const int jj = static_cast<int>(wave_incl_max(static_cast<uint32_t>(own)));
+        uint32_t q = static_cast<uint32_t>(__shfl(static_cast<int>(lfirst - lexcl), jj)) + e;
         q = q < last_part ? q : last_part;
         const uint32_t chunk = ltot - b < kWave ? ltot - b : kWave;
         if (e < ltot) {
@@ -733,34 +705,16 @@ __device__ bool traverse(const WalkArgs& a, Lds& L, uint32_t* gfr, const Box6& b
         }
         pp_cnt += chunk;
         n_pp += chunk;
-        while (pp_cnt >= B) flush_pp();
+        if (pp_cnt >= kBatch) flush_pp(Eval::take(pp_cnt));
       }
     }
     __builtin_amdgcn_wave_barrier();
     if (om) ++depth;
   }
   if (!ok) return false;
-  // final partial batches (fewer than B entries), padded to B; each slice
-  // evaluates only its share of the entries actually staged
-  if (pp_cnt) {
-    if (static_cast<uint32_t>(lane) >= pp_cnt && static_cast<uint32_t>(lane) < B) L.pp[lane] = pad_entry<Real>();
-    ev.last_batch(pp_cnt);
-    pp_cnt = B;
-    flush_pp();
-    ev.restore();
-  }
-  if (pc_cnt) {
-    if (static_cast<uint32_t>(lane) >= pc_cnt && static_cast<uint32_t>(lane) < B) {
-      L.pc.a[lane] = pad_entry<Real>();
-      L.pc.b[lane] = make_entry<Real>(0.0, 0.0, 0.0, 0.0);
-      L.pc.c[lane].x = Real(0);
-      L.pc.c[lane].y = Real(0);
-    }
-    ev.last_batch(pc_cnt);
-    pc_cnt = B;
-    flush_pc();
-    ev.restore();
-  }
+  // the last, smaller batches
+  if (pp_cnt) flush_pp(pp_cnt);
+  if (pc_cnt) flush_pc(pc_cnt);
   __builtin_amdgcn_wave_barrier();
   return true;
 }
@@ -885,15 +839,11 @@ __device__ void walk_target(const WalkArgs& a, Lds& L, uint32_t* gfr, uint32_t t
 
   for (uint32_t c0 = 0; c0 < T; c0 += kWave) {
     const uint32_t tc = T - c0 < kWave ? T - c0 : kWave;
-    const int S = kWave / static_cast<int>(tc) < kBatch ? kWave / static_cast<int>(tc) : kBatch;
+    const int S = kWave / static_cast<int>(tc);
     TargetEval<Real, kMask> ev;
-    ev.S = S;
-    ev.C = kBatch / S;
-    ev.B = static_cast<uint32_t>(S * ev.C);
-    ev.fold_every = ev.C >= TargetEval<Real, kMask>::kFoldEntries ? 1 : TargetEval<Real, kMask>::kFoldEntries / ev.C;
+    ev.sh.setup(static_cast<uint32_t>(S), static_cast<uint32_t>(lane) / tc);
     ev.active = lane < static_cast<int>(tc) * S;
     const int p = lane % static_cast<int>(tc);
-    ev.s = lane / static_cast<int>(tc);
     ev.eps2 = static_cast<Real>(sp.eps2);
     {
       const double4 q = a.posm[tb + c0 + p];
@@ -1051,16 +1001,16 @@ __device__ void walk_group(const WalkArgs& a, Lds& L, uint32_t slot, uint32_t g)
     // P2C ring is free after the walk); the group's are stored for its
     // targets, a target's finish its particles
     double* red = reinterpret_cast<double*>(L.pc.a);  // 3 x 64 doubles
-    const int used = ev.nc == 2 || ev.c1 > 0 ? 2 : 1;
+    const int used = ev.nc == 2 || ev.tail ? 2 : 1;
 #pragma unroll
     for (int k = 0; k < kGroupChunks; ++k) {
       if (k < used) {
-        const uint32_t P = ev.rows[k], S = ev.slices[k];
+        const uint32_t P = k ? ev.rows1 : ev.rows0, S = k ? ev.sh1.slices : ev.sh0.slices;
         red[3 * lane + 0] = ev.acc[k].sx();
         red[3 * lane + 1] = ev.acc[k].sy();
         red[3 * lane + 2] = ev.acc[k].sz();
         __builtin_amdgcn_wave_barrier();
-        const uint32_t i = ev.base[k] + static_cast<uint32_t>(lane);
+        const uint32_t i = (k ? ev.base1 : 0u) + static_cast<uint32_t>(lane);
         if (static_cast<uint32_t>(lane) < P && i < size) {
           double ax = 0.0, ay = 0.0, az = 0.0;
           for (uint32_t s2 = 0; s2 < S; ++s2) {
