@@ -82,7 +82,8 @@ struct Scratch {
   uint16_t* sid = nullptr;
   uint8_t* tables = nullptr;
   TreeDev t{};
-  uint32_t *mark = nullptr, *targets = nullptr, *gmark = nullptr, *groups = nullptr, *unit_n = nullptr;
+  uint32_t *mark = nullptr, *gmark = nullptr, *unit_n = nullptr, *unit_lb = nullptr;
+  uint2* units = nullptr;
   uint32_t *defer = nullptr, *deep_frames = nullptr;
   double* gacc = nullptr;
 };
@@ -159,7 +160,8 @@ struct Ctx {
   DevBuf<double4> posm;
   DevBuf<uint8_t> L, H;
   DevBuf<uint32_t> tcounts, tprefix;
-  DevBuf<uint32_t> mark, targets, gmark, groups, unit_n, defer, deep_frames;
+  DevBuf<uint32_t> mark, gmark, unit_n, unit_lb, defer, deep_frames;
+  DevBuf<uint2> units;
   DevBuf<double> gacc, nbox;
   DevBuf<uint32_t> begin, count, cs, first_child, parent, leaf_idx, leaf_node, leaf_first, level_off;
   DevBuf<uint8_t> depth, leaf, nchild;
@@ -383,7 +385,8 @@ int plan_systems(Ctx* c, const HostSys* sys, uint32_t S, bool no_grow, Plan* p) 
     sd[k].max_leaf = h.max_leaf;
     sd[k].tsm = std::min(h.target_size, h.group_size);
     sd[k].use_quad = h.fp.use_quadrupole != 0;
-    sd[k].tile = h.tile ? h.tile : c->walk_tile;
+    sd[k].tile = static_cast<uint16_t>(h.tile ? h.tile : c->walk_tile);
+    sd[k].piece = kGroupCap;
     first[k] = static_cast<uint32_t>(ci);
     for (uint64_t b = 0; b < h.n; b += kChunk)
       ch[ci++] = make_uint4(k, static_cast<uint32_t>(off + b), static_cast<uint32_t>(off + std::min<uint64_t>(h.n, b + kChunk)), 0);
@@ -468,9 +471,9 @@ int provision(Ctx* c, const Plan& p, Scratch* b) {
   }
   if (p.walk) {
     TRY(ensure(c, c->mark, n, "targets"));
-    TRY(ensure(c, c->targets, n, "targets"));
-    TRY(ensure(c, c->gmark, n, "groups"));
-    TRY(ensure(c, c->groups, n, "groups"));
+    TRY(ensure(c, c->gmark, n, "walk units"));
+    TRY(ensure(c, c->units, n, "walk units"));
+    TRY(ensure(c, c->unit_lb, unit_list_words(n), "walk units"));
     TRY(ensure(c, c->unit_n, m, "walk units"));
     TRY(ensure(c, c->gacc, 3ull * n, "group sums"));
     TRY(ensure(c, c->defer, uint64_t(p.slots) * kDefer, "deferred nodes"));
@@ -520,9 +523,9 @@ int provision(Ctx* c, const Plan& p, Scratch* b) {
   t.cap = m;
   if (p.walk) {
     s.mark = c->mark.p;
-    s.targets = c->targets.p;
     s.gmark = c->gmark.p;
-    s.groups = c->groups.p;
+    s.units = c->units.p;
+    s.unit_lb = c->unit_lb.p;
     s.unit_n = c->unit_n.p;
     s.gacc = c->gacc.p;
     s.defer = c->defer.p;
@@ -567,9 +570,9 @@ bool carve(uint8_t* base, size_t bytes, Plan* p, Scratch* b) {
   s.sid = reinterpret_cast<uint16_t*>(take(2ull * n));
   s.tables = take(p->table_bytes);
   s.mark = reinterpret_cast<uint32_t*>(take(4ull * n));
-  s.targets = reinterpret_cast<uint32_t*>(take(4ull * n));
   s.gmark = reinterpret_cast<uint32_t*>(take(4ull * n));
-  s.groups = reinterpret_cast<uint32_t*>(take(4ull * n));
+  s.units = reinterpret_cast<uint2*>(take(8ull * n));
+  s.unit_lb = s.tcounts;  // the tree's tile counts are free by then
   s.gacc = reinterpret_cast<double*>(take(24ull * n));
   s.defer = reinterpret_cast<uint32_t*>(take(4ull * p->slots * kDefer));
   s.deep_frames = reinterpret_cast<uint32_t*>(take(4ull * p->slots * (kLevels - kShallowFrames) * kWave));
@@ -674,15 +677,31 @@ int enqueue_walk(Ctx* c, const Plan& p, const Scratch& b, bh_particle* parts, do
   const uint32_t n = p.n;
   const SysDev* sys = reinterpret_cast<const SysDev*>(b.tables);
   const bool grouped = c->walk_mode == BH_WALK_GROUPED;
-  // a walk on its own (bh_accel) clears what an earlier walk left
-  HIP_OK(c, launch_fill_u32(b.misc + kMiscIncomplete, 0u, 1, s));
-  HIP_OK(c, launch_fill_u32(b.misc + kMiscQueue, 0u, 8, s));
-  HIP_OK(c, launch_fill_u32(reinterpret_cast<uint32_t*>(b.totals), 0u, 4, s));
-  HIP_OK(c, launch_targets(b.t, n, b.sid, sys, false, b.mark, b.tcounts, b.tprefix, b.targets, b.misc + kMiscTargets,
-                           nullptr, s));
+  // what the unit list and the walk need zeroed, in one launch (a walk on its
+  // own, bh_accel, clears what an earlier walk left)
+  {
+    ZeroRanges z;
+    z.p[0] = b.misc + kMiscIncomplete;
+    z.n[0] = 1;
+    z.p[1] = b.misc + kMiscTargets;
+    z.n[1] = kMiscQueue + 8 - kMiscTargets;  // target and unit counts, queue heads
+    z.p[2] = reinterpret_cast<uint32_t*>(b.totals);
+    z.n[2] = 4;
+    z.p[3] = b.mark;
+    z.n[3] = n;
+    z.p[4] = b.gmark;
+    z.n[4] = n;
+    z.p[5] = b.unit_lb;
+    z.n[5] = unit_list_words(n);
+    if (parts && p.carry_out) {
+      // read by this step's build already (carried_in)
+      z.p[6] = c->carry_flag.p;
+      z.n[6] = 1;
+    }
+    HIP_OK(c, launch_zero(z, s));
+  }
   // per-target mode: the walk units are the targets themselves
-  HIP_OK(c, launch_targets(b.t, n, b.sid, sys, grouped, b.gmark, b.tcounts, b.tprefix, b.groups, b.misc + kMiscGroups,
-                           grouped ? b.unit_n : nullptr, s));
+  HIP_OK(c, launch_units(b.t, n, b.sid, sys, grouped, b.mark, b.gmark, b.unit_n, b.unit_lb, b.units, s));
   if (events) HIP_OK(c, hipEventRecord(c->ev[3], s));
   WalkArgs a;
   a.rec = b.t.rec;
@@ -691,7 +710,7 @@ int enqueue_walk(Ctx* c, const Plan& p, const Scratch& b, bh_particle* parts, do
   a.begin = b.t.begin;
   a.count = b.t.count;
   a.posm = b.posm;
-  a.groups = b.groups;
+  a.units = b.units;
   a.unit_n = grouped ? b.unit_n : nullptr;
   a.tmark = b.mark;
   a.sid = b.sid;
@@ -710,8 +729,6 @@ int enqueue_walk(Ctx* c, const Plan& p, const Scratch& b, bh_particle* parts, do
   a.carry = nullptr;
   a.carry_bad = nullptr;
   if (parts && p.carry_out) {
-    // read by this step's build already (carried_in): cleared for the walk's
-    HIP_OK(c, launch_fill_u32(c->carry_flag.p, 0u, 1, s));
     a.carry = c->carry.p;
     a.carry_bad = c->carry_flag.p;
   }
@@ -1085,9 +1102,9 @@ void bh_ctx_destroy(bh_ctx* h) {
   release(c->tcounts);
   release(c->tprefix);
   release(c->mark);
-  release(c->targets);
   release(c->gmark);
-  release(c->groups);
+  release(c->units);
+  release(c->unit_lb);
   release(c->unit_n);
   release(c->defer);
   release(c->deep_frames);

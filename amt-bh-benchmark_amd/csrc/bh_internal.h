@@ -35,7 +35,8 @@ struct SysDev {
   uint32_t max_leaf;
   uint32_t tsm;      // min(target_size, group_size)
   int32_t use_quad;
-  uint32_t tile;     // walk tile: particles a walk unit holds (kMinTile..kGroupCap)
+  uint16_t tile;     // particles a unit of several targets holds at most (0: every target is a unit)
+  uint16_t piece;    // particles a target's unit holds at most (a wider target is cut into pieces)
 };
 static_assert(sizeof(SysDev) == 64, "SysDev layout");
 
@@ -111,7 +112,7 @@ struct WalkArgs {
   const uint32_t* begin;
   const uint32_t* count;
   const double4* posm;     // x, y, z, m in Morton order
-  const uint32_t* groups;  // walk units (first node of each), Morton order
+  const uint2* units;      // walk units, Morton order: {node, first particle} (a cut target: a unit per piece)
   const uint32_t* unit_n;  // [n_nodes] particles | 1 << 31 of a packed unit at its first node, else 0 (nullable)
   const uint32_t* tmark;   // [n] target node + 1 at each target's first particle, else 0
   const uint16_t* sid;     // system of each particle
@@ -138,9 +139,9 @@ struct WalkArgs {
 // ---- bh_sort.hip
 // Up to kMax device ranges of 32-bit words to zero (unused: n = 0).
 struct ZeroRanges {
-  static constexpr int kMax = 4;
-  uint32_t* p[kMax] = {nullptr, nullptr, nullptr, nullptr};
-  uint64_t n[kMax] = {0, 0, 0, 0};
+  static constexpr int kMax = 8;
+  uint32_t* p[kMax] = {};
+  uint64_t n[kMax] = {};
 };
 hipError_t launch_zero(const ZeroRanges& r, hipStream_t s);
 
@@ -193,15 +194,25 @@ hipError_t launch_tree_emit(const uint8_t* L, const uint8_t* H, uint32_t n, cons
 // bound a level's node count by n_sys * 8^d).
 hipError_t launch_tree_finish(const uint64_t* keys, const double4* posm, uint32_t n, const uint16_t* sid, uint32_t n_sys,
                               const double* lohi, uint32_t depth_plan, TreeDev t, hipStream_t s);
-// Marks (node + 1 at its first particle) and lists the topmost nodes with
-// leaf || count <= thr: thr = the system's tsm (walk targets) or, with
-// groups set, max(tsm, tile) (walk groups; tile = the system's walk tile).
-// With groups and unit_n, runs of sibling single-target groups are packed
-// into walk units of at most tile particles (unit_n per node: particles |
-// 1 << 31 at a unit's first node, else 0).
-hipError_t launch_targets(TreeDev t, uint32_t n, const uint16_t* sid, const SysDev* sys, bool groups, uint32_t* mark,
-                          uint32_t* tile_counts, uint32_t* tile_prefix, uint32_t* targets, uint32_t* n_targets,
-                          uint32_t* unit_n, hipStream_t s);
+// Marks the walk targets (node + 1 at the first particle in tmark; their
+// number is added to misc[kMiscTargets]) and lists the walk units (their
+// number to misc[kMiscGroups]). Targets: topmost nodes with leaf || count <=
+// tsm. Units: with grouped, topmost nodes with leaf || count <= max(tsm,
+// tile), runs of sibling ones that are single targets packed up to tile
+// particles (unit_n per node: particles | 1 << 31 at a packed unit's first
+// node, else 0); otherwise the targets. A unit that is one target of more than
+// `piece` particles is listed once per piece. tmark, gmark, the two counts and
+// the unit_list_words() look-back words must be zero.
+hipError_t launch_units(TreeDev t, uint32_t n, const uint16_t* sid, const SysDev* sys, bool grouped, uint32_t* tmark,
+                        uint32_t* gmark, uint32_t* unit_n, uint32_t* lookback, uint2* units, hipStream_t s);
+inline uint64_t unit_list_words(uint64_t n) { return (n + kTreeTile - 1) / kTreeTile + 1; }
+
+// The first particle of piece j of a target of cnt particles, and what a
+// piece holds (the last one the rest): equal pieces of at most `piece`.
+__host__ __device__ inline uint32_t piece_size(uint32_t cnt, uint32_t piece) {
+  const uint32_t k = (cnt + piece - 1) / piece;
+  return k > 1 ? (cnt + k - 1) / k : cnt;
+}
 
 // ---- bh_walk.hip
 // slots workgroups (a multiple of 8, at most kWalkSlots) take the units from

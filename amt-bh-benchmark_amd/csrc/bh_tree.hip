@@ -614,108 +614,169 @@ __global__ __launch_bounds__(kBlock) void k_upward(int level, TreeDev t) {
   }
 }
 
-// Marks each walk target at its first particle: topmost nodes with
-// leaf || count <= tsm (tsm = min(target_size, group_size), which makes the
-// group-root / target nesting of grouped_ttg.h:251-288 a single predicate).
-// With `groups`, the walk groups instead: topmost nodes with
-// leaf || count <= max(tsm, tile).
-__global__ __launch_bounds__(kBlock) void k_target_mark(TreeDev t, const uint16_t* __restrict__ sid,
-                                                        const SysDev* __restrict__ sys, bool groups,
-                                                        uint32_t* __restrict__ mark) {
-  if (t.misc[kMiscAbort]) return;
-  const uint32_t n_nodes = t.level_off[kLevels];
-  for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n_nodes; i += gridDim.x * kBlock) {
-    const SysDev& q = sys[sid[t.begin[i]]];
-    const uint32_t tsm = groups ? max(q.tsm, q.tile) : q.tsm;
-    const bool pred = t.leaf[i] || t.count[i] <= tsm;
-    if (!pred) continue;
-    const bool ppred = (t.depth[i] != 0) && (t.count[t.parent[i]] <= tsm);
-    if (!ppred) mark[t.begin[i]] = i + 1;
-  }
+// Walk targets and walk units in one pass over the nodes.
+//
+// Targets: topmost nodes with leaf || count <= tsm (tsm = min(target_size,
+// group_size), which makes the group-root / target nesting of
+// grouped_ttg.h:251-288 a single predicate), marked at their first particle.
+//
+// Units, grouped: topmost nodes with leaf || count <= max(tsm, tile), marked
+// by their parent. Below a node with more particles, a run of consecutive
+// children that are single targets (leaf || count <= tsm) is packed greedily
+// into units of at most tile particles; a unit of two or more walks as one
+// group (one shared walk, then its targets), the others keep their own walks.
+// The unit's first child is marked and gets unit_n = particles | 1 << 31, the
+// other members are not marked; every other walk group gets unit_n = 0. Any
+// box holding the targets' boxes gives the same lists (near2 and far2 are
+// monotone in the box), so a unit is exact whatever it groups. Not grouped:
+// every target is a unit.
+//
+// A unit that is a single target of more than `piece` particles is marked at
+// the first particle of each of its pieces: every piece walks the target's
+// list (its box) for its own particles.
+//
+// The phase is bound by launches for all but the largest inputs: marks,
+// packing, counts, scan and lists of targets and units took 15 launches; with
+// the target list that nothing read gone, one zero fill and these two kernels
+// are left (events, 1,000 to 250,000 particles: 42-54 us -> 18-22; 1M: 62 ->
+// 30-39; 4M: 79 -> 60).
+__device__ inline void mark_unit(uint32_t* gmark, uint32_t node, uint32_t begin, uint32_t cnt, bool single,
+                                 uint32_t piece) {
+  const uint32_t len = single ? piece_size(cnt, piece) : cnt;
+  for (uint32_t o = 0; o < cnt; o += len) gmark[begin + o] = node + 1;
 }
 
-// Walk units from the walk groups. Below a node with more than
-// max(tsm, tile) particles (tile: the system's walk tile), a run of
-// consecutive children that are single targets (leaf || count <= tsm) is
-// packed greedily into units of at most tile particles; a unit of two or
-// more walks as one group (one
-// shared walk, then its targets), the others keep their own walks. The
-// unit's first child keeps its mark and gets unit_n = particles | 1 << 31,
-// the other members lose theirs; every other walk group gets unit_n = 0.
-// Any box holding the targets' boxes gives the same lists (near2 and far2
-// are monotone in the box), so a unit is exact whatever it groups.
-__global__ __launch_bounds__(kBlock) void k_group_units(TreeDev t, const uint16_t* __restrict__ sid,
-                                                        const SysDev* __restrict__ sys, uint32_t* __restrict__ mark,
-                                                        uint32_t* __restrict__ unit_n) {
+__global__ __launch_bounds__(kBlock) void k_units_mark(TreeDev t, const uint16_t* __restrict__ sid,
+                                                       const SysDev* __restrict__ sys, bool grouped,
+                                                       uint32_t* __restrict__ tmark, uint32_t* __restrict__ gmark,
+                                                       uint32_t* __restrict__ unit_n) {
+  __shared__ uint32_t s_targets;
   if (t.misc[kMiscAbort]) return;
+  if (threadIdx.x == 0) s_targets = 0;
+  __syncthreads();
   const uint32_t n_nodes = t.level_off[kLevels];
+  uint32_t mine = 0;
   for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n_nodes; i += gridDim.x * kBlock) {
-    const SysDev& q = sys[sid[t.begin[i]]];
-    const uint32_t tsm = q.tsm, tile = q.tile;
+    const uint32_t b = t.begin[i], cnt = t.count[i];
+    const SysDev& q = sys[sid[b]];
+    const uint32_t tsm = q.tsm, tile = q.tile, piece = q.piece;
+    const bool leaf = t.leaf[i] != 0, root = t.depth[i] == 0;
+    const bool single = leaf || cnt <= tsm;
+    if (single && (root || t.count[t.parent[i]] > tsm)) {
+      tmark[b] = i + 1;
+      ++mine;
+      if (!grouped) mark_unit(gmark, i, b, cnt, true, piece);
+    }
+    if (!grouped) continue;
     const uint32_t thr = max(tsm, tile);
-    const bool is_group = t.leaf[i] || t.count[i] <= thr;
-    if (t.depth[i] == 0 && is_group) unit_n[i] = 0u;  // a system that is one walk group
-    if (is_group) continue;
+    if (leaf || cnt <= thr) {
+      if (root) {  // a system that is one walk group
+        unit_n[i] = 0u;
+        mark_unit(gmark, i, b, cnt, single, piece);
+      }
+      continue;
+    }
     const uint32_t fc = t.first_child[i], k = t.nchild[i];
-    uint32_t run = 0, run_len = 0, run_n = 0;
-    for (uint32_t c = fc; c <= fc + k; ++c) {
-      const bool in = c < fc + k;
-      const uint32_t cn = in ? t.count[c] : 0u;
-      const bool single = in && (t.leaf[c] || cn <= tsm) && cn <= tile;
-      if (in && (t.leaf[c] || cn <= thr)) unit_n[c] = 0u;
-      if (single && run_len > 0 && run_n + cn <= tile) {
-        mark[t.begin[c]] = 0u;
+    uint32_t run = 0, run_b = 0, run_len = 0, run_n = 0;
+    auto end_run = [&]() {  // a run is the first child of a unit and what is packed behind it
+      if (run_len == 0) return;
+      unit_n[run] = run_len > 1 ? run_n | 0x80000000u : 0u;
+      mark_unit(gmark, run, run_b, run_n, run_len == 1, piece);
+      run_len = 0;
+    };
+    for (uint32_t c = fc; c < fc + k; ++c) {
+      const uint32_t cn = t.count[c];
+      const bool cleaf = t.leaf[c] != 0;
+      if (!cleaf && cn > thr) {
+        end_run();
+        continue;
+      }
+      const bool csingle = cleaf || cn <= tsm;
+      if (csingle && cn <= tile && run_len > 0 && run_n + cn <= tile) {
         ++run_len;
         run_n += cn;
         continue;
       }
-      if (run_len > 1) unit_n[run] = run_n | 0x80000000u;
-      run_len = single ? 1u : 0u;
-      run = c;
-      run_n = cn;
+      end_run();
+      if (csingle) {
+        run = c;
+        run_b = t.begin[c];
+        run_n = cn;
+        run_len = 1;
+        if (cn > tile) end_run();
+      } else {
+        unit_n[c] = 0u;
+        mark_unit(gmark, c, t.begin[c], cn, false, piece);
+      }
     }
+    end_run();
   }
+  for (int o = 32; o > 0; o >>= 1) mine += __shfl_xor(mine, o);
+  if (__lane_id() == 0 && mine) atomicAdd(&s_targets, mine);
+  __syncthreads();
+  if (threadIdx.x == 0 && s_targets) atomicAdd(&t.misc[kMiscTargets], s_targets);
 }
 
-__global__ __launch_bounds__(kBlock) void k_compact_count(const uint32_t* __restrict__ mark, uint32_t n,
-                                                          uint32_t* __restrict__ tile_counts) {
-  __shared__ uint32_t s;
-  if (threadIdx.x == 0) s = 0;
-  __syncthreads();
-  const uint32_t base = blockIdx.x * kTreeTile;
-  uint32_t c = 0;
-  for (uint32_t e = threadIdx.x; e < kTreeTile; e += kBlock) {
-    const uint32_t i = base + e;
-    if (i < n && mark[i]) ++c;
-  }
-  for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o);
-  if (__lane_id() == 0) atomicAdd(&s, c);
-  __syncthreads();
-  if (threadIdx.x == 0) tile_counts[blockIdx.x] = s;
-}
-
-__global__ __launch_bounds__(kBlock) void k_compact_write(const uint32_t* __restrict__ mark, uint32_t n,
-                                                          const uint32_t* __restrict__ tile_prefix, uint32_t* __restrict__ out) {
+// The marked units in particle order, {node, first particle}, in one pass: a
+// tile's place comes from decoupled look-back over the tiles before it (64 at
+// a time), tiles taken in the order of a counter.
+__global__ __launch_bounds__(kBlock) void k_units_list(const uint32_t* __restrict__ mark, uint32_t n, uint32_t tiles,
+                                                       uint32_t* __restrict__ lookback, uint32_t* __restrict__ n_units,
+                                                       uint2* __restrict__ out) {
   __shared__ uint32_t s_wc[4];
-  const uint32_t base = blockIdx.x * kTreeTile;
+  __shared__ uint32_t s_tile, s_excl;
+  if (threadIdx.x == 0) s_tile = atomicAdd(&lookback[tiles], 1u);
+  __syncthreads();
+  const uint32_t tile = s_tile, base = tile * kTreeTile;
   const int w = threadIdx.x >> 6, lane = __lane_id();
   uint32_t vals[kItems];
-  uint32_t cnt = 0;
 #pragma unroll
   for (int j = 0; j < kItems; ++j) {
     const uint32_t i = base + w * (kTreeTile / 4) + j * 64 + lane;
     vals[j] = i < n ? mark[i] : 0u;
-    cnt += __popcll(__ballot(vals[j] != 0));
   }
+  uint32_t cnt = 0;
+#pragma unroll
+  for (int j = 0; j < kItems; ++j) cnt += __popcll(__ballot(vals[j] != 0));
   if (lane == 0) s_wc[w] = cnt;
   __syncthreads();
-  uint32_t pos = tile_prefix[blockIdx.x];
+  if (w == 0) {
+    const uint32_t total = s_wc[0] + s_wc[1] + s_wc[2] + s_wc[3];
+    uint32_t excl = 0;
+    if (tile > 0) {
+      if (lane == 0)
+        __hip_atomic_store(&lookback[tile], kLbAgg | total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      for (int64_t j = static_cast<int64_t>(tile) - 1;;) {
+        // lane l reads tile j - l: sums back to the nearest inclusive prefix,
+        // once every tile up to it has published
+        const int64_t p = j - lane;
+        const uint32_t val = p >= 0 ? __hip_atomic_load(&lookback[p], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : kLbPre;
+        const uint64_t pre = __ballot((val & ~kLbVal) == kLbPre);
+        const uint64_t none = __ballot((val & ~kLbVal) == 0u);
+        const int stop = pre ? __ffsll(static_cast<long long>(pre)) - 1 : 63;
+        const uint64_t upto = stop == 63 ? ~0ull : (2ull << stop) - 1ull;
+        if (none & upto) continue;
+        uint32_t v = lane <= stop ? val & kLbVal : 0u;
+        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
+        excl += v;
+        if (pre) break;
+        j -= 64;
+      }
+    }
+    if (lane == 0) {
+      __hip_atomic_store(&lookback[tile], kLbPre | (excl + total), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      s_excl = excl;
+      if (tile + 1 == tiles) *n_units = excl + total;
+    }
+  }
+  __syncthreads();
+  uint32_t pos = s_excl;
   for (int k = 0; k < w; ++k) pos += s_wc[k];
   const uint64_t lt = lanemask_lt();
 #pragma unroll
   for (int j = 0; j < kItems; ++j) {
     const uint64_t m = __ballot(vals[j] != 0);
-    if (vals[j]) out[pos + __popcll(m & lt)] = vals[j] - 1;
+    if (vals[j]) out[pos + __popcll(m & lt)] = make_uint2(vals[j] - 1, base + w * (kTreeTile / 4) + j * 64 + lane);
     pos += __popcll(m);
   }
 }
@@ -769,18 +830,13 @@ hipError_t launch_tree_finish(const uint64_t* keys, const double4* posm, uint32_
   return hipGetLastError();
 }
 
-hipError_t launch_targets(TreeDev t, uint32_t n, const uint16_t* sid, const SysDev* sys, bool groups, uint32_t* mark,
-                          uint32_t* tile_counts, uint32_t* tile_prefix, uint32_t* targets, uint32_t* n_targets,
-                          uint32_t* unit_n, hipStream_t s) {
+hipError_t launch_units(TreeDev t, uint32_t n, const uint16_t* sid, const SysDev* sys, bool grouped, uint32_t* tmark,
+                        uint32_t* gmark, uint32_t* unit_n, uint32_t* lookback, uint2* units, hipStream_t s) {
   const uint32_t tiles = (n + kTreeTile - 1) / kTreeTile;
-  hipError_t e = launch_fill_u32(mark, 0u, n, s);
-  if (e != hipSuccess) return e;
-  hipLaunchKernelGGL(k_target_mark, dim3(grid_for(t.cap, 4096)), dim3(kBlock), 0, s, t, sid, sys, groups, mark);
-  if (groups && unit_n)
-    hipLaunchKernelGGL(k_group_units, dim3(grid_for(t.cap, 4096)), dim3(kBlock), 0, s, t, sid, sys, mark, unit_n);
-  hipLaunchKernelGGL(k_compact_count, dim3(tiles), dim3(kBlock), 0, s, mark, n, tile_counts);
-  hipLaunchKernelGGL(k_col_scan, dim3(1), dim3(1024), 0, s, tile_counts, tiles, 1u, tile_prefix, n_targets);
-  hipLaunchKernelGGL(k_compact_write, dim3(tiles), dim3(kBlock), 0, s, mark, n, tile_prefix, targets);
+  hipLaunchKernelGGL(k_units_mark, dim3(grid_for(t.cap, 4096)), dim3(kBlock), 0, s, t, sid, sys, grouped, tmark, gmark,
+                     unit_n);
+  hipLaunchKernelGGL(k_units_list, dim3(tiles), dim3(kBlock), 0, s, gmark, n, tiles, lookback, t.misc + kMiscGroups,
+                     units);
   return hipGetLastError();
 }
 

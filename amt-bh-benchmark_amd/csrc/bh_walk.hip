@@ -812,73 +812,64 @@ __device__ inline void finish_particle(const WalkArgs& a, uint32_t k3, double ax
 }
 
 // Targets of at least kWideMin particles use the group evaluator (its
-// layouts cover 33 to kGroupCap particles, two slots per lane; larger
-// targets walk in chunks of kGroupCap); smaller ones use lane = (particle,
-// slice).
+// layouts cover 33 to kGroupCap particles, two slots per lane); smaller ones
+// use lane = (particle, slice).
 constexpr uint32_t kWideMin = 33;
 
-// One target (node tnode) with the target evaluator (the unit's loop gives
-// it targets of at most 32 particles): the walk over `start` (the group's
-// deferred nodes) or from the root, for each chunk of <= 64 of its
-// particles; then the slices' sums, plus the group's share (gacc, counts
-// g_pp / g_pc) when given.
+// Particles [tb, tb + T) of a target (node tnode; the whole of it or a piece,
+// at most 32 particles) with the target evaluator: the walk over `start` (the
+// group's deferred nodes) or from the root with the target's box, then the
+// slices' sums, plus the group's share (gacc, counts g_pp / g_pc) when given.
 template <typename Real, bool kMask, typename Lds>
-__device__ void walk_target(const WalkArgs& a, Lds& L, uint32_t* gfr, uint32_t tnode, const uint32_t* start,
-                            uint32_t n_start, const double* gacc, uint32_t g_pp, uint32_t g_pc,
+__device__ void walk_target(const WalkArgs& a, Lds& L, uint32_t* gfr, uint32_t tnode, uint32_t tb, uint32_t T,
+                            const uint32_t* start, uint32_t n_start, const double* gacc, uint32_t g_pp, uint32_t g_pc,
                             unsigned long long& tot_pp, unsigned long long& tot_pc) {
   const int lane = __lane_id();
-  const uint32_t tb = uniform(a.begin[tnode]);
-  const uint32_t T = uniform(a.count[tnode]);
   const uint32_t sys_id = uniform(a.sid[tb]);
   const SysDev& sp = a.sys[sys_id];
   const bool use_quad = sp.use_quad != 0;
   const double4 tcv = a.ctr[tnode];
   const double tcx = tcv.x, tcy = tcv.y, tcz = tcv.z;
   const Box6 box = node_box(a, tnode);
-  const double theta2 = sp.theta2;
 
-  for (uint32_t c0 = 0; c0 < T; c0 += kWave) {
-    const uint32_t tc = T - c0 < kWave ? T - c0 : kWave;
-    const int S = kWave / static_cast<int>(tc);
-    TargetEval<Real, kMask> ev;
-    ev.sh.setup(static_cast<uint32_t>(S), static_cast<uint32_t>(lane) / tc);
-    ev.active = lane < static_cast<int>(tc) * S;
-    const int p = lane % static_cast<int>(tc);
-    ev.eps2 = static_cast<Real>(sp.eps2);
-    {
-      const double4 q = a.posm[tb + c0 + p];
-      ev.tx = static_cast<Real>(q.x - tcx);
-      ev.ty = static_cast<Real>(q.y - tcy);
-      ev.tz = static_cast<Real>(q.z - tcz);
-    }
-    uint32_t n_pp = 0, n_pc = 0, n_def = 0;
-    traverse<Real, kMask, false>(a, L, gfr, box, tcx, tcy, tcz, sys_id, start, n_start, use_quad, theta2, ev, n_pp,
-                                 n_pc, nullptr, n_def);
-    n_pp += g_pp;
-    n_pc += g_pc;
-    ev.fold();
-    // combine slices in FP64 (the P2C ring is free now)
-    double* red = reinterpret_cast<double*>(L.pc.a);  // 3 x 64 doubles
-    if (ev.active) {
-      red[3 * lane + 0] = ev.acc.sx();
-      red[3 * lane + 1] = ev.acc.sy();
-      red[3 * lane + 2] = ev.acc.sz();
-    }
-    __builtin_amdgcn_wave_barrier();
-    if (lane < static_cast<int>(tc)) {
-      double ax = 0.0, ay = 0.0, az = 0.0;
-      for (int k2 = 0; k2 < S; ++k2) {
-        const int src = k2 * static_cast<int>(tc) + lane;
-        ax += red[3 * src + 0];
-        ay += red[3 * src + 1];
-        az += red[3 * src + 2];
-      }
-      finish_particle(a, tb + c0 + lane, ax, ay, az, gacc, sp.G, sp.kick_dt, sp.drift_dt, n_pp, n_pc);
-    }
-    tot_pp += static_cast<unsigned long long>(n_pp) * tc;
-    tot_pc += static_cast<unsigned long long>(n_pc) * tc;
-    __builtin_amdgcn_wave_barrier();
+  const int S = kWave / static_cast<int>(T);
+  TargetEval<Real, kMask> ev;
+  ev.sh.setup(static_cast<uint32_t>(S), static_cast<uint32_t>(lane) / T);
+  ev.active = lane < static_cast<int>(T) * S;
+  ev.eps2 = static_cast<Real>(sp.eps2);
+  {
+    const double4 q = a.posm[tb + lane % static_cast<int>(T)];
+    ev.tx = static_cast<Real>(q.x - tcx);
+    ev.ty = static_cast<Real>(q.y - tcy);
+    ev.tz = static_cast<Real>(q.z - tcz);
   }
+  uint32_t n_pp = 0, n_pc = 0, n_def = 0;
+  traverse<Real, kMask, false>(a, L, gfr, box, tcx, tcy, tcz, sys_id, start, n_start, use_quad, sp.theta2, ev, n_pp,
+                               n_pc, nullptr, n_def);
+  n_pp += g_pp;
+  n_pc += g_pc;
+  ev.fold();
+  // combine slices in FP64 (the P2C ring is free now)
+  double* red = reinterpret_cast<double*>(L.pc.a);  // 3 x 64 doubles
+  if (ev.active) {
+    red[3 * lane + 0] = ev.acc.sx();
+    red[3 * lane + 1] = ev.acc.sy();
+    red[3 * lane + 2] = ev.acc.sz();
+  }
+  __builtin_amdgcn_wave_barrier();
+  if (lane < static_cast<int>(T)) {
+    double ax = 0.0, ay = 0.0, az = 0.0;
+    for (int k2 = 0; k2 < S; ++k2) {
+      const int src = k2 * static_cast<int>(T) + lane;
+      ax += red[3 * src + 0];
+      ay += red[3 * src + 1];
+      az += red[3 * src + 2];
+    }
+    finish_particle(a, tb + lane, ax, ay, az, gacc, sp.G, sp.kick_dt, sp.drift_dt, n_pp, n_pc);
+  }
+  tot_pp += static_cast<unsigned long long>(n_pp) * T;
+  tot_pc += static_cast<unsigned long long>(n_pc) * T;
+  __builtin_amdgcn_wave_barrier();
 }
 
 // One walk unit starting at node g: a walk group (topmost node with leaf ||
@@ -890,15 +881,15 @@ __device__ void walk_target(const WalkArgs& a, Lds& L, uint32_t* gfr, uint32_t t
 // unit walks only those.
 //
 // The unit's work is a sequence of jobs: the group's shared walk (if any),
-// then its targets in particle order (a target of more than 128 particles
-// as jobs of 128 of them, each walking the target's list with its box). The
-// group's walk and the targets of 33 particles or more use the group
-// evaluator (its layouts keep the lanes busy for those sizes, and a target
-// of 65-128 particles walks once, not once per 64) through one call of its
-// traversal; smaller targets use the target evaluator. Deferral is off for
-// target jobs (no deferred list): their decisions are accept or open.
+// then its targets in particle order; a unit that is one target, or the piece
+// of one that starts at particle p0, is one job. The group's walk and
+// targets of 33 particles or more use the group evaluator (its layouts keep
+// the lanes busy for those sizes, and a target of 65-128 particles walks
+// once, not once per 64) through one call of its traversal; smaller targets
+// use the target evaluator. Deferral is off for target jobs (no deferred
+// list): their decisions are accept or open.
 template <typename Real, bool kMask, typename Lds>
-__device__ void walk_group(const WalkArgs& a, Lds& L, uint32_t slot, uint32_t g) {
+__device__ void walk_group(const WalkArgs& a, Lds& L, uint32_t slot, uint32_t g, uint32_t p0) {
   const int lane = __lane_id();
   const uint32_t gb = uniform(a.begin[g]);
   // a unit packed from sibling single-target groups spans several nodes
@@ -918,20 +909,18 @@ __device__ void walk_group(const WalkArgs& a, Lds& L, uint32_t slot, uint32_t g)
   uint32_t c = 0;     // next 64-particle chunk of the unit to scan for targets
   uint64_t bits = 0;  // targets of the scanned chunk not yet walked
   uint32_t m = 0;     // this lane's mark in the scanned chunk
-  uint32_t big = 0, big_T = 0, big_off = 0;  // a target of > kGroupCap particles, walked in chunks
   for (;;) {
-    // the next job: the group's walk, a target node, or the next chunk of a
-    // large target
+    // the next job: the group's walk, the unit's one target or a target node
     bool is_group = false;
-    uint32_t tnode = g, off = 0;
+    uint32_t tnode = g, b0 = gb, size = G;
     if (group_job) {
       is_group = true;
       group_job = false;
-    } else if (big_off < big_T) {
-      tnode = big;
-      off = big_off;
     } else if (single_job) {
       single_job = false;
+      const uint32_t len = piece_size(G, sp.piece), left = gb + G - p0;
+      b0 = p0;
+      size = len < left ? len : left;
     } else {
       if (single) break;
       while (!bits && c < G) {
@@ -944,27 +933,18 @@ __device__ void walk_group(const WalkArgs& a, Lds& L, uint32_t slot, uint32_t g)
       const int j = __ffsll(static_cast<long long>(bits)) - 1;
       bits &= bits - 1;
       tnode = uniform(__builtin_amdgcn_readlane(m, j)) - 1u;
+      b0 = uniform(a.begin[tnode]);
+      size = uniform(a.count[tnode]);
     }
     const uint32_t* start = ok ? dl : nullptr;
     const uint32_t n_start = ok ? n_def : 0u;
     const double* gacc = ok ? a.gacc : nullptr;
     const uint32_t jpp = ok ? g_pp : 0u, jpc = ok ? g_pc : 0u;
-    const uint32_t T = is_group ? 0u : uniform(a.count[tnode]);
-    if (!is_group && T < kWideMin) {
-      walk_target<Real, kMask>(a, L, gfr, tnode, start, n_start, gacc, jpp, jpc, tot_pp, tot_pc);
+    if (!is_group && size < kWideMin) {
+      walk_target<Real, kMask>(a, L, gfr, tnode, b0, size, start, n_start, gacc, jpp, jpc, tot_pp, tot_pc);
       continue;
     }
-    if (!is_group && T > kGroupCap && off == 0 && big_T == 0) {
-      big = tnode;  // its chunks follow, this one first
-      big_T = T;
-    }
-    if (!is_group && T > kGroupCap) big_off = off + kGroupCap;
-    if (!is_group && big_T != 0 && big_off >= big_T) big_T = big_off = 0;
-    // group evaluator: the group's shared walk, a target of 33-128 particles
-    // or a chunk of up to 128 of a larger target (its box and list, its
-    // chunk's particles)
-    const uint32_t b0 = is_group ? gb : uniform(a.begin[tnode]) + off;
-    const uint32_t size = is_group ? G : (T - off < kGroupCap ? T - off : kGroupCap);
+    // group evaluator: the group's shared walk or 33-128 particles of a target
     // a packed unit's box and the origin of its relative coordinates (the
     // box centre); a group's or target's: its node box and centre
     const bool pbox = is_group && packed;
@@ -1075,7 +1055,8 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(4))
   __builtin_amdgcn_wave_barrier();
   const uint32_t first = gridDim.x >> 3;
   for (uint32_t k = blockIdx.x >> 3; k < hi - lo;) {
-    walk_group<Real, kMask>(a, L, blockIdx.x, uniform(a.groups[lo + k]));
+    const uint2 u = a.units[lo + k];
+    walk_group<Real, kMask>(a, L, blockIdx.x, uniform(u.x), uniform(u.y));
     // Every lane takes part in the claim (adding 1 for lane 0, 0 for the
     // others) and the unit is read from lane 0's result: no branch on the
     // lane id inside the loop, so all 64 lanes stay together in it (a
