@@ -34,9 +34,10 @@ struct SysDev {
   uint32_t n;
   uint32_t max_leaf;
   uint32_t tsm;      // min(target_size, group_size)
-  int32_t use_quad;
-  uint16_t tile;     // particles a unit of several targets holds at most (0: every target is a unit)
-  uint16_t piece;    // particles a target's unit holds at most (a wider target is cut into pieces)
+  uint16_t use_quad;
+  uint16_t tile;         // walk tile: particles a unit of several targets holds (kMinTile..kGroupCap)
+  uint16_t unit_piece;   // particles of a piece of a unit of several targets
+  uint16_t target_piece; // particles of a piece of a unit that is one target
 };
 static_assert(sizeof(SysDev) == 64, "SysDev layout");
 
@@ -112,7 +113,7 @@ struct WalkArgs {
   const uint32_t* begin;
   const uint32_t* count;
   const double4* posm;     // x, y, z, m in Morton order
-  const uint2* units;      // walk units, Morton order: {node, first particle} (a cut target: a unit per piece)
+  const uint2* units;      // walk units, Morton order: {node, first particle} of each piece
   const uint32_t* unit_n;  // [n_nodes] particles | 1 << 31 of a packed unit at its first node, else 0 (nullable)
   const uint32_t* tmark;   // [n] target node + 1 at each target's first particle, else 0
   const uint16_t* sid;     // system of each particle
@@ -200,15 +201,15 @@ hipError_t launch_tree_finish(const uint64_t* keys, const double4* posm, uint32_
 // tsm. Units: with grouped, topmost nodes with leaf || count <= max(tsm,
 // tile), runs of sibling ones that are single targets packed up to tile
 // particles (unit_n per node: particles | 1 << 31 at a packed unit's first
-// node, else 0); otherwise the targets. A unit that is one target of more than
-// `piece` particles is listed once per piece. tmark, gmark, the two counts and
+// node, else 0); otherwise the targets. A unit of more particles than its
+// kind's piece is listed once per piece. tmark, gmark, the two counts and
 // the unit_list_words() look-back words must be zero.
 hipError_t launch_units(TreeDev t, uint32_t n, const uint16_t* sid, const SysDev* sys, bool grouped, uint32_t* tmark,
                         uint32_t* gmark, uint32_t* unit_n, uint32_t* lookback, uint2* units, hipStream_t s);
 inline uint64_t unit_list_words(uint64_t n) { return (n + kTreeTile - 1) / kTreeTile + 1; }
 
-// The first particle of piece j of a target of cnt particles, and what a
-// piece holds (the last one the rest): equal pieces of at most `piece`.
+// What a piece of a unit of cnt particles holds (the last one the rest): equal
+// pieces of at most `piece`.
 __host__ __device__ inline uint32_t piece_size(uint32_t cnt, uint32_t piece) {
   const uint32_t k = (cnt + piece - 1) / piece;
   return k > 1 ? (cnt + k - 1) / k : cnt;

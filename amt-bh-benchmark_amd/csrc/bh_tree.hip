@@ -631,18 +631,17 @@ __global__ __launch_bounds__(kBlock) void k_upward(int level, TreeDev t) {
 // monotone in the box), so a unit is exact whatever it groups. Not grouped:
 // every target is a unit.
 //
-// A unit that is a single target of more than `piece` particles is marked at
-// the first particle of each of its pieces: every piece walks the target's
-// list (its box) for its own particles.
+// A unit of more particles than its kind's piece (unit_piece, or target_piece
+// for a single target) is marked at the first particle of each of its pieces;
+// the walk moves the ends of pieces to targets.
 //
 // The phase is bound by launches for all but the largest inputs: marks,
 // packing, counts, scan and lists of targets and units took 15 launches; with
 // the target list that nothing read gone, one zero fill and these two kernels
 // are left (events, 1,000 to 250,000 particles: 42-54 us -> 18-22; 1M: 62 ->
 // 30-39; 4M: 79 -> 60).
-__device__ inline void mark_unit(uint32_t* gmark, uint32_t node, uint32_t begin, uint32_t cnt, bool single,
-                                 uint32_t piece) {
-  const uint32_t len = single ? piece_size(cnt, piece) : cnt;
+__device__ inline void mark_unit(uint32_t* gmark, uint32_t node, uint32_t begin, uint32_t cnt, uint32_t piece) {
+  const uint32_t len = piece_size(cnt, piece);
   for (uint32_t o = 0; o < cnt; o += len) gmark[begin + o] = node + 1;
 }
 
@@ -659,20 +658,20 @@ __global__ __launch_bounds__(kBlock) void k_units_mark(TreeDev t, const uint16_t
   for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n_nodes; i += gridDim.x * kBlock) {
     const uint32_t b = t.begin[i], cnt = t.count[i];
     const SysDev& q = sys[sid[b]];
-    const uint32_t tsm = q.tsm, tile = q.tile, piece = q.piece;
+    const uint32_t tsm = q.tsm, tile = q.tile, upiece = q.unit_piece, tpiece = q.target_piece;
     const bool leaf = t.leaf[i] != 0, root = t.depth[i] == 0;
     const bool single = leaf || cnt <= tsm;
     if (single && (root || t.count[t.parent[i]] > tsm)) {
       tmark[b] = i + 1;
       ++mine;
-      if (!grouped) mark_unit(gmark, i, b, cnt, true, piece);
+      if (!grouped) mark_unit(gmark, i, b, cnt, tpiece);
     }
     if (!grouped) continue;
     const uint32_t thr = max(tsm, tile);
     if (leaf || cnt <= thr) {
       if (root) {  // a system that is one walk group
         unit_n[i] = 0u;
-        mark_unit(gmark, i, b, cnt, single, piece);
+        mark_unit(gmark, i, b, cnt, single ? tpiece : upiece);
       }
       continue;
     }
@@ -681,7 +680,7 @@ __global__ __launch_bounds__(kBlock) void k_units_mark(TreeDev t, const uint16_t
     auto end_run = [&]() {  // a run is the first child of a unit and what is packed behind it
       if (run_len == 0) return;
       unit_n[run] = run_len > 1 ? run_n | 0x80000000u : 0u;
-      mark_unit(gmark, run, run_b, run_n, run_len == 1, piece);
+      mark_unit(gmark, run, run_b, run_n, run_len == 1 ? tpiece : upiece);
       run_len = 0;
     };
     for (uint32_t c = fc; c < fc + k; ++c) {
@@ -706,7 +705,7 @@ __global__ __launch_bounds__(kBlock) void k_units_mark(TreeDev t, const uint16_t
         if (cn > tile) end_run();
       } else {
         unit_n[c] = 0u;
-        mark_unit(gmark, c, t.begin[c], cn, false, piece);
+        mark_unit(gmark, c, t.begin[c], cn, upiece);
       }
     }
     end_run();

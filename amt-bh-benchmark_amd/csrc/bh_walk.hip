@@ -872,6 +872,26 @@ __device__ void walk_target(const WalkArgs& a, Lds& L, uint32_t* gfr, uint32_t t
   __builtin_amdgcn_wave_barrier();
 }
 
+// The target that holds particle p of a unit that starts at particle gb: the
+// last mark at or before p (a unit of several targets spans at most kGroupCap
+// particles).
+__device__ inline uint32_t covering_target(const WalkArgs& a, uint32_t gb, uint32_t p) {
+  for (uint32_t back = 0;; back += kWave) {
+    const uint32_t d = back + __lane_id();
+    const uint32_t m = d <= p - gb ? a.tmark[p - d] : 0u;
+    const uint64_t have = __ballot(m != 0);
+    if (have) return uniform(__builtin_amdgcn_readlane(m, __ffsll(static_cast<long long>(have)) - 1)) - 1u;
+    if (back + kWave > p - gb) return 0u;  // not reached: a unit's first particle begins a target
+  }
+}
+
+// Where the cut at particle p of such a unit lies.
+__device__ inline uint32_t cut_place(const WalkArgs& a, uint32_t gb, uint32_t p, uint32_t target_piece) {
+  const uint32_t node = covering_target(a, gb, p);
+  const uint32_t b = uniform(a.begin[node]), n = uniform(a.count[node]);
+  return b == p || n > target_piece ? p : b + n;
+}
+
 // One walk unit starting at node g: a walk group (topmost node with leaf ||
 // count <= max(tsm, 128)) or a run of sibling single-target groups packed
 // into one unit (unit_n). A group that is itself a target walks as one.
@@ -880,9 +900,16 @@ __device__ void walk_target(const WalkArgs& a, Lds& L, uint32_t* gfr, uint32_t t
 // unit's particles and keeping the deferred nodes; then each target of the
 // unit walks only those.
 //
+// A unit of more particles than its kind's piece is walked in pieces, one
+// wavefront each (p0: this piece's place). A piece does the unit's walks, with
+// the unit's box and centre or the target's, for its own particles: every
+// pair is computed from the same rounded coordinates however a unit is cut.
+// A cut that falls inside a target of at most target_piece particles moves
+// to its end.
+//
 // The unit's work is a sequence of jobs: the group's shared walk (if any),
-// then its targets in particle order; a unit that is one target, or the piece
-// of one that starts at particle p0, is one job. The group's walk and
+// then its targets in particle order; a unit that is one target, or a piece
+// of one, is one job. The group's walk and
 // targets of 33 particles or more use the group evaluator (its layouts keep
 // the lanes busy for those sizes, and a target of 65-128 particles walks
 // once, not once per 64) through one call of its traversal; smaller targets
@@ -905,43 +932,61 @@ __device__ void walk_group(const WalkArgs& a, Lds& L, uint32_t slot, uint32_t g,
   uint32_t g_pp = 0, g_pc = 0, n_def = 0;
   bool ok = false;  // the group's shared walk kept all its deferred nodes
   unsigned long long tot_pp = 0, tot_pc = 0;
-  bool group_job = !single, single_job = single;
-  uint32_t c = 0;     // next 64-particle chunk of the unit to scan for targets
+  // this piece's particles [r0, r1)
+  uint32_t r0 = p0, r1;
+  {
+    const uint32_t len = piece_size(G, single ? sp.target_piece : sp.unit_piece), left = gb + G - p0;
+    r1 = p0 + (len < left ? len : left);
+    if (!single) {
+      if (r0 > gb) r0 = cut_place(a, gb, r0, sp.target_piece);
+      if (r1 < gb + G) r1 = cut_place(a, gb, r1, sp.target_piece);
+      if (r0 >= r1) return;
+    }
+  }
+  bool group_job = !single;
+  uint32_t b0 = r0;   // first particle of the next target job
+  uint32_t c = r0;    // next 64-particle chunk of the piece to scan for targets
   uint64_t bits = 0;  // targets of the scanned chunk not yet walked
   uint32_t m = 0;     // this lane's mark in the scanned chunk
   for (;;) {
     // the next job: the group's walk, the unit's one target or a target node
+    // (the piece's first may have begun before it)
     bool is_group = false;
-    uint32_t tnode = g, b0 = gb, size = G;
+    uint32_t tnode = g, jb = r0, size = r1 - r0;
     if (group_job) {
       is_group = true;
       group_job = false;
-    } else if (single_job) {
-      single_job = false;
-      const uint32_t len = piece_size(G, sp.piece), left = gb + G - p0;
-      b0 = p0;
-      size = len < left ? len : left;
+    } else if (b0 >= r1) {
+      break;
+    } else if (single) {
+      b0 = r1;
     } else {
-      if (single) break;
-      while (!bits && c < G) {
-        const uint32_t i = c + lane;
-        m = i < G ? a.tmark[gb + i] : 0u;
-        bits = __ballot(m != 0);
-        c += kWave;
+      if (b0 == r0) {
+        tnode = covering_target(a, gb, r0);
+        c = r0 + 1;
+      } else {
+        while (!bits && c < r1) {
+          const uint32_t i = c + lane;
+          m = i < r1 ? a.tmark[i] : 0u;
+          bits = __ballot(m != 0);
+          c += kWave;
+        }
+        if (!bits) break;  // not reached: targets fill the unit
+        const int j = __ffsll(static_cast<long long>(bits)) - 1;
+        bits &= bits - 1;
+        tnode = uniform(__builtin_amdgcn_readlane(m, j)) - 1u;
       }
-      if (!bits) break;
-      const int j = __ffsll(static_cast<long long>(bits)) - 1;
-      bits &= bits - 1;
-      tnode = uniform(__builtin_amdgcn_readlane(m, j)) - 1u;
-      b0 = uniform(a.begin[tnode]);
-      size = uniform(a.count[tnode]);
+      jb = b0;
+      const uint32_t e = uniform(a.begin[tnode]) + uniform(a.count[tnode]);
+      b0 = e < r1 ? e : r1;
+      size = b0 - jb;
     }
     const uint32_t* start = ok ? dl : nullptr;
     const uint32_t n_start = ok ? n_def : 0u;
     const double* gacc = ok ? a.gacc : nullptr;
     const uint32_t jpp = ok ? g_pp : 0u, jpc = ok ? g_pc : 0u;
     if (!is_group && size < kWideMin) {
-      walk_target<Real, kMask>(a, L, gfr, tnode, b0, size, start, n_start, gacc, jpp, jpc, tot_pp, tot_pc);
+      walk_target<Real, kMask>(a, L, gfr, tnode, jb, size, start, n_start, gacc, jpp, jpc, tot_pp, tot_pc);
       continue;
     }
     // group evaluator: the group's shared walk or 33-128 particles of a target
@@ -957,7 +1002,7 @@ __device__ void walk_group(const WalkArgs& a, Lds& L, uint32_t slot, uint32_t g,
     ev.eps2 = static_cast<Real>(sp.eps2);
 #pragma unroll
     for (int k = 0; k < kGroupChunks; ++k) {
-      const double4 q = a.posm[b0 + ev.particle(k, lane, size)];
+      const double4 q = a.posm[jb + ev.particle(k, lane, size)];
       ev.gx[k] = static_cast<Real>(q.x - ccv.x);
       ev.gy[k] = static_cast<Real>(q.y - ccv.y);
       ev.gz[k] = static_cast<Real>(q.z - ccv.z);
@@ -1000,11 +1045,11 @@ __device__ void walk_group(const WalkArgs& a, Lds& L, uint32_t slot, uint32_t g,
             az += red[3 * src + 2];
           }
           if (is_group) {
-            a.gacc[3 * uint64_t(gb + i) + 0] = ax;
-            a.gacc[3 * uint64_t(gb + i) + 1] = ay;
-            a.gacc[3 * uint64_t(gb + i) + 2] = az;
+            a.gacc[3 * uint64_t(jb + i) + 0] = ax;
+            a.gacc[3 * uint64_t(jb + i) + 1] = ay;
+            a.gacc[3 * uint64_t(jb + i) + 2] = az;
           } else {
-            finish_particle(a, b0 + i, ax, ay, az, gacc, sp.G, sp.kick_dt, sp.drift_dt, n_pp, n_pc);
+            finish_particle(a, jb + i, ax, ay, az, gacc, sp.G, sp.kick_dt, sp.drift_dt, n_pp, n_pc);
           }
         }
         __builtin_amdgcn_wave_barrier();

@@ -123,8 +123,10 @@ int bh_set_graph_mode(bh_ctx* ctx, int mode);
  * targets are packed into units up to it. Results do not depend on it (every
  * target gets its own walk's interaction list either way; sums may round
  * differently); smaller tiles give small systems more wavefronts, larger
- * ones share more of the walk. Applies to the single-system entry points
- * and to batch systems whose walk_tile is 0. */
+ * ones share more of the walk. (Systems of up to 2M particles are walked in
+ * pieces of units too small to be worth a tile, by the system's size alone.)
+ * Applies to the single-system entry points and to batch systems whose
+ * walk_tile is 0. */
 #define BH_MIN_WALK_TILE 16u
 #define BH_MAX_WALK_TILE 128u
 int bh_set_walk_tile(bh_ctx* ctx, uint32_t tile);
