@@ -72,7 +72,7 @@ struct DevBuf {
 struct Scratch {
   uint64_t *keys_a = nullptr, *keys_b = nullptr;
   uint32_t *vals_a = nullptr, *vals_b = nullptr;
-  uint32_t *hist = nullptr, *dbase = nullptr, *lookback = nullptr;
+  uint32_t *hist = nullptr, *lookback = nullptr;
   double *lohi = nullptr, *partial = nullptr;
   uint32_t* misc = nullptr;              // kMiscWords
   unsigned long long* totals = nullptr;  // [2] interaction totals
@@ -95,6 +95,8 @@ struct Plan {
   uint32_t n_chunks = 0;  // bounds blocks
   uint32_t mlx = 0;       // largest max_leaf
   int sid_passes = 0;     // radix passes over the system id
+  int key_passes = 8;     // radix passes over the keys' leading bits (8: all of them)
+  uint64_t largest = 0;   // particles of the largest system
   bool unsoftened = false;
   size_t table_bytes = 0, off_chunks = 0, off_first = 0, off_hist = 0;
   uint64_t node_estimate = 0;
@@ -114,7 +116,7 @@ struct GraphKey {
   uint64_t gen;
   uint32_t n, S, n_chunks, mlx, cap_nodes, depth_plan, slots;
   uint32_t table_bytes;
-  uint8_t deep, unsoftened, precision, mode, carry_out, carried_in;
+  uint8_t deep, unsoftened, precision, mode, carry_out, carried_in, key_passes, pad;
   bool operator==(const GraphKey& o) const { return std::memcmp(this, &o, sizeof *this) == 0; }
 };
 struct GraphEntry {
@@ -153,7 +155,7 @@ struct Ctx {
   DevBuf<bh_particle> tmp_in, tmp_out;  // host-path staging (bh_step, bh_step_batch_host, bh_build_tree)
   DevBuf<uint64_t> keys_a, keys_b;
   DevBuf<uint32_t> vals_a, vals_b;
-  DevBuf<uint32_t> hist, dbase, lookback;
+  DevBuf<uint32_t> hist, lookback;
   DevBuf<double> lohi, partial;
   DevBuf<uint32_t> misc;
   DevBuf<unsigned long long> totals;
@@ -183,6 +185,7 @@ struct Ctx {
   // plans learnt from earlier steps
   uint32_t cap_nodes = 0;        // node capacity asked for (grow-only)
   bool depth_known = false;
+  bool full_sort = false;        // some step's keys shared too many leading bits
   uint32_t depth_hint = kDepthCap;
 
   std::vector<GraphEntry> graphs;
@@ -362,7 +365,7 @@ int plan_systems(Ctx* c, const HostSys* sys, uint32_t S, bool no_grow, Plan* p) 
     set_err(c, "a batch holds 1..%u systems, %u given", kMaxSystems, S);
     return BH_ERR_INVALID;
   }
-  uint64_t n = 0, chunks = 0;
+  uint64_t n = 0, chunks = 0, largest = 0;
   uint32_t mlx = 0, live = 0;
   bool unsoftened = false;
   double nodes = 0.0;
@@ -377,6 +380,7 @@ int plan_systems(Ctx* c, const HostSys* sys, uint32_t S, bool no_grow, Plan* p) 
     n += sys[k].n;
     chunks += (sys[k].n + kChunk - 1) / kChunk;
     mlx = std::max(mlx, sys[k].max_leaf);
+    largest = std::max(largest, sys[k].n);
     unsoftened |= static_cast<float>(sys[k].fp.eps2) == 0.0f;  // zero in the FP32 walk too
     // nodes per particle of Plummer, Hernquist and uniform trees: at most
     // min(1.6, 4 / max_leaf), with a quarter to spare
@@ -388,6 +392,7 @@ int plan_systems(Ctx* c, const HostSys* sys, uint32_t S, bool no_grow, Plan* p) 
   }
   *p = Plan{};
   p->n = static_cast<uint32_t>(n);
+  p->largest = largest;
   if (n == 0) return BH_OK;
   p->S = live;
   p->n_chunks = static_cast<uint32_t>(chunks);
@@ -450,9 +455,19 @@ uint32_t walk_slots(uint32_t n, uint32_t limit) {
   return (s + 7) / 8 * 8;
 }
 
+// Radix passes over the leading key bits of systems of up to n particles.
+// 8 p bits are 10, 13 or 16 octree levels (p = 4, 5, 6); the runs of particles
+// that share them are ordered by one more pass, so the cells of that level
+// should hold few: the centre of a Hernquist sphere (density 1 / r, radius up
+// to 20), the most clustered of the initial conditions, has 5 particles in
+// such a cell at 32,768, 8 at 2M, 1 at 16M. A pass is 6 to 8 us up to 64
+// tiles, 20 at 1M and 134 at 16M.
+int sort_passes(uint64_t n) { return n <= 32768 ? 4 : n <= (2u << 20) ? 5 : 6; }
+
 // The plan's sizes that depend on what the context has learnt.
 void plan_shape(Ctx* c, Plan* p, bool walk) {
   p->walk = walk;
+  p->key_passes = c->full_sort ? 8 : sort_passes(p->largest);
   const uint64_t want = std::max<uint64_t>(p->node_estimate, c->cap_nodes);
   p->cap_nodes = static_cast<uint32_t>(std::min<uint64_t>(want, 1ull << 30));
   p->depth_plan = c->depth_known ? c->depth_hint : static_cast<uint32_t>(kDepthCap);
@@ -469,7 +484,6 @@ int provision(Ctx* c, const Plan& p, Scratch* b) {
   TRY(ensure(c, c->vals_a, n, "indices"));
   TRY(ensure(c, c->vals_b, n, "indices"));
   TRY(ensure(c, c->hist, 10 * 256, "histograms"));
-  TRY(ensure(c, c->dbase, 10 * 256, "digit offsets"));
   TRY(ensure(c, c->lookback, radix_lookback_words(n), "look-back"));
   TRY(ensure(c, c->lohi, 6ull * p.S, "bounds"));
   TRY(ensure(c, c->partial, 6ull * p.n_chunks, "bounds"));
@@ -522,7 +536,6 @@ int provision(Ctx* c, const Plan& p, Scratch* b) {
   s.vals_a = c->vals_a.p;
   s.vals_b = c->vals_b.p;
   s.hist = c->hist.p;
-  s.dbase = c->dbase.p;
   s.lookback = c->lookback.p;
   s.lohi = c->lohi.p;
   s.partial = c->partial.p;
@@ -592,7 +605,6 @@ bool carve(uint8_t* base, size_t bytes, Plan* p, Scratch* b) {
   s.vals_a = reinterpret_cast<uint32_t*>(take(4ull * n));
   s.vals_b = reinterpret_cast<uint32_t*>(take(4ull * n));
   s.hist = reinterpret_cast<uint32_t*>(take(4 * 10 * 256));
-  s.dbase = reinterpret_cast<uint32_t*>(take(4 * 10 * 256));
   s.lookback = reinterpret_cast<uint32_t*>(take(4 * radix_lookback_words(n)));
   s.lohi = reinterpret_cast<double*>(take(48ull * p->S));
   s.partial = reinterpret_cast<double*>(take(48ull * p->n_chunks));
@@ -685,13 +697,13 @@ int enqueue_build(Ctx* c, const Plan& p, const Scratch& b, const bh_particle* d_
   if (p.carried_in) {
     HIP_OK(c, launch_bounds(c->carry.p, n, c->carry_flag.p, chunks, p.n_chunks, chunk_first, p.S, b.partial,
                             b.misc + kMiscNonfinite, b.lohi, s));
-    HIP_OK(c, launch_keys_hist(c->carry.p, n, b.sid, b.lohi, b.keys_a, b.hist, s));
+    HIP_OK(c, launch_keys_hist(c->carry.p, n, p.key_passes, b.sid, b.lohi, b.keys_a, b.hist, s));
   } else {
     HIP_OK(c, launch_bounds(d_in, chunks, p.n_chunks, chunk_first, p.S, b.partial, b.misc + kMiscNonfinite, b.lohi, s));
-    HIP_OK(c, launch_keys_hist(d_in, n, b.sid, b.lohi, b.keys_a, b.hist, s));
+    HIP_OK(c, launch_keys_hist(d_in, n, p.key_passes, b.sid, b.lohi, b.keys_a, b.hist, s));
   }
-  HIP_OK(c, launch_radix_sort(b.keys_a, b.vals_a, b.keys_b, b.vals_b, n, p.sid_passes, b.sid, b.hist, b.dbase,
-                              b.lookback, b.lookback + (lb_words - 10), &out->keys, &out->perm, s));
+  HIP_OK(c, launch_radix_sort(b.keys_a, b.vals_a, b.keys_b, b.vals_b, n, p.key_passes, p.sid_passes, b.sid, b.hist,
+                              b.lookback, b.lookback + (lb_words - 10), b.misc + kMiscAbort, &out->keys, &out->perm, s));
   if (p.carried_in && walk_writes_out)
     HIP_OK(c, launch_gather(c->carry.p, out->perm, b.posm, n, s));
   else
@@ -808,6 +820,7 @@ GraphKey graph_key(const Ctx* c, const Plan& p, const void* in, const void* out)
   k.mode = static_cast<uint8_t>(c->walk_mode);
   k.carry_out = p.carry_out ? 1 : 0;
   k.carried_in = p.carried_in ? 1 : 0;
+  k.key_passes = static_cast<uint8_t>(p.key_passes);
   return k;
 }
 
@@ -820,7 +833,7 @@ int launch_graph(Ctx* c, const Plan& p, const Scratch& b, const bh_particle* d_i
   for (auto& g : c->graphs)
     if (g.key == key) hit = &g;
   // the sort's output buffers follow from the pass count alone
-  const int passes = 8 + p.sid_passes;
+  const int passes = p.key_passes + p.sid_passes;
   sorted->keys = (passes % 2 == 0) ? b.keys_a : b.keys_b;
   sorted->perm = (passes % 2 == 0) ? b.vals_a : b.vals_b;
   if (!hit) {
@@ -930,6 +943,7 @@ int run(Ctx* c, Plan p, const bh_particle* d_in, bh_particle* d_out, bool walk, 
         need = std::max(need, nodes);
         c->cap_nodes = static_cast<uint32_t>(std::min<uint64_t>(need + need / 8 + 64, 1ull << 30));
       }
+      if (abort & kAbortSort) c->full_sort = true;
       if (abort & kAbortDepth) {
         c->depth_hint = std::max(c->depth_known ? c->depth_hint : 0u, m[kMiscMaxDepth]);
         c->depth_known = true;
@@ -1126,7 +1140,6 @@ void bh_ctx_destroy(bh_ctx* h) {
   release(c->vals_a);
   release(c->vals_b);
   release(c->hist);
-  release(c->dbase);
   release(c->lookback);
   release(c->lohi);
   release(c->partial);

@@ -66,6 +66,7 @@ constexpr int kMiscQueue = 48;      // [48, 56): walk-unit queue heads, one per 
 constexpr int kMiscWords = 64;
 constexpr uint32_t kAbortNodes = 1;  // more nodes or leaves than the node arrays hold
 constexpr uint32_t kAbortDepth = 2;  // deeper than the levels the upward pass launched
+constexpr uint32_t kAbortSort = 4;   // too many keys share the sort's leading bits
 
 // The device a context was created on.
 int ctx_device(const bh_ctx* ctx);
@@ -152,8 +153,9 @@ hipError_t launch_fill_u32(uint32_t* p, uint32_t value, uint64_t n, hipStream_t 
 hipError_t launch_fill_sid(const uint4* chunks, uint32_t n_chunks, uint16_t* sid, hipStream_t s);
 hipError_t launch_bounds(const bh_particle* p, const uint4* chunks, uint32_t n_chunks, const uint32_t* chunk_first,
                          uint32_t n_sys, double* partial, uint32_t* nonfinite, double* lohi, hipStream_t s);
-hipError_t launch_keys_hist(const bh_particle* p, uint32_t n, const uint16_t* sid, const double* lohi, uint64_t* keys,
-                            uint32_t* hist, hipStream_t s);
+// Keys, and the histograms of their `passes` leading 8-bit digits.
+hipError_t launch_keys_hist(const bh_particle* p, uint32_t n, int passes, const uint16_t* sid, const double* lohi,
+                            uint64_t* keys, uint32_t* hist, hipStream_t s);
 // The same from the compact copy a resident step's walk wrote for its
 // output (the next step's input): blocks of n x, y, z and m, of which these
 // read x, y, z (24 of the records' 64 bytes). carried_bad: that walk's
@@ -161,15 +163,17 @@ hipError_t launch_keys_hist(const bh_particle* p, uint32_t n, const uint16_t* si
 hipError_t launch_bounds(const double* pos, uint32_t n, const uint32_t* carried_bad, const uint4* chunks,
                          uint32_t n_chunks, const uint32_t* chunk_first, uint32_t n_sys, double* partial,
                          uint32_t* nonfinite, double* lohi, hipStream_t s);
-hipError_t launch_keys_hist(const double* pos, uint32_t n, const uint16_t* sid, const double* lohi, uint64_t* keys,
-                            uint32_t* hist, hipStream_t s);
-// 8 passes over the 63-bit keys, then sid_passes (0-2) over the system id
-// taken from sid[index]: a stable sort of each system's (key, index) pairs
-// in place. hist holds 10 x 256 digit counts (passes 8-9: the systems).
+hipError_t launch_keys_hist(const double* pos, uint32_t n, int passes, const uint16_t* sid, const double* lohi,
+                            uint64_t* keys, uint32_t* hist, hipStream_t s);
+// key_passes passes over the keys' leading bits, sid_passes (0-2) over the
+// system id taken from sid[index], and the runs of equal leading bits (none
+// with 8 passes) ordered by the bits below: a stable sort of each system's
+// (key, index) pairs in place. hist: 10 x 256 digit counts (8-9: the
+// systems). abort: gets kAbortSort when such a run is too long.
 hipError_t launch_radix_sort(uint64_t* keys_a, uint32_t* vals_a, uint64_t* keys_b, uint32_t* vals_b, uint32_t n,
-                             int sid_passes, const uint16_t* sid, uint32_t* hist, uint32_t* digit_base,
-                             uint32_t* lookback, uint32_t* tile_counters, uint64_t** keys_out, uint32_t** vals_out,
-                             hipStream_t s);
+                             int key_passes, int sid_passes, const uint16_t* sid, const uint32_t* hist,
+                             uint32_t* lookback, uint32_t* tile_counters, uint32_t* abort, uint64_t** keys_out,
+                             uint32_t** vals_out, hipStream_t s);
 // The FP64 walk copy (x, y, z, m) in Morton order; with out, also the
 // Morton-ordered particles (a step's walk writes those itself).
 hipError_t launch_gather(const bh_particle* in, bh_particle* out, const uint32_t* perm, double4* posm, uint32_t n,

@@ -10,12 +10,19 @@
 // This file is compiled with -ffp-contract=off: the domain and key
 // arithmetic must round exactly as the reference's FP64 code does.
 //
-// The sort is an LSD radix sort over the 63-bit keys with the input index as
-// payload, 8 passes of 8-bit digits. LSD radix sorting is stable, so the
-// result is exactly the (key, index) order. Each pass is a single "onesweep"
-// kernel: a workgroup ranks a 4096-key tile in LDS with wavefront ballots,
-// obtains its global digit offsets by decoupled look-back over the preceding
-// tiles, and writes the tile out digit-sorted so stores coalesce.
+// The sort is an LSD radix sort over the leading 8 p bits of the 63-bit keys
+// with the input index as payload, p passes of 8-bit digits, and a last pass
+// over the result (k_fix_runs) that orders the runs of keys whose leading bits
+// are equal by the bits below. LSD radix sorting is stable, so the result is
+// exactly the (key, index) order. p is chosen so that such runs are short
+// (sort_passes): 32, 40 or 48 bits hold 10 to 16 octree levels, and the keys
+// below them decide only between particles closer together than that. With
+// all 63 bits (p = 8) there is nothing to fix. Each radix pass is a single
+// "onesweep" kernel: a workgroup ranks a 4096-key tile in LDS with wavefront
+// ballots, obtains its global digit offsets by decoupled look-back over the
+// preceding tiles, and writes the tile out digit-sorted so stores coalesce.
+#include <utility>
+
 #include "bh_internal.h"
 
 namespace bhk {
@@ -23,7 +30,8 @@ namespace bhk {
 namespace {
 
 constexpr int kBlock = 256;
-constexpr int kItems = static_cast<int>(kSortTile) / kBlock;
+constexpr int kSortThreads = 512;
+constexpr int kFixTile = 1024;  // positions per k_fix_runs workgroup
 
 __device__ inline uint64_t lanemask_lt() {
   const int lane = __lane_id();
@@ -202,14 +210,16 @@ __global__ __launch_bounds__(kBlock) void k_bounds_final(const double* __restric
   }
 }
 
-// Morton key per particle (input order) and the 8 digit histograms of all
-// keys, for the onesweep passes' global digit offsets.
-template <typename Src>
+// Morton key per particle (input order) and the histograms of the kDigits
+// leading 8-bit digits of all keys, for the onesweep passes' global digit
+// offsets.
+template <typename Src, int kDigits>
 __global__ __launch_bounds__(kBlock) void k_keys_hist(Src src, uint32_t n,
                                                       const uint16_t* __restrict__ sid, const double* __restrict__ lohi,
                                                       uint64_t* __restrict__ keys, uint32_t* __restrict__ hist) {
-  __shared__ uint32_t s_h[8 * 256];
-  for (int i = threadIdx.x; i < 8 * 256; i += kBlock) s_h[i] = 0;
+  constexpr int kShift = kDigits == 8 ? 0 : 63 - 8 * kDigits;
+  __shared__ uint32_t s_h[kDigits * 256];
+  for (int i = threadIdx.x; i < kDigits * 256; i += kBlock) s_h[i] = 0;
   __syncthreads();
   const int lane = __lane_id();
   const uint32_t stride = gridDim.x * kBlock;
@@ -217,6 +227,9 @@ __global__ __launch_bounds__(kBlock) void k_keys_hist(Src src, uint32_t n,
   // loads of round r + 1 are in flight while round r computes
   double nx = 0.0, ny = 0.0, nz = 0.0;
   uint32_t ns = 0;
+  // the domain of the lane's system, computed when it changes
+  double lx = 0.0, ly = 0.0, lz = 0.0, scale = 0.0;
+  uint32_t have = 0xffffffffu;
   {
     const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
     if (i < n) {
@@ -239,10 +252,15 @@ __global__ __launch_bounds__(kBlock) void k_keys_hist(Src src, uint32_t n,
     }
     uint64_t key = 0;
     if (ok) {
-      double c[3], hw;
-      domain_from_lohi(lohi + 6 * sys_i, c, &hw);
-      const double scale = 2097152.0 / (2.0 * hw);
-      const double lx = c[0] - hw, ly = c[1] - hw, lz = c[2] - hw;
+      if (sys_i != have) {
+        double c[3], hw;
+        domain_from_lohi(lohi + 6 * sys_i, c, &hw);
+        scale = 2097152.0 / (2.0 * hw);
+        lx = c[0] - hw;
+        ly = c[1] - hw;
+        lz = c[2] - hw;
+        have = sys_i;
+      }
       key = spread_bits3(quantize(x, lx, scale)) | (spread_bits3(quantize(y, ly, scale)) << 1) |
             (spread_bits3(quantize(z, lz, scale)) << 2);
       keys[i] = key;
@@ -253,9 +271,9 @@ __global__ __launch_bounds__(kBlock) void k_keys_hist(Src src, uint32_t n,
     const uint32_t nvalid = static_cast<uint32_t>(__popcll(__ballot(ok)));
     const uint64_t prev = __shfl_up(key, 1);
 #pragma unroll
-    for (int b = 0; b < 8; ++b) {
-      const uint32_t d = static_cast<uint32_t>(key >> (8 * b)) & 255u;
-      const uint32_t pd = static_cast<uint32_t>(prev >> (8 * b)) & 255u;
+    for (int b = 0; b < kDigits; ++b) {
+      const uint32_t d = static_cast<uint32_t>(key >> (kShift + 8 * b)) & 255u;
+      const uint32_t pd = static_cast<uint32_t>(prev >> (kShift + 8 * b)) & 255u;
       const bool head = ok && (lane == 0 || d != pd);
       const uint64_t heads = __ballot(head);
       const uint64_t after = lane == 63 ? 0ull : heads & (~0ull << (lane + 1));
@@ -264,12 +282,13 @@ __global__ __launch_bounds__(kBlock) void k_keys_hist(Src src, uint32_t n,
     }
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < 8 * 256; i += kBlock)
+  for (int i = threadIdx.x; i < kDigits * 256; i += kBlock)
     if (s_h[i]) atomicAdd(&hist[i], s_h[i]);
 }
 
-// Exclusive block scan of one value per thread (256 threads).
-__device__ inline uint32_t block_excl_scan(uint32_t v, uint32_t* s_wsum, uint32_t* total) {
+// Exclusive block scan of one value per thread.
+template <int kWavesB>
+__device__ inline uint32_t block_excl_scan(uint32_t v, uint32_t* s_wsum) {
   const int lane = __lane_id(), w = threadIdx.x >> 6;
   uint32_t x = v;
   for (int o = 1; o < 64; o <<= 1) {
@@ -278,54 +297,59 @@ __device__ inline uint32_t block_excl_scan(uint32_t v, uint32_t* s_wsum, uint32_
   }
   if (lane == 63) s_wsum[w] = x;
   __syncthreads();
-  uint32_t off = 0, tot = 0;
-  for (int k = 0; k < kBlock / 64; ++k) {
+  uint32_t off = 0;
+  for (int k = 0; k < kWavesB; ++k)
     if (k < w) off += s_wsum[k];
-    tot += s_wsum[k];
-  }
-  if (total) *total = tot;
   __syncthreads();
   return off + x - v;
 }
 
-__global__ __launch_bounds__(kBlock) void k_hist_scan(const uint32_t* __restrict__ hist, uint32_t* __restrict__ dbase) {
-  __shared__ uint32_t s_w[4];
-  const uint32_t pass = blockIdx.x;
-  const uint32_t v = hist[pass * 256 + threadIdx.x];
-  dbase[pass * 256 + threadIdx.x] = block_excl_scan(v, s_w, nullptr);
-}
-
 // kMode 0: first key pass (payload = input index); 1: key pass; 2: system
-// pass (digit of sid[payload], keys carried along).
+// pass (digit of sid[payload], keys carried along). hist: this pass's digit
+// counts over all keys (each workgroup scans the 256 of them for itself).
+//
+// For small inputs a pass is a chain of latencies (few tiles, one per CU):
+// 512 threads hold 8 keys each, so ranking and scattering take half the
+// rounds of 256 with 16, and the look-back reads kWindow tiles at a time
+// (one by one it was most of the pass when all tiles publish together). For
+// large ones the same tile has twice the wavefronts to hide its loads. A pass
+// at 65,536 particles 12 -> 10 us, 1M 22 -> 19, 16M 146 -> 134.
 template <int kMode>
-__global__ __launch_bounds__(kBlock) void k_onesweep(const uint64_t* __restrict__ kin, const uint32_t* __restrict__ vin,
-                                                     uint64_t* __restrict__ kout, uint32_t* __restrict__ vout, uint32_t n,
-                                                     uint32_t shift, const uint16_t* __restrict__ sid,
-                                                     const uint32_t* __restrict__ dbase, uint32_t* __restrict__ lookback,
-                                                     uint32_t* __restrict__ tile_counter) {
-  __shared__ uint32_t s_hist[4][256];   // per-wave digit counters, then per-wave exclusive bases
+__global__ __launch_bounds__(kSortThreads) void k_onesweep(const uint64_t* __restrict__ kin,
+                                                           const uint32_t* __restrict__ vin, uint64_t* __restrict__ kout,
+                                                           uint32_t* __restrict__ vout, uint32_t n, uint32_t shift,
+                                                           const uint16_t* __restrict__ sid,
+                                                           const uint32_t* __restrict__ hist,
+                                                           uint32_t* __restrict__ lookback,
+                                                           uint32_t* __restrict__ tile_counter) {
+  constexpr int kW = kSortThreads / 64;
+  constexpr int kI = static_cast<int>(kSortTile) / kSortThreads;
+  constexpr uint32_t kPerWave = kSortTile / kW;
+  constexpr int kWindow = 8;
+  __shared__ uint32_t s_hist[kW][256];  // per-wave digit counters, then per-wave exclusive bases
   __shared__ uint32_t s_lexcl[256];     // tile-local exclusive digit offsets
   __shared__ uint32_t s_adj[256];       // global position - local position, per digit
   __shared__ uint64_t s_k[kSortTile];   // the tile in digit order: keys, then (reused) payloads
   __shared__ uint8_t s_d[kSortTile];
   uint32_t* s_v = reinterpret_cast<uint32_t*>(s_k);
-  __shared__ uint32_t s_w[4];
+  __shared__ uint32_t s_w[kW];
   __shared__ uint32_t s_tile;
 
   const int tid = threadIdx.x, w = tid >> 6, lane = __lane_id();
   if (tid == 0) s_tile = atomicAdd(tile_counter, 1u);
-  for (int i = tid; i < 4 * 256; i += kBlock) (&s_hist[0][0])[i] = 0;
+  const uint32_t count = tid < 256 ? hist[tid] : 0u;
+  for (int i = tid; i < kW * 256; i += kSortThreads) (&s_hist[0][0])[i] = 0;
   __syncthreads();
   const uint32_t tile = s_tile;
   const uint32_t base = tile * kSortTile;
 
-  uint64_t k[kItems];
-  uint32_t v[kItems];
-  uint32_t r[kItems];
-  uint32_t dg[kItems];
+  uint64_t k[kI];
+  uint32_t v[kI];
+  uint32_t r[kI];
+  uint32_t dg[kI];
 #pragma unroll
-  for (int j = 0; j < kItems; ++j) {
-    const uint32_t idx = base + w * (kSortTile / 4) + j * 64 + lane;
+  for (int j = 0; j < kI; ++j) {
+    const uint32_t idx = base + w * kPerWave + j * 64 + lane;
     const bool ok = idx < n;
     k[j] = ok ? kin[idx] : ~0ull;
     v[j] = kMode == 0 ? idx : (ok ? vin[idx] : 0u);
@@ -334,12 +358,13 @@ __global__ __launch_bounds__(kBlock) void k_onesweep(const uint64_t* __restrict_
     else
       dg[j] = static_cast<uint32_t>(k[j] >> shift) & 255u;
   }
+  const uint32_t dbase = block_excl_scan<kW>(count, s_w);  // keys with smaller digits
   const uint64_t lt = lanemask_lt();
   // Stable in-tile ranking: items in (wave, item, lane) order follow the
   // input order; lanes with an equal digit are found with 8 ballots.
 #pragma unroll
-  for (int j = 0; j < kItems; ++j) {
-    const uint32_t idx = base + w * (kSortTile / 4) + j * 64 + lane;
+  for (int j = 0; j < kI; ++j) {
+    const uint32_t idx = base + w * kPerWave + j * 64 + lane;
     const bool ok = idx < n;
     const uint32_t d = dg[j];
     uint64_t peers = __ballot(ok);
@@ -357,41 +382,57 @@ __global__ __launch_bounds__(kBlock) void k_onesweep(const uint64_t* __restrict_
     __builtin_amdgcn_wave_barrier();
   }
   __syncthreads();
-  // per digit: totals over waves and per-wave exclusive bases
+  // per digit (thread t < 256): totals over waves and per-wave exclusive bases
   const uint32_t t = tid;
   uint32_t total = 0;
-  {
-    uint32_t c0 = s_hist[0][t], c1 = s_hist[1][t], c2 = s_hist[2][t], c3 = s_hist[3][t];
-    s_hist[0][t] = 0;
-    s_hist[1][t] = c0;
-    s_hist[2][t] = c0 + c1;
-    s_hist[3][t] = c0 + c1 + c2;
-    total = c0 + c1 + c2 + c3;
-  }
   uint32_t* my = &lookback[uint64_t(tile) * 256 + t];
-  __hip_atomic_store(my, (tile == 0 ? kLbPre : kLbAgg) | total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  const uint32_t lex = block_excl_scan(total, s_w, nullptr);
-  s_lexcl[t] = lex;
-  uint32_t excl = 0;
-  if (tile > 0) {
-    int64_t j = static_cast<int64_t>(tile) - 1;
-    for (;;) {
-      const uint32_t val = __hip_atomic_load(&lookback[uint64_t(j) * 256 + t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      const uint32_t f = val & ~kLbVal;
-      if (f == 0) continue;
-      excl += val & kLbVal;
-      if (f == kLbPre) break;
-      --j;
+  if (t < 256) {
+#pragma unroll
+    for (int q = 0; q < kW; ++q) {
+      const uint32_t c = s_hist[q][t];
+      s_hist[q][t] = total;
+      total += c;
     }
-    __hip_atomic_store(my, kLbPre | (excl + total), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(my, (tile == 0 ? kLbPre : kLbAgg) | total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-  s_adj[t] = dbase[t] + excl - lex;
+  const uint32_t lex = block_excl_scan<kW>(total, s_w);
+  if (t < 256) {
+    s_lexcl[t] = lex;
+    uint32_t excl = 0;
+    if (tile > 0) {
+      // tiles j, j - 1, ... : aggregates up to the nearest inclusive prefix
+      for (int64_t j = static_cast<int64_t>(tile) - 1;;) {
+        uint32_t val[kWindow];
+#pragma unroll
+        for (int q = 0; q < kWindow; ++q)
+          val[q] = j - q >= 0 ? __hip_atomic_load(&lookback[uint64_t(j - q) * 256 + t], __ATOMIC_RELAXED,
+                                                  __HIP_MEMORY_SCOPE_AGENT)
+                              : kLbPre;
+        bool found = false, wait = false;
+        int used = 0;
+#pragma unroll
+        for (int q = 0; q < kWindow; ++q) {
+          const uint32_t f = val[q] & ~kLbVal;
+          wait |= f == 0;
+          if (!found && !wait) {
+            excl += val[q] & kLbVal;
+            ++used;
+            found = f == kLbPre;
+          }
+        }
+        if (found) break;
+        j -= used;
+      }
+      __hip_atomic_store(my, kLbPre | (excl + total), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    s_adj[t] = dbase + excl - lex;
+  }
   __syncthreads();
   // keys, then payloads, through the same LDS tile in digit order, so that
   // the stores coalesce (one tile buffer keeps three workgroups per CU)
 #pragma unroll
-  for (int j = 0; j < kItems; ++j) {
-    const uint32_t idx = base + w * (kSortTile / 4) + j * 64 + lane;
+  for (int j = 0; j < kI; ++j) {
+    const uint32_t idx = base + w * kPerWave + j * 64 + lane;
     if (idx < n) {
       const uint32_t d = dg[j];
       const uint32_t pos = s_lexcl[d] + s_hist[w][d] + r[j];
@@ -402,24 +443,117 @@ __global__ __launch_bounds__(kBlock) void k_onesweep(const uint64_t* __restrict_
   }
   __syncthreads();
   const uint32_t tn = n - base < kSortTile ? n - base : kSortTile;
-  uint32_t g[kItems];
+  uint32_t g[kI];
 #pragma unroll
-  for (int j = 0; j < kItems; ++j) {
-    const uint32_t e = tid + j * kBlock;
+  for (int j = 0; j < kI; ++j) {
+    const uint32_t e = tid + j * kSortThreads;
     g[j] = e < tn ? s_adj[s_d[e]] + e : 0u;
     if (e < tn) kout[g[j]] = s_k[e];
   }
   __syncthreads();
 #pragma unroll
-  for (int j = 0; j < kItems; ++j) {
-    const uint32_t idx = base + w * (kSortTile / 4) + j * 64 + lane;
+  for (int j = 0; j < kI; ++j) {
+    const uint32_t idx = base + w * kPerWave + j * 64 + lane;
     if (idx < n) s_v[r[j]] = v[j];
   }
   __syncthreads();
 #pragma unroll
-  for (int j = 0; j < kItems; ++j) {
-    const uint32_t e = tid + j * kBlock;
+  for (int j = 0; j < kI; ++j) {
+    const uint32_t e = tid + j * kSortThreads;
     if (e < tn) vout[g[j]] = s_v[e];
+  }
+}
+
+// Orders the runs of equal leading key bits (key >> shift, within a system)
+// by (key, index). The radix passes left each run in index order, so a run
+// whose keys ascend is done, which equal positions always are. A wavefront
+// takes a run: up to 64 keys are ranked among each other in registers, longer
+// ones key by key against the run in memory, written to the other pair of
+// sort buffers (tk, tv) and copied back. A run of more than kRunCap keys sets
+// kAbortSort: the host runs the step again with full keys.
+constexpr uint32_t kRunCap = 1024;
+
+__global__ __launch_bounds__(kBlock) void k_fix_runs(uint64_t* keys, uint32_t* vals, uint64_t* tk, uint32_t* tv,
+                                                     uint32_t n, uint32_t shift, const uint16_t* __restrict__ sid,
+                                                     uint32_t* __restrict__ abort) {
+  __shared__ uint32_t s_head[kFixTile];
+  __shared__ uint32_t s_n;
+  const uint32_t base = blockIdx.x * kFixTile;
+  const int w = threadIdx.x >> 6, lane = __lane_id();
+  if (threadIdx.x == 0) s_n = 0;
+  __syncthreads();
+  constexpr int kI = kFixTile / kBlock;
+  uint64_t k0[kI], k1[kI], kp[kI];
+#pragma unroll
+  for (int j = 0; j < kI; ++j) {
+    const uint32_t i = base + j * kBlock + threadIdx.x;
+    k0[j] = i < n ? keys[i] : 0ull;
+    k1[j] = i + 1 < n ? keys[i + 1] : ~0ull;
+    kp[j] = i > 0 && i < n ? keys[i - 1] : ~0ull;
+  }
+#pragma unroll
+  for (int j = 0; j < kI; ++j) {
+    const uint32_t i = base + j * kBlock + threadIdx.x;
+    const uint64_t top = k0[j] >> shift;
+    if (i + 1 >= n || (k1[j] >> shift) != top || sid[i] != sid[i + 1]) continue;
+    if (i > 0 && (kp[j] >> shift) == top && sid[i - 1] == sid[i]) continue;
+    s_head[atomicAdd(&s_n, 1u)] = i;  // the first of a run of at least two
+  }
+  __syncthreads();
+  const uint32_t runs = s_n;
+  for (uint32_t h = w; h < runs; h += kBlock / 64) {
+    const uint32_t b = s_head[h];
+    const uint64_t top = keys[b] >> shift;
+    const uint16_t sys = sid[b];
+    // the run's end, and whether it ascends
+    uint32_t e = b;
+    bool sorted = true;
+    for (;;) {
+      const uint32_t i = e + lane;
+      const bool in = i < n && (keys[i] >> shift) == top && sid[i] == sys;
+      const uint64_t m = __ballot(!in);
+      const uint32_t len = m ? static_cast<uint32_t>(__ffsll(static_cast<long long>(m)) - 1) : 64u;
+      const bool falls = in && static_cast<uint32_t>(lane) < len && i > b && keys[i - 1] > keys[i];
+      if (__ballot(falls)) sorted = false;
+      e += len;
+      if (len < 64u) break;
+    }
+    if (sorted) continue;
+    const uint32_t len = e - b;
+    if (len > kRunCap) {
+      if (lane == 0) atomicOr(abort, kAbortSort);
+      continue;
+    }
+    if (len <= 64u) {
+      const bool in = static_cast<uint32_t>(lane) < len;
+      const uint64_t k = in ? keys[b + lane] : ~0ull;
+      const uint32_t v = in ? vals[b + lane] : ~0u;
+      uint32_t rank = 0;
+      for (uint32_t q = 0; q < len; ++q) {
+        const uint64_t kq = __shfl(k, static_cast<int>(q));
+        rank += kq < k || (kq == k && q < static_cast<uint32_t>(lane)) ? 1u : 0u;
+      }
+      if (in) {
+        keys[b + rank] = k;
+        vals[b + rank] = v;
+      }
+    } else {
+      for (uint32_t c = b + lane; c < e; c += 64) {
+        const uint64_t k = keys[c];
+        uint32_t rank = 0;
+        for (uint32_t q = b; q < e; ++q) {
+          const uint64_t kq = keys[q];
+          rank += kq < k || (kq == k && q < c) ? 1u : 0u;
+        }
+        tk[b + rank] = k;
+        tv[b + rank] = vals[c];
+      }
+      __threadfence_block();
+      for (uint32_t c = b + lane; c < e; c += 64) {
+        keys[c] = tk[c];
+        vals[c] = tv[c];
+      }
+    }
   }
 }
 
@@ -509,18 +643,35 @@ hipError_t launch_bounds(const double* pos, uint32_t n, const uint32_t* carried_
   return hipGetLastError();
 }
 
-hipError_t launch_keys_hist(const bh_particle* p, uint32_t n, const uint16_t* sid, const double* lohi, uint64_t* keys,
-                            uint32_t* hist, hipStream_t s) {
-  hipLaunchKernelGGL(k_keys_hist<RecordSrc>, dim3(grid_for(n, 2048)), dim3(kBlock), 0, s, RecordSrc{p}, n, sid, lohi,
-                     keys, hist);
+namespace {
+template <typename Src>
+hipError_t keys_hist(Src src, uint32_t n, int passes, const uint16_t* sid, const double* lohi, uint64_t* keys,
+                     uint32_t* hist, hipStream_t s) {
+  // Every workgroup adds its digit counts to the global ones, kDigits * 256
+  // atomics on the same words: a thread takes 2 to 16 particles so that they
+  // stay few (us, by particles per thread: 65,536 1: 8.7, 2: 6.3, 8: 10.8;
+  // 262,144 1: 24, 8: 12.1; 1M 2: 49, 16: 19.9; 4M 8: 68, 16: 54).
+  const uint32_t few = n / 512 < 128 ? n / 512 + 1 : 128, many = n / 4096 < 2048 ? n / 4096 : 2048;
+  const dim3 g(few > many ? few : many), b(kBlock);
+  switch (passes) {
+    case 4: hipLaunchKernelGGL((k_keys_hist<Src, 4>), g, b, 0, s, src, n, sid, lohi, keys, hist); break;
+    case 5: hipLaunchKernelGGL((k_keys_hist<Src, 5>), g, b, 0, s, src, n, sid, lohi, keys, hist); break;
+    case 6: hipLaunchKernelGGL((k_keys_hist<Src, 6>), g, b, 0, s, src, n, sid, lohi, keys, hist); break;
+    case 8: hipLaunchKernelGGL((k_keys_hist<Src, 8>), g, b, 0, s, src, n, sid, lohi, keys, hist); break;
+    default: return hipErrorInvalidValue;
+  }
   return hipGetLastError();
 }
+}  // namespace
 
-hipError_t launch_keys_hist(const double* pos, uint32_t n, const uint16_t* sid, const double* lohi, uint64_t* keys,
-                            uint32_t* hist, hipStream_t s) {
-  hipLaunchKernelGGL(k_keys_hist<CompactSrc>, dim3(grid_for(n, 2048)), dim3(kBlock), 0, s, CompactSrc{pos, n}, n, sid,
-                     lohi, keys, hist);
-  return hipGetLastError();
+hipError_t launch_keys_hist(const bh_particle* p, uint32_t n, int passes, const uint16_t* sid, const double* lohi,
+                            uint64_t* keys, uint32_t* hist, hipStream_t s) {
+  return keys_hist(RecordSrc{p}, n, passes, sid, lohi, keys, hist, s);
+}
+
+hipError_t launch_keys_hist(const double* pos, uint32_t n, int passes, const uint16_t* sid, const double* lohi,
+                            uint64_t* keys, uint32_t* hist, hipStream_t s) {
+  return keys_hist(CompactSrc{pos, n}, n, passes, sid, lohi, keys, hist, s);
 }
 
 uint64_t radix_lookback_words(uint32_t n) {
@@ -529,35 +680,32 @@ uint64_t radix_lookback_words(uint32_t n) {
 }
 
 hipError_t launch_radix_sort(uint64_t* keys_a, uint32_t* vals_a, uint64_t* keys_b, uint32_t* vals_b, uint32_t n,
-                             int sid_passes, const uint16_t* sid, uint32_t* hist, uint32_t* digit_base,
-                             uint32_t* lookback, uint32_t* tile_counters, uint64_t** keys_out, uint32_t** vals_out,
-                             hipStream_t s) {
+                             int key_passes, int sid_passes, const uint16_t* sid, const uint32_t* hist,
+                             uint32_t* lookback, uint32_t* tile_counters, uint32_t* abort, uint64_t** keys_out,
+                             uint32_t** vals_out, hipStream_t s) {
   const uint32_t tiles = (n + kSortTile - 1) / kSortTile;
-  const int passes = 8 + sid_passes;
-  hipLaunchKernelGGL(k_hist_scan, dim3(passes), dim3(kBlock), 0, s, hist, digit_base);
+  const uint32_t low = key_passes == 8 ? 0u : 63u - 8u * key_passes;  // bits below the radix digits
   uint64_t* kin = keys_a;
   uint32_t* vin = vals_a;
   uint64_t* ko = keys_b;
   uint32_t* vo = vals_b;
-  for (int pass = 0; pass < passes; ++pass) {
+  for (int pass = 0; pass < key_passes + sid_passes; ++pass) {
     uint32_t* lb = lookback + uint64_t(pass) * tiles * 256;
-    const uint32_t* db = digit_base + pass * 256;
     if (pass == 0)
-      hipLaunchKernelGGL(k_onesweep<0>, dim3(tiles), dim3(kBlock), 0, s, kin, vin, ko, vo, n, 0u, sid, db, lb,
+      hipLaunchKernelGGL(k_onesweep<0>, dim3(tiles), dim3(kSortThreads), 0, s, kin, vin, ko, vo, n, low, sid, hist, lb,
                          tile_counters + pass);
-    else if (pass < 8)
-      hipLaunchKernelGGL(k_onesweep<1>, dim3(tiles), dim3(kBlock), 0, s, kin, vin, ko, vo, n, 8u * pass, sid, db, lb,
-                         tile_counters + pass);
+    else if (pass < key_passes)
+      hipLaunchKernelGGL(k_onesweep<1>, dim3(tiles), dim3(kSortThreads), 0, s, kin, vin, ko, vo, n, low + 8u * pass, sid,
+                         hist + pass * 256, lb, tile_counters + pass);
     else
-      hipLaunchKernelGGL(k_onesweep<2>, dim3(tiles), dim3(kBlock), 0, s, kin, vin, ko, vo, n, 8u * (pass - 8), sid, db,
-                         lb, tile_counters + pass);
-    uint64_t* tk = kin;
-    kin = ko;
-    ko = tk;
-    uint32_t* tv = vin;
-    vin = vo;
-    vo = tv;
+      hipLaunchKernelGGL(k_onesweep<2>, dim3(tiles), dim3(kSortThreads), 0, s, kin, vin, ko, vo, n,
+                         8u * (pass - key_passes), sid, hist + (8 + pass - key_passes) * 256, lb, tile_counters + pass);
+    std::swap(kin, ko);
+    std::swap(vin, vo);
   }
+  if (low)
+    hipLaunchKernelGGL(k_fix_runs, dim3((n + kFixTile - 1) / kFixTile), dim3(kBlock), 0, s, kin, vin, ko, vo, n, low, sid,
+                       abort);
   *keys_out = kin;
   *vals_out = vin;
   return hipGetLastError();

@@ -277,7 +277,7 @@ __global__ __launch_bounds__(kBlock) void k_tree_emit(const uint8_t* __restrict_
     if (tile == 0) {
       t.misc[kMiscMaxDepth] = deepest;
       const uint32_t abort = (over ? kAbortNodes : 0u) | (deepest > depth_plan ? kAbortDepth : 0u);
-      if (abort) t.misc[kMiscAbort] = abort;
+      if (abort) t.misc[kMiscAbort] |= abort;  // the sort may have set its own bit
       if (!over)
         for (int d = 0; d < kLevels + 2; ++d) t.level_off[d] = s_loff[d];
     }
