@@ -41,6 +41,14 @@ namespace {
 
 constexpr int kBlock = 256;
 constexpr int kItems = 16;
+// The kernels that take a tile of 4,096 particles run it with 1,024 threads:
+// with few tiles they are chains of latencies (loads, ballots and LDS steps of
+// each thread's particles in turn), and four particles per thread instead of
+// sixteen shorten them (65,536 particles: count 17.9 -> 8.0 us, emit 34 ->
+// 14.4; 1M: 18 -> 9, 35 -> 14; at 16M, where the tiles fill the chip, equal).
+constexpr int kTileThreads = 1024;
+constexpr int kTileItems = static_cast<int>(kTreeTile) / kTileThreads;
+constexpr int kTileWaves = kTileThreads / 64;
 
 __device__ inline uint64_t lanemask_lt() {
   const int lane = __lane_id();
@@ -88,10 +96,11 @@ __device__ inline void domain_from_lohi(const double* lohi, double c[3], double*
 // With several systems the windows stop at system boundaries: a system's
 // first particle begins its root (L = 0) and P, W only look at particles of
 // the same system, with that system's max_leaf.
-__global__ __launch_bounds__(kBlock) void k_tree_count(const uint64_t* __restrict__ keys, uint32_t n,
-                                                       const uint16_t* __restrict__ sid, const SysDev* __restrict__ sys,
-                                                       uint32_t mlx, uint8_t* __restrict__ L, uint8_t* __restrict__ H,
-                                                       uint32_t* __restrict__ tile_counts) {
+__global__ __launch_bounds__(kTileThreads) void k_tree_count(const uint64_t* __restrict__ keys, uint32_t n,
+                                                             const uint16_t* __restrict__ sid,
+                                                             const SysDev* __restrict__ sys, uint32_t mlx,
+                                                             uint8_t* __restrict__ L, uint8_t* __restrict__ H,
+                                                             uint32_t* __restrict__ tile_counts) {
   // dynamic LDS sized by the batch's largest max_leaf (mlx): keys of
   // [base - mlx - 1, base + tile + mlx), then P of [base - mlx, base + tile)
   extern __shared__ __align__(8) unsigned char s_dyn[];
@@ -101,23 +110,23 @@ __global__ __launch_bounds__(kBlock) void k_tree_count(const uint64_t* __restric
   __shared__ uint32_t s_one;  // 1 + system id when the tile and its halo hold one system, else 0
   const uint32_t tile = blockIdx.x, base = tile * kTreeTile;
   const int64_t g0 = static_cast<int64_t>(base) - mlx - 1;  // global index of s_k[0]
-  constexpr int kPer = static_cast<int>(kTreeTile) / kBlock;
+  constexpr int kPer = static_cast<int>(kTreeTile) / kTileThreads;
   {
     // the tile's keys: every load in flight before the first LDS write
     uint64_t kv[kPer];
 #pragma unroll
     for (int j = 0; j < kPer; ++j) {
-      const uint32_t i = base + threadIdx.x + j * kBlock;
+      const uint32_t i = base + threadIdx.x + j * kTileThreads;
       kv[j] = i < n ? keys[i] : 0ull;
     }
     // the halos [g0, base) and [base + tile, base + tile + mlx)
-    for (uint32_t h = threadIdx.x; h < 2 * mlx + 1; h += kBlock) {
+    for (uint32_t h = threadIdx.x; h < 2 * mlx + 1; h += kTileThreads) {
       const uint32_t e = h <= mlx ? h : h + kTreeTile;
       const int64_t g = g0 + e;
       s_k[e] = (g >= 0 && g < n) ? keys[g] : 0ull;
     }
 #pragma unroll
-    for (int j = 0; j < kPer; ++j) s_k[mlx + 1 + threadIdx.x + j * kBlock] = kv[j];
+    for (int j = 0; j < kPer; ++j) s_k[mlx + 1 + threadIdx.x + j * kTileThreads] = kv[j];
   }
   if (threadIdx.x < kTreeCols) s_cnt[threadIdx.x] = 0;
   if (threadIdx.x == 0) {
@@ -136,7 +145,7 @@ __global__ __launch_bounds__(kBlock) void k_tree_count(const uint64_t* __restric
     o_ml = sys[one - 1u].max_leaf;
   }
   // P_u for u in [base - mlx, base + tile)
-  for (uint32_t e = threadIdx.x; e < kTreeTile + mlx; e += kBlock) {
+  for (uint32_t e = threadIdx.x; e < kTreeTile + mlx; e += kTileThreads) {
     const int64_t u = static_cast<int64_t>(base) - mlx + e;
     int8_t pv = -1;
     if (u >= 0 && u < n) {
@@ -156,7 +165,7 @@ __global__ __launch_bounds__(kBlock) void k_tree_count(const uint64_t* __restric
   int li_r[kPer];
 #pragma unroll
   for (int j = 0; j < kPer; ++j) {
-    const uint32_t e = threadIdx.x + j * kBlock, i = base + e;
+    const uint32_t e = threadIdx.x + j * kTileThreads, i = base + e;
     li_r[j] = 0;
     if (i < n) {
       const uint32_t qo = one ? o_off : sys[sid[i]].off;
@@ -182,7 +191,7 @@ __global__ __launch_bounds__(kBlock) void k_tree_count(const uint64_t* __restric
     for (int k = 1; k <= K; ++k) {
       int8_t* dst = (k & 1) ? tb0 : tb1;
       const uint32_t h = 1u << (k - 1);
-      for (uint32_t e = threadIdx.x; e < np; e += kBlock) {
+      for (uint32_t e = threadIdx.x; e < np; e += kTileThreads) {
         const int a0 = top[e];
         const int a1 = e + h < np ? top[e + h] : -1;
         dst[e] = static_cast<int8_t>(a0 > a1 ? a0 : a1);
@@ -193,7 +202,7 @@ __global__ __launch_bounds__(kBlock) void k_tree_count(const uint64_t* __restric
   }
 #pragma unroll
   for (int j = 0; j < kPer; ++j) {
-    const uint32_t e = threadIdx.x + j * kBlock, i = base + e;
+    const uint32_t e = threadIdx.x + j * kTileThreads, i = base + e;
     if (i >= n) break;
     uint32_t qoff = o_off, qn = o_n, ml = o_ml;
     if (!one) {
@@ -254,11 +263,11 @@ __global__ __launch_bounds__(1024) void k_col_scan(const uint32_t* __restrict__ 
 // nodes or leaves than the arrays hold (kAbortNodes; the host grows them and
 // runs the step again); a tree deeper than the upward launches planned is
 // numbered but flagged (kAbortDepth), so the kernels after this one skip it.
-__global__ __launch_bounds__(kBlock) void k_tree_emit(const uint8_t* __restrict__ L, const uint8_t* __restrict__ H, uint32_t n,
-                                                      const uint32_t* __restrict__ tile_prefix, TreeDev t,
-                                                      uint32_t depth_plan) {
+__global__ __launch_bounds__(kTileThreads) void k_tree_emit(const uint8_t* __restrict__ L, const uint8_t* __restrict__ H,
+                                                            uint32_t n, const uint32_t* __restrict__ tile_prefix,
+                                                            TreeDev t, uint32_t depth_plan) {
   __shared__ uint32_t s_loff[kLevels + 2];
-  __shared__ uint32_t s_wc[4][kTreeCols];
+  __shared__ uint32_t s_wc[kTileWaves][kTreeCols];
   __shared__ uint32_t s_over;
   const uint32_t tile = blockIdx.x, base = tile * kTreeTile;
   const int w = threadIdx.x >> 6, lane = __lane_id();
@@ -291,14 +300,14 @@ __global__ __launch_bounds__(kBlock) void k_tree_emit(const uint8_t* __restrict_
   // an item's L and H, packed (255 = no particle); the next item's load is
   // issued before the current item's levels are counted
   auto load_lh = [&](int j) -> uint32_t {
-    const uint32_t idx = base + w * (kTreeTile / 4) + j * 64 + lane;
+    const uint32_t idx = base + w * (kTreeTile / kTileWaves) + j * 64 + lane;
     return idx < n ? static_cast<uint32_t>(L[idx]) | (static_cast<uint32_t>(H[idx]) << 8) : 255u;
   };
   uint32_t nlh = load_lh(0);
 #pragma unroll 1
-  for (int j = 0; j < kItems; ++j) {
+  for (int j = 0; j < kTileItems; ++j) {
     const uint32_t lh = nlh;
-    if (j + 1 < kItems) nlh = load_lh(j + 1);
+    if (j + 1 < kTileItems) nlh = load_lh(j + 1);
     const int lj = static_cast<int>(lh & 255u), hj = static_cast<int>(lh >> 8);
     // only the levels where some lane begins a node
     const uint32_t wm = wave_or(level_bits(lj, hj));
@@ -314,7 +323,7 @@ __global__ __launch_bounds__(kBlock) void k_tree_emit(const uint8_t* __restrict_
   __syncthreads();
   if (threadIdx.x <= kLevels) {
     uint32_t a = 0;
-    for (int k = 0; k < 4; ++k) {
+    for (int k = 0; k < kTileWaves; ++k) {
       const uint32_t v = s_wc[k][threadIdx.x];
       s_wc[k][threadIdx.x] = a;
       a += v;
@@ -330,10 +339,10 @@ __global__ __launch_bounds__(kBlock) void k_tree_emit(const uint8_t* __restrict_
   const uint64_t lt = lanemask_lt();
   nlh = load_lh(0);
 #pragma unroll 1
-  for (int j = 0; j < kItems; ++j) {
-    const uint32_t idx = base + w * (kTreeTile / 4) + j * 64 + lane;
+  for (int j = 0; j < kTileItems; ++j) {
+    const uint32_t idx = base + w * (kTreeTile / kTileWaves) + j * 64 + lane;
     const uint32_t lh = nlh;
-    if (j + 1 < kItems) nlh = load_lh(j + 1);
+    if (j + 1 < kTileItems) nlh = load_lh(j + 1);
     const int lj = static_cast<int>(lh & 255u), hj = static_cast<int>(lh >> 8);
     const uint64_t lm = __ballot(lj <= hj);
     const uint32_t lr = run[kLevels] + __popcll(lm & lt);
@@ -469,19 +478,22 @@ __device__ inline void finalize_write(TreeDev t, uint32_t i, const double4& cc, 
 // into LDS in coalesced chunks of kUpChunk; each thread then adds the
 // particles of its leaf that lie in the chunk, in order, so its sums run
 // over the leaf's particles in the reference's order.
+// 128 threads: a workgroup covers few enough leaves that small systems reach
+// several CUs (262,144 particles: 26 -> 18 us with 256 -> 128).
 constexpr uint32_t kUpChunk = 1024;
+constexpr int kLeafThreads = 128;
 
-__global__ __launch_bounds__(kBlock) void k_upward_leaves(const double4* __restrict__ posm, uint32_t n, TreeDev t) {
+__global__ __launch_bounds__(kLeafThreads) void k_upward_leaves(const double4* __restrict__ posm, uint32_t n, TreeDev t) {
   // one array per coordinate: lanes read scattered particles, and 8-byte
   // elements spread those reads over the banks better than 32-byte ones
   __shared__ double s_x[kUpChunk], s_y[kUpChunk], s_z[kUpChunk], s_m[kUpChunk];
   if (t.misc[kMiscAbort]) return;
   const uint32_t n_leaves = t.misc[kMiscLevels + kLevels];
   const double inf = __builtin_huge_val();
-  for (uint32_t l0 = blockIdx.x * kBlock; l0 < n_leaves; l0 += gridDim.x * kBlock) {
+  for (uint32_t l0 = blockIdx.x * kLeafThreads; l0 < n_leaves; l0 += gridDim.x * kLeafThreads) {
     const uint32_t lr = l0 + threadIdx.x;
     const bool mine = lr < n_leaves;
-    const uint32_t l1 = l0 + kBlock < n_leaves ? l0 + kBlock : n_leaves;
+    const uint32_t l1 = l0 + kLeafThreads < n_leaves ? l0 + kLeafThreads : n_leaves;
     const uint32_t span_lo = t.leaf_first[l0];
     const uint32_t span_hi = l1 < n_leaves ? t.leaf_first[l1] : n;
     uint32_t i = 0, b = 0, e = 0;
@@ -500,16 +512,16 @@ __global__ __launch_bounds__(kBlock) void k_upward_leaves(const double4* __restr
       __syncthreads();
       {
         // every load of the chunk in flight before the first LDS write
-        constexpr int kR = kUpChunk / kBlock;
+        constexpr int kR = kUpChunk / kLeafThreads;
         double4 q[kR];
 #pragma unroll
         for (int r = 0; r < kR; ++r) {
-          const uint32_t k = threadIdx.x + r * kBlock;
+          const uint32_t k = threadIdx.x + r * kLeafThreads;
           q[r] = posm[c0 + (k < cn ? k : cn - 1)];
         }
 #pragma unroll
         for (int r = 0; r < kR; ++r) {
-          const uint32_t k = threadIdx.x + r * kBlock;
+          const uint32_t k = threadIdx.x + r * kLeafThreads;
           if (k < cn) {
             s_x[k] = q[r].x;
             s_y[k] = q[r].y;
@@ -548,69 +560,103 @@ __global__ __launch_bounds__(kBlock) void k_upward_leaves(const double4* __restr
 // finalize_node for the interior nodes of one level, children already
 // final. A team of 8 lanes takes a node: lane j loads child j (at most 8)
 // and forms its terms as the reference does (mass, m d, the child's second
-// moment + m d_a d_b, its box); the team then adds the terms in child
-// order through shuffles, so the sums are the reference's to the bit, and
-// every lane holds them; lane 0 writes the node. (Loading the children one
-// after another from one thread left each level waiting on ~8 dependent
-// memory round trips.)
+// moment + m d_a d_b, its box). The terms go to LDS, where each lane adds two
+// or three of the 17 sums over the children in child order (the reference's
+// sums to the bit), and lane 0 collects them and writes the node. (Adding
+// through shuffles took 272 lane permutes in turn: 7 us a level at 65,536
+// particles against 5; loading the children one after another from one thread
+// left each level waiting on ~8 dependent memory round trips.)
 constexpr int kKids = 8;
+constexpr int kTerms = 16;  // mass, 3 first and 6 second moments, 6 box corners
 
-__global__ __launch_bounds__(kBlock) void k_upward(int level, TreeDev t) {
-  if (t.misc[kMiscAbort]) return;
-  const uint32_t lo = t.level_off[level], hi = t.level_off[level + 1];
+struct Team {
+  double term[kTerms][kKids];
+  uint32_t count[kKids];
+};
+
+// Nodes i, i + step, ... < hi of a level, one per team and round; every lane
+// of the team's wavefront takes part in each round (i0 = the wavefront's first).
+__device__ inline void upward_nodes(TreeDev t, Team& team, uint32_t lo, uint32_t i0, uint32_t hi, uint32_t step) {
   const double inf = __builtin_huge_val();
   const int j = static_cast<int>(threadIdx.x) & (kKids - 1);
-  const uint32_t teams = gridDim.x * (kBlock / kKids);
-  for (uint32_t i0 = lo + blockIdx.x * (kBlock / kKids); i0 < hi; i0 += teams) {
-    const uint32_t i = i0 + threadIdx.x / kKids;
+  for (; i0 < hi; i0 += step) {
+    const uint32_t i = i0 + (threadIdx.x & 63u) / kKids;
     const bool node_ok = i < hi && !t.leaf[i < hi ? i : lo];
     const uint32_t fc = node_ok ? t.first_child[i] : 0u;
     const uint32_t k = node_ok ? t.nchild[i] : 0u;
     const double4 cc = node_ok ? t.ctr[i] : make_double4(0.0, 0.0, 0.0, 0.0);
     // this lane's child and its terms
-    const bool has = static_cast<uint32_t>(j) < k;
-    const uint32_t c = fc + static_cast<uint32_t>(j);
-    double tm = 0.0, t1[3] = {0.0, 0.0, 0.0}, t2[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    double clo[3] = {inf, inf, inf}, chi[3] = {-inf, -inf, -inf};
-    uint32_t ccount = 0;
-    if (has) {
+    if (static_cast<uint32_t>(j) < k) {
+      const uint32_t c = fc + static_cast<uint32_t>(j);
       const double mass = t.mass[c];
       const double d[3] = {t.com[3 * c + 0] - cc.x, t.com[3 * c + 1] - cc.y, t.com[3 * c + 2] - cc.z};
-      tm = mass;
-      for (int a = 0; a < 3; ++a) t1[a] = d[a] * mass;
       const double* ib = &t.iab[6 * c];
-      t2[0] = ib[0] + mass * d[0] * d[0];
-      t2[1] = ib[1] + mass * d[1] * d[1];
-      t2[2] = ib[2] + mass * d[2] * d[2];
-      t2[3] = ib[3] + mass * d[0] * d[1];
-      t2[4] = ib[4] + mass * d[0] * d[2];
-      t2[5] = ib[5] + mass * d[1] * d[2];
-      ccount = t.count[c];
       const double* cb = &t.nbox[6 * uint64_t(c)];
-      for (int a = 0; a < 3; ++a) {
-        clo[a] = cb[a];
-        chi[a] = cb[3 + a];
-      }
+      team.term[0][j] = mass;
+      for (int a = 0; a < 3; ++a) team.term[1 + a][j] = d[a] * mass;
+      team.term[4][j] = ib[0] + mass * d[0] * d[0];
+      team.term[5][j] = ib[1] + mass * d[1] * d[1];
+      team.term[6][j] = ib[2] + mass * d[2] * d[2];
+      team.term[7][j] = ib[3] + mass * d[0] * d[1];
+      team.term[8][j] = ib[4] + mass * d[0] * d[2];
+      team.term[9][j] = ib[5] + mass * d[1] * d[2];
+      for (int a = 0; a < 6; ++a) team.term[10 + a][j] = cb[a];
+      team.count[j] = t.count[c];
     }
-    // sums in child order; the team's lanes share k, so every shuffle reads
-    // a lane of the team that is in the loop
-    double rm = 0.0, m1[3] = {0.0, 0.0, 0.0}, m2[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    double blo[3] = {inf, inf, inf}, bhi[3] = {-inf, -inf, -inf};
+    __builtin_amdgcn_wave_barrier();
+    // lane j: terms j and j + 8, in child order (sums; from 10 on the box)
+    double r0 = 0.0, r1 = j < 2 ? 0.0 : (j < 5 ? inf : -inf);
     uint32_t cnt = 0;
     for (uint32_t q = 0; q < k; ++q) {
-      rm += __shfl(tm, static_cast<int>(q), kKids);
-      for (int a = 0; a < 3; ++a) m1[a] += __shfl(t1[a], static_cast<int>(q), kKids);
-      for (int a = 0; a < 6; ++a) m2[a] += __shfl(t2[a], static_cast<int>(q), kKids);
-      for (int a = 0; a < 3; ++a) {
-        blo[a] = fmin(blo[a], __shfl(clo[a], static_cast<int>(q), kKids));
-        bhi[a] = fmax(bhi[a], __shfl(chi[a], static_cast<int>(q), kKids));
-      }
-      cnt += static_cast<uint32_t>(__shfl(static_cast<int>(ccount), static_cast<int>(q), kKids));
+      r0 += team.term[j][q];
+      const double v = team.term[8 + j][q];
+      r1 = j < 2 ? r1 + v : (j < 5 ? fmin(r1, v) : fmax(r1, v));
+      cnt += team.count[q];
     }
+    __builtin_amdgcn_wave_barrier();
+    team.term[j][0] = r0;
+    team.term[8 + j][0] = r1;
+    __builtin_amdgcn_wave_barrier();
     if (node_ok && j == 0) {
+      const double rm = team.term[0][0];
+      const double m1[3] = {team.term[1][0], team.term[2][0], team.term[3][0]};
+      double m2[6], blo[3], bhi[3];
+      for (int a = 0; a < 6; ++a) m2[a] = team.term[4 + a][0];
+      for (int a = 0; a < 3; ++a) {
+        blo[a] = team.term[10 + a][0];
+        bhi[a] = team.term[13 + a][0];
+      }
       t.count[i] = cnt;
       finalize_write(t, i, cc, rm, m1, m2, blo, bhi, cnt, false);
     }
+    __builtin_amdgcn_wave_barrier();
+  }
+}
+
+__global__ __launch_bounds__(kBlock) void k_upward(int level, TreeDev t) {
+  __shared__ Team teams[kBlock / kKids];
+  const uint32_t lo = t.level_off[level], hi = t.level_off[level + 1];
+  if (t.misc[kMiscAbort]) return;
+  constexpr uint32_t kPer = kBlock / kKids;
+  upward_nodes(t, teams[threadIdx.x / kKids], lo, lo + blockIdx.x * kPer + (threadIdx.x >> 6) * (64 / kKids), hi,
+               gridDim.x * kPer);
+}
+
+// Levels top, top - 1, ... 0 of a single system in one workgroup, one round
+// of teams each: a launch less for every level but one (65,536 particles: tree
+// phase 79 -> 76 us with levels 0-2; with level 3 too, whose 512 nodes take
+// several rounds here and one in a launch of its own, 80).
+constexpr int kTopLevel = 2;  // at most 8^2 = 64 nodes
+constexpr int kTopThreads = 64 * kKids;
+
+__global__ __launch_bounds__(kTopThreads) void k_upward_top(int top, TreeDev t) {
+  constexpr uint32_t kPer = kTopThreads / kKids;
+  __shared__ Team teams[kPer];
+  if (t.misc[kMiscAbort]) return;
+  for (int d = top; d >= 0; --d) {
+    const uint32_t lo = t.level_off[d], hi = t.level_off[d + 1];
+    upward_nodes(t, teams[threadIdx.x / kKids], lo, lo + (threadIdx.x >> 6) * (64 / kKids), hi, kPer);
+    __syncthreads();  // the level's nodes are written before its parents read them
   }
 }
 
@@ -683,9 +729,21 @@ __global__ __launch_bounds__(kBlock) void k_units_mark(TreeDev t, const uint16_t
       mark_unit(gmark, run, run_b, run_n, run_len == 1 ? tpiece : upiece);
       run_len = 0;
     };
-    for (uint32_t c = fc; c < fc + k; ++c) {
-      const uint32_t cn = t.count[c];
-      const bool cleaf = t.leaf[c] != 0;
+    // every child's fields loaded before the first is looked at
+    uint32_t kid_n[8], kid_b[8];
+    uint8_t kid_leaf[8];
+#pragma unroll
+    for (uint32_t j = 0; j < 8; ++j) {
+      const uint32_t c = fc + (j < k ? j : 0u);
+      kid_n[j] = t.count[c];
+      kid_b[j] = t.begin[c];
+      kid_leaf[j] = t.leaf[c];
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < 8; ++j) {
+      if (j >= k) break;
+      const uint32_t c = fc + j, cn = kid_n[j];
+      const bool cleaf = kid_leaf[j] != 0;
       if (!cleaf && cn > thr) {
         end_run();
         continue;
@@ -699,13 +757,13 @@ __global__ __launch_bounds__(kBlock) void k_units_mark(TreeDev t, const uint16_t
       end_run();
       if (csingle) {
         run = c;
-        run_b = t.begin[c];
+        run_b = kid_b[j];
         run_n = cn;
         run_len = 1;
         if (cn > tile) end_run();
       } else {
         unit_n[c] = 0u;
-        mark_unit(gmark, c, t.begin[c], cn, upiece);
+        mark_unit(gmark, c, kid_b[j], cn, upiece);
       }
     }
     end_run();
@@ -792,7 +850,7 @@ hipError_t launch_tree_count(const uint64_t* keys, uint32_t n, const uint16_t* s
                              uint32_t max_leaf_max, uint8_t* L, uint8_t* H, uint32_t* tile_counts, hipStream_t s) {
   const uint32_t tiles = (n + kTreeTile - 1) / kTreeTile;
   const size_t lds = (kTreeTile + 2 * size_t(max_leaf_max) + 1) * sizeof(uint64_t) + kTreeTile + max_leaf_max;
-  hipLaunchKernelGGL(k_tree_count, dim3(tiles), dim3(kBlock), lds, s, keys, n, sid, sys, max_leaf_max, L, H, tile_counts);
+  hipLaunchKernelGGL(k_tree_count, dim3(tiles), dim3(kTileThreads), lds, s, keys, n, sid, sys, max_leaf_max, L, H, tile_counts);
   return hipGetLastError();
 }
 
@@ -806,7 +864,7 @@ hipError_t launch_tree_scan(const uint32_t* tile_counts, uint32_t tiles, uint32_
 hipError_t launch_tree_emit(const uint8_t* L, const uint8_t* H, uint32_t n, const uint32_t* tile_prefix, TreeDev t,
                             uint32_t depth_plan, hipStream_t s) {
   const uint32_t tiles = (n + kTreeTile - 1) / kTreeTile;
-  hipLaunchKernelGGL(k_tree_emit, dim3(tiles), dim3(kBlock), 0, s, L, H, n, tile_prefix, t, depth_plan);
+  hipLaunchKernelGGL(k_tree_emit, dim3(tiles), dim3(kTileThreads), 0, s, L, H, n, tile_prefix, t, depth_plan);
   return hipGetLastError();
 }
 
@@ -818,14 +876,18 @@ hipError_t launch_tree_finish(const uint64_t* keys, const double4* posm, uint32_
   // below the planned depth (the deepest level holds leaves only), each
   // reading its level's range on the device and grid-striding over it.
   // Level d holds at most min(n_sys * 8^d, n) nodes, which sizes its grid.
-  hipLaunchKernelGGL(k_upward_leaves, dim3(grid_for(n, 4096)), dim3(kBlock), 0, s, posm, n, t);
+  hipLaunchKernelGGL(k_upward_leaves, dim3(grid_for(uint64_t(n) * kBlock / kLeafThreads, 8192)), dim3(kLeafThreads), 0, s,
+                     posm, n, t);
   const int top = static_cast<int>(depth_plan < kDepthCap ? depth_plan : kDepthCap);
-  for (int d = top - 1; d >= 0; --d) {
+  // a single system's upper levels (at most 8^kTopLevel nodes) in one launch
+  const int single = n_sys == 1 ? (top - 1 < kTopLevel ? top - 1 : kTopLevel) : -1;
+  for (int d = top - 1; d > single; --d) {
     uint64_t bound = n_sys;
     for (int e = 0; e < d && bound < n; ++e) bound *= 8;
     if (bound > n) bound = n;
     hipLaunchKernelGGL(k_upward, dim3(grid_for(bound * kKids, 4096)), dim3(kBlock), 0, s, d, t);
   }
+  if (single >= 0) hipLaunchKernelGGL(k_upward_top, dim3(1), dim3(kTopThreads), 0, s, single, t);
   return hipGetLastError();
 }
 
