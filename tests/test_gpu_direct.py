@@ -1,0 +1,53 @@
+"""The direct sum's tiles of 256 sources, its own-source check and its two forms.
+
+Sources and targets whose distances stay finite go through the reciprocal
+square root, others (any coordinate of 1e150 or more, or not a number) through
+the square root and the division. Both against the sum in numpy's float64:
+a term of either has a relative error below 16 roundings and a sum of n terms
+one below n, so an acceleration is within (n + 16) 2^-52 of the sum of its
+terms' magnitudes."""
+import numpy as np
+import pytest
+
+from bhgpu import ic
+
+pytestmark = pytest.mark.gpu
+
+
+def reference(p, idx, eps2):
+    x, m = p["pos"].astype(np.float64), p["mass"].astype(np.float64)
+    acc, size = np.zeros((len(idx), 3)), np.zeros((len(idx), 3))
+    with np.errstate(all="ignore"):
+        for k, i in enumerate(idx):
+            d = np.delete(x, i, 0) - x[i]
+            r2 = (d * d).sum(1) + eps2
+            t = d * (np.delete(m, i) * (1.0 / (r2 * np.sqrt(r2))))[:, None]
+            acc[k], size[k] = t.sum(0), np.abs(t).sum(0)
+    return acc, size
+
+
+@pytest.mark.parametrize("n,eps2", [(1, 1e-4), (2, 0.0), (255, 1e-6), (256, 0.0), (257, 1e-4), (513, 1e300), (1500, 1e-250)])
+@pytest.mark.parametrize("wild", ["none", "far", "infinite", "nan", "heavy", "twins"])
+def test_direct_forms(gpu, n, eps2, wild):
+    p = ic.plummer(n, 3)
+    j = n // 2
+    if wild == "far":
+        p["pos"][j] = (1e160, -2e151, 0.0)
+    elif wild == "infinite":
+        p["pos"][j, 1] = np.inf
+    elif wild == "nan":
+        p["pos"][j, 2] = np.nan
+    elif wild == "heavy":
+        p["mass"][j] = np.inf
+    elif wild == "twins":  # without softening their pull is not a number
+        p["pos"][j] = p["pos"][0]
+    idx = np.unique([0, j, n - 1, n // 3, min(n - 1, 255), min(n - 1, 256)]).astype(np.uint32)
+    print(f"direct n={n} eps2={eps2} {wild}", flush=True)
+    for sel in (idx, None):
+        got = gpu.direct_sum(p, sel, eps2)
+        got = got if sel is not None else got[idx]
+        ref, size = reference(p, idx, eps2)
+        assert np.array_equal(np.isnan(got), np.isnan(ref))
+        ok = np.isfinite(ref) & np.isfinite(size)
+        assert np.array_equal(got[~ok & ~np.isnan(ref)], ref[~ok & ~np.isnan(ref)])
+        assert (np.abs(got - ref)[ok] <= ((n + 16) * 2.0 ** -52 * size)[ok]).all()
