@@ -224,6 +224,8 @@ __host__ __device__ inline uint32_t piece_size(uint32_t cnt, uint32_t piece) {
 // per-XCD queues; deep selects the variant whose stack also uses deep_frames
 // (trees of more than kShallowFrames levels).
 hipError_t launch_walk(const WalkArgs& a, uint32_t slots, bool deep, int fp64, bool any_unsoftened, hipStream_t s);
+// dst[i] = (x, y, z, m) of record i
+hipError_t launch_points(const bh_particle* p, uint32_t n, double4* dst, hipStream_t s);
 hipError_t launch_direct(const double4* src, uint32_t n, const uint32_t* tidx, uint32_t m, double eps2, double G,
                          double* partial, uint32_t splits, double* acc, hipStream_t s);
 uint32_t direct_splits(uint32_t n, uint32_t m);

@@ -1116,6 +1116,11 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(4))
   }
 }
 
+__global__ __launch_bounds__(256) void k_points(const bh_particle* __restrict__ p, uint32_t n, double4* __restrict__ dst) {
+  const uint32_t i = blockIdx.x * 256 + threadIdx.x;
+  if (i < n) dst[i] = make_double4(p[i].pos[0], p[i].pos[1], p[i].pos[2], p[i].mass);
+}
+
 // One source's pull on a target, in FP64: G is applied at the end.
 // The general form, for any operands.
 __device__ __forceinline__ void direct_term(const double4& t, const double4& q, double eps2, double (&a)[3]) {
@@ -1211,6 +1216,7 @@ __global__ __launch_bounds__(256) void k_direct_reduce(const double* __restrict_
   const uint32_t k = blockIdx.x * 256 + threadIdx.x;
   if (k >= m) return;
   double a0 = 0.0, a1 = 0.0, a2 = 0.0;
+#pragma unroll 16
   for (uint32_t s = 0; s < splits; ++s) {
     const double* o = &partial[(uint64_t(s) * m + k) * 3];
     a0 += o[0];
@@ -1328,6 +1334,12 @@ hipError_t launch_walk(const WalkArgs& a, uint32_t slots, bool deep, int fp64, b
   // per workgroup: 49.7 ms at 16M, 4: 53.9, 8: 64.8; 1: 47.0).
   return fp64 ? launch_walk_t<double, 1>(a, slots, deep, any_unsoftened, s)
               : launch_walk_t<float, 1>(a, slots, deep, any_unsoftened, s);
+}
+
+hipError_t launch_points(const bh_particle* p, uint32_t n, double4* dst, hipStream_t s) {
+  if (n == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_points, dim3((n + 255) / 256), dim3(256), 0, s, p, n, dst);
+  return hipGetLastError();
 }
 
 hipError_t launch_potential(const double4* src, uint32_t n, double* partial, uint32_t splits, hipStream_t s) {

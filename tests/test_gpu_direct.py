@@ -51,3 +51,13 @@ def test_direct_forms(gpu, n, eps2, wild):
         ok = np.isfinite(ref) & np.isfinite(size)
         assert np.array_equal(got[~ok & ~np.isnan(ref)], ref[~ok & ~np.isnan(ref)])
         assert (np.abs(got - ref)[ok] <= ((n + 16) * 2.0 ** -52 * size)[ok]).all()
+
+
+def test_records_loaded_in_pieces(gpu):
+    """Records go to the GPU 2^20 at a time; the last piece holds three."""
+    n = (1 << 20) + 3
+    p = ic.uniform_cube(n, 4)
+    idx = np.array([0, (1 << 20) - 1, 1 << 20, n - 1], np.uint32)
+    print(f"direct n={n}", flush=True)
+    ref, size = reference(p, idx, 1e-6)
+    assert (np.abs(gpu.direct_sum(p, idx, 1e-6) - ref) <= (n + 16) * 2.0 ** -52 * size).all()
