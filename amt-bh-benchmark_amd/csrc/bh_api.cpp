@@ -92,7 +92,8 @@ struct Scratch {
 struct Plan {
   uint32_t n = 0;         // particles of all systems
   uint32_t S = 0;         // non-empty systems
-  uint32_t n_chunks = 0;  // bounds blocks
+  uint32_t n_chunks = 0;  // bounds blocks ...
+  uint32_t chunk = kChunk;  // ... of at most this many particles
   uint32_t mlx = 0;       // largest max_leaf
   int sid_passes = 0;     // radix passes over the system id
   int key_passes = 8;     // radix passes over the keys' leading bits (8: all of them)
@@ -129,8 +130,8 @@ constexpr size_t kGraphCache = 256;
 struct Ctx {
   int device = 0;
   hipStream_t stream = nullptr;
-  // events: 0 step start, 1 sorted, 2 tree built, 3 targets chosen, 4 walk start, 5 walk (step) end
-  hipEvent_t ev[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+  double clock_khz = 0.0;   // rate of the GPU's constant clock
+  unsigned long long stamps[kStamps] = {};  // when the last step's phases began
   bool have_stats = false;
   bool last_graph = false;  // the last step ran as a graph: only its total time is known
   uint32_t reruns = 0;      // times the last step ran again with larger arrays
@@ -158,7 +159,6 @@ struct Ctx {
   DevBuf<uint32_t> hist, lookback;
   DevBuf<double> lohi, partial;
   DevBuf<uint32_t> misc;
-  DevBuf<unsigned long long> totals;
   DevBuf<double4> posm;
   DevBuf<uint8_t> L, H;
   DevBuf<uint32_t> tcounts, tprefix;
@@ -178,7 +178,7 @@ struct Ctx {
   DevBuf<uint32_t> didx, dcnt;
   DevBuf<double> dpart, dacc;
 
-  uint32_t* host_misc = nullptr;  // pinned: kMiscWords flag/count words, then the two totals
+  uint32_t* host_misc = nullptr;  // pinned: the last step's report (kReportWords)
   uint8_t* host_tables = nullptr; // pinned system table staging
   size_t host_tables_cap = 0;
   uint64_t gen = 1;               // bumped whenever a buffer a graph may hold moves
@@ -358,8 +358,8 @@ int host_table_room(Ctx* c, size_t bytes, bool no_grow) {
 
 // The batch's system table: per-system parameters, chunks of <= kChunk
 // particles for the per-system bounds, and the system-id digit counts of the
-// sort's last passes, written to the pinned staging (the step uploads it
-// with one copy). Empty systems take no part: the device table lists the
+// sort's last passes, written to the pinned staging (the step's first kernel
+// reads it there). Empty systems take no part: the device table lists the
 // others, in order, and a particle's system id indexes that list.
 int plan_systems(Ctx* c, const HostSys* sys, uint32_t S, bool no_grow, Plan* p) {
   if (S == 0 || S > kMaxSystems) {
@@ -379,7 +379,6 @@ int plan_systems(Ctx* c, const HostSys* sys, uint32_t S, bool no_grow, Plan* p) 
     if (sys[k].n == 0) continue;
     ++live;
     n += sys[k].n;
-    chunks += (sys[k].n + kChunk - 1) / kChunk;
     mlx = std::max(mlx, sys[k].max_leaf);
     largest = std::max(largest, sys[k].n);
     unsoftened |= static_cast<float>(sys[k].fp.eps2) == 0.0f;  // zero in the FP32 walk too
@@ -391,8 +390,13 @@ int plan_systems(Ctx* c, const HostSys* sys, uint32_t S, bool no_grow, Plan* p) 
     set_err(c, "batch of %llu particles exceeds the supported %llu", (unsigned long long)n, (unsigned long long)kMaxN);
     return BH_ERR_TOO_LARGE;
   }
+  // up to 256 chunks of a quarter, so that a small system's bounds reach
+  // more CUs; the allocation-free step's table has room for full ones
+  const uint32_t chunk = !no_grow && n <= 64 * kChunk ? kChunk / 4 : kChunk;
+  for (uint32_t k = 0; k < S; ++k) chunks += (sys[k].n + chunk - 1) / chunk;
   *p = Plan{};
   p->n = static_cast<uint32_t>(n);
+  p->chunk = chunk;
   p->largest = largest;
   if (n == 0) return BH_OK;
   p->S = live;
@@ -430,8 +434,8 @@ int plan_systems(Ctx* c, const HostSys* sys, uint32_t S, bool no_grow, Plan* p) 
     sd[k].unit_piece = pieces.unit;
     sd[k].target_piece = pieces.target;
     first[k] = static_cast<uint32_t>(ci);
-    for (uint64_t b = 0; b < h.n; b += kChunk)
-      ch[ci++] = make_uint4(k, static_cast<uint32_t>(off + b), static_cast<uint32_t>(off + std::min<uint64_t>(h.n, b + kChunk)), 0);
+    for (uint64_t b = 0; b < h.n; b += chunk)
+      ch[ci++] = make_uint4(k, static_cast<uint32_t>(off + b), static_cast<uint32_t>(off + std::min<uint64_t>(h.n, b + chunk)), 0);
     hist[k & 255] += static_cast<uint32_t>(h.n);
     hist[256 + (k >> 8)] += static_cast<uint32_t>(h.n);
     off += h.n;
@@ -488,8 +492,7 @@ int provision(Ctx* c, const Plan& p, Scratch* b) {
   TRY(ensure(c, c->lookback, radix_lookback_words(n), "look-back"));
   TRY(ensure(c, c->lohi, 6ull * p.S, "bounds"));
   TRY(ensure(c, c->partial, 6ull * p.n_chunks, "bounds"));
-  TRY(ensure(c, c->misc, kMiscWords, "flags"));
-  TRY(ensure(c, c->totals, 2, "totals"));
+  TRY(ensure(c, c->misc, kReportWords, "flags"));
   TRY(ensure(c, c->posm, n, "walk copy"));
   TRY(ensure(c, c->L, n, "tree build"));
   TRY(ensure(c, c->H, n, "tree build"));
@@ -541,7 +544,7 @@ int provision(Ctx* c, const Plan& p, Scratch* b) {
   s.lohi = c->lohi.p;
   s.partial = c->partial.p;
   s.misc = c->misc.p;
-  s.totals = c->totals.p;
+  s.totals = reinterpret_cast<unsigned long long*>(s.misc + kMiscTotals);
   s.posm = c->posm.p;
   s.L = c->L.p;
   s.H = c->H.p;
@@ -609,8 +612,8 @@ bool carve(uint8_t* base, size_t bytes, Plan* p, Scratch* b) {
   s.lookback = reinterpret_cast<uint32_t*>(take(4 * radix_lookback_words(n)));
   s.lohi = reinterpret_cast<double*>(take(48ull * p->S));
   s.partial = reinterpret_cast<double*>(take(48ull * p->n_chunks));
-  s.misc = reinterpret_cast<uint32_t*>(take(4 * kMiscWords));
-  s.totals = reinterpret_cast<unsigned long long*>(take(16));
+  s.misc = reinterpret_cast<uint32_t*>(take(4 * kReportWords));
+  s.totals = reinterpret_cast<unsigned long long*>(s.misc + kMiscTotals);
   s.posm = reinterpret_cast<double4*>(take(32ull * n));
   s.L = take(n);
   s.H = take(n);
@@ -667,40 +670,49 @@ struct Sorted {
 // build_flat_tree (flat_build_ttg.h:276-281) of every system of the plan,
 // d_in[0..n) into the scratch; the Morton-ordered particles (each system in
 // its own range) go to d_out, here or (walk_writes_out) by the step's walk,
-// which reads them from d_in. `events`: record the phase events.
-int enqueue_build(Ctx* c, const Plan& p, const Scratch& b, const bh_particle* d_in, bh_particle* d_out, bool events,
-                  Sorted* out, bool walk_writes_out) {
+// which reads them from d_in.
+int enqueue_build(Ctx* c, const Plan& p, const Scratch& b, const bh_particle* d_in, bh_particle* d_out, Sorted* out,
+                  bool walk_writes_out) {
   hipStream_t s = c->stream;
   const uint32_t n = p.n;
   const uint32_t tiles = (n + kTreeTile - 1) / kTreeTile;
-  const uint4* chunks = reinterpret_cast<const uint4*>(b.tables + p.off_chunks);
-  const uint32_t* chunk_first = reinterpret_cast<const uint32_t*>(b.tables + p.off_first);
   const SysDev* sys = reinterpret_cast<const SysDev*>(b.tables);
   const uint64_t lb_words = radix_lookback_words(n);
-  HIP_OK(c, hipMemcpyAsync(b.tables, c->host_tables, p.table_bytes, hipMemcpyHostToDevice, s));
-  {
-    // the step's flag words, totals, key digit histograms and look-back
-    // words, in one launch
-    ZeroRanges z;
-    z.p[0] = b.misc;
-    z.n[0] = kMiscWords;
-    z.p[1] = reinterpret_cast<uint32_t*>(b.totals);
-    z.n[1] = 4;
-    z.p[2] = b.hist;
-    z.n[2] = 8 * 256;
-    z.p[3] = b.lookback;
-    z.n[3] = lb_words;
-    HIP_OK(c, launch_zero(z, s));
+  StartArgs a{};
+  a.host_table = reinterpret_cast<const uint4*>(c->host_tables);
+  a.table = reinterpret_cast<uint4*>(b.tables);
+  a.table_quads = static_cast<uint32_t>(p.off_hist / sizeof(uint4));
+  if (p.sid_passes) a.host_hist = reinterpret_cast<const uint4*>(c->host_tables + p.off_hist);
+  a.hist = reinterpret_cast<uint4*>(b.hist + 8 * 256);
+  // the step's flag words and totals, key digit histograms and look-back
+  // words, and the walk's marks
+  a.zero.p[0] = b.misc;
+  a.zero.n[0] = kMiscStamps;
+  a.zero.p[1] = b.hist;
+  a.zero.n[1] = 8 * 256;
+  a.zero.p[2] = b.lookback;
+  a.zero.n[2] = lb_words;
+  if (p.walk) {
+    a.zero.p[3] = b.mark;
+    a.zero.n[3] = n;
+    a.zero.p[4] = b.gmark;
+    a.zero.n[4] = n;
   }
-  if (p.sid_passes)
-    HIP_OK(c, hipMemcpyAsync(b.hist + 8 * 256, c->host_tables + p.off_hist, 2 * 256 * 4, hipMemcpyHostToDevice, s));
-  HIP_OK(c, launch_fill_sid(chunks, p.n_chunks, b.sid, s));
+  a.host_chunks = reinterpret_cast<const uint4*>(c->host_tables + p.off_chunks);
+  a.chunk_first = reinterpret_cast<const uint32_t*>(b.tables + p.off_first);
+  a.n_chunks = p.n_chunks;
+  a.n_sys = p.S;
+  a.n = n;
+  a.chunk = p.chunk;
+  a.sid = b.sid;
+  a.partial = b.partial;
+  a.lohi = b.lohi;
+  a.misc = b.misc;
   if (p.carried_in) {
-    HIP_OK(c, launch_bounds(c->carry.p, n, c->carry_flag.p, chunks, p.n_chunks, chunk_first, p.S, b.partial,
-                            b.misc + kMiscNonfinite, b.lohi, s));
+    HIP_OK(c, launch_start(c->carry.p, c->carry_flag.p, a, s));
     HIP_OK(c, launch_keys_hist(c->carry.p, n, p.key_passes, b.sid, b.lohi, b.keys_a, b.hist, s));
   } else {
-    HIP_OK(c, launch_bounds(d_in, chunks, p.n_chunks, chunk_first, p.S, b.partial, b.misc + kMiscNonfinite, b.lohi, s));
+    HIP_OK(c, launch_start(d_in, a, s));
     HIP_OK(c, launch_keys_hist(d_in, n, p.key_passes, b.sid, b.lohi, b.keys_a, b.hist, s));
   }
   HIP_OK(c, launch_radix_sort(b.keys_a, b.vals_a, b.keys_b, b.vals_b, n, p.key_passes, p.sid_passes, b.sid, b.hist,
@@ -709,49 +721,35 @@ int enqueue_build(Ctx* c, const Plan& p, const Scratch& b, const bh_particle* d_
     HIP_OK(c, launch_gather(c->carry.p, out->perm, b.posm, n, s));
   else
     HIP_OK(c, launch_gather(d_in, walk_writes_out ? nullptr : d_out, out->perm, b.posm, n, s));
-  if (events) HIP_OK(c, hipEventRecord(c->ev[1], s));
-  HIP_OK(c, launch_tree_count(out->keys, n, b.sid, sys, p.mlx, b.L, b.H, b.tcounts, s));
+  HIP_OK(c, launch_tree_count(out->keys, n, b.sid, sys, p.mlx, b.L, b.H, b.tcounts, b.misc, s));
   HIP_OK(c, launch_tree_scan(b.tcounts, tiles, b.tprefix, b.misc + kMiscLevels, s));
   HIP_OK(c, launch_tree_emit(b.L, b.H, n, b.tprefix, b.t, p.depth_plan, s));
-  HIP_OK(c, launch_tree_finish(out->keys, b.posm, n, b.sid, p.S, b.lohi, p.depth_plan, b.t, s));
-  if (events) HIP_OK(c, hipEventRecord(c->ev[2], s));
+  // what the walk needs zeroed and could not be before: unit_lb may lie over
+  // tcounts, and the carried flag has been read
+  ZeroRanges z;
+  if (p.walk) {
+    z.p[0] = b.unit_lb;
+    z.n[0] = unit_list_words(n);
+  }
+  if (p.walk && p.carry_out) {
+    z.p[1] = c->carry_flag.p;
+    z.n[1] = 1;
+  }
+  HIP_OK(c, launch_tree_finish(out->keys, b.posm, n, b.sid, p.S, b.lohi, p.depth_plan, z, b.t, s));
   return BH_OK;
 }
 
 // run_grouped_pass (grouped_ttg.h:297-323) over every system of the tree in
-// the scratch, with each system's parameters from the system table.
+// the scratch, with each system's parameters from the system table. The build
+// zeroed what it and the unit list need zero.
 int enqueue_walk(Ctx* c, const Plan& p, const Scratch& b, bh_particle* parts, double* d_acc, uint32_t* d_npp,
-                 uint32_t* d_npc, bool events, const bh_particle* src = nullptr, const uint32_t* perm = nullptr) {
+                 uint32_t* d_npc, const bh_particle* src = nullptr, const uint32_t* perm = nullptr) {
   hipStream_t s = c->stream;
   const uint32_t n = p.n;
   const SysDev* sys = reinterpret_cast<const SysDev*>(b.tables);
   const bool grouped = c->walk_mode == BH_WALK_GROUPED;
-  // what the unit list and the walk need zeroed, in one launch (a walk on its
-  // own, bh_accel, clears what an earlier walk left)
-  {
-    ZeroRanges z;
-    z.p[0] = b.misc + kMiscIncomplete;
-    z.n[0] = 1;
-    z.p[1] = b.misc + kMiscTargets;
-    z.n[1] = kMiscQueue + 8 - kMiscTargets;  // target and unit counts, queue heads
-    z.p[2] = reinterpret_cast<uint32_t*>(b.totals);
-    z.n[2] = 4;
-    z.p[3] = b.mark;
-    z.n[3] = n;
-    z.p[4] = b.gmark;
-    z.n[4] = n;
-    z.p[5] = b.unit_lb;
-    z.n[5] = unit_list_words(n);
-    if (parts && p.carry_out) {
-      // read by this step's build already (carried_in)
-      z.p[6] = c->carry_flag.p;
-      z.n[6] = 1;
-    }
-    HIP_OK(c, launch_zero(z, s));
-  }
   // per-target mode: the walk units are the targets themselves
   HIP_OK(c, launch_units(b.t, n, b.sid, sys, grouped, b.mark, b.gmark, b.unit_n, b.unit_lb, b.units, s));
-  if (events) HIP_OK(c, hipEventRecord(c->ev[3], s));
   WalkArgs a;
   a.rec = b.t.rec;
   a.q64 = b.t.q64;
@@ -785,20 +783,26 @@ int enqueue_walk(Ctx* c, const Plan& p, const Scratch& b, bh_particle* parts, do
   a.n_pp = d_npp;
   a.n_pc = d_npc;
   a.totals = b.totals;
-  if (events) HIP_OK(c, hipEventRecord(c->ev[4], s));
   HIP_OK(c, launch_walk(a, p.slots, p.deep, c->precision == BH_FP64, p.unsoftened, s));
-  if (events) HIP_OK(c, hipEventRecord(c->ev[5], s));
   return BH_OK;
 }
 
-// Copies the flag/count words and the totals to the pinned report and
-// waits for the stream: the step's only synchronisation.
-int finish(Ctx* c, const Scratch& b) {
-  HIP_OK(c, hipMemcpyAsync(c->host_misc, b.misc, kMiscWords * sizeof(uint32_t), hipMemcpyDeviceToHost, c->stream));
-  HIP_OK(c, hipMemcpyAsync(c->host_misc + kMiscWords, b.totals, 2 * sizeof(unsigned long long), hipMemcpyDeviceToHost,
-                           c->stream));
-  HIP_OK(c, hipStreamSynchronize(c->stream));
+int enqueue_report(Ctx* c, const Scratch& b) {
+  HIP_OK(c, launch_report(b.misc, c->host_misc, c->stream));
   return BH_OK;
+}
+
+// Waits for the stream, whose last kernel wrote the report: the step's only
+// synchronisation.
+int finish(Ctx* c) {
+  HIP_OK(c, hipStreamSynchronize(c->stream));
+  std::memcpy(c->stamps, c->host_misc + kMiscStamps, sizeof c->stamps);
+  return BH_OK;
+}
+
+// Milliseconds from the beginning of one phase of the last step to another's.
+double phase_ms(const Ctx* c, Stamp from, Stamp to) {
+  return static_cast<double>(c->stamps[to] - c->stamps[from]) / c->clock_khz;
 }
 
 GraphKey graph_key(const Ctx* c, const Plan& p, const void* in, const void* out) {
@@ -840,8 +844,9 @@ int launch_graph(Ctx* c, const Plan& p, const Scratch& b, const bh_particle* d_i
   if (!hit) {
     HIP_OK(c, hipStreamBeginCapture(c->stream, hipStreamCaptureModeRelaxed));
     Sorted sd;
-    int rc = enqueue_build(c, p, b, d_in, d_out, false, &sd, true);
-    if (rc == BH_OK) rc = enqueue_walk(c, p, b, d_out, nullptr, nullptr, nullptr, false, d_in, sd.perm);
+    int rc = enqueue_build(c, p, b, d_in, d_out, &sd, true);
+    if (rc == BH_OK) rc = enqueue_walk(c, p, b, d_out, nullptr, nullptr, nullptr, d_in, sd.perm);
+    if (rc == BH_OK) rc = enqueue_report(c, b);
     hipGraph_t graph = nullptr;
     const hipError_t ec = hipStreamEndCapture(c->stream, &graph);
     if (rc != BH_OK) {
@@ -868,19 +873,8 @@ int launch_graph(Ctx* c, const Plan& p, const Scratch& b, const bh_particle* d_i
     hit = &c->graphs.back();
   }
   hit->used = ++c->graph_clock;
-  HIP_OK(c, hipEventRecord(c->ev[0], c->stream));
   HIP_OK(c, hipGraphLaunch(hit->exec, c->stream));
-  HIP_OK(c, hipEventRecord(c->ev[5], c->stream));
   return BH_OK;
-}
-
-float elapsed(hipEvent_t a, hipEvent_t b) {
-  float ms = 0.f;
-  if (hipEventElapsedTime(&ms, a, b) != hipSuccess) {
-    (void)hipGetLastError();
-    return 0.f;
-  }
-  return ms;
 }
 
 // Keeps the report of a finished step or build.
@@ -921,11 +915,11 @@ int run(Ctx* c, Plan p, const bh_particle* d_in, bh_particle* d_out, bool walk, 
     if (graph) {
       TRY(launch_graph(c, p, b, d_in, d_out, &sd));
     } else {
-      HIP_OK(c, hipEventRecord(c->ev[0], c->stream));
-      TRY(enqueue_build(c, p, b, d_in, d_out, true, &sd, walk));
-      if (walk) TRY(enqueue_walk(c, p, b, d_out, nullptr, nullptr, nullptr, true, d_in, sd.perm));
+      TRY(enqueue_build(c, p, b, d_in, d_out, &sd, walk));
+      if (walk) TRY(enqueue_walk(c, p, b, d_out, nullptr, nullptr, nullptr, d_in, sd.perm));
+      TRY(enqueue_report(c, b));
     }
-    TRY(finish(c, b));
+    TRY(finish(c));
     const uint32_t* m = c->host_misc;
     if (m[kMiscNonfinite]) {
       set_err(c, "non-finite position, velocity or mass in the input");
@@ -961,10 +955,10 @@ int run(Ctx* c, Plan p, const bh_particle* d_in, bh_particle* d_out, bool walk, 
     if (timing) {
       if (graph) {
         timing->tree_build_ms = 0.0;
-        timing->traversal_ms = elapsed(c->ev[0], c->ev[5]);  // the whole step: a graph has no inner events
+        timing->traversal_ms = phase_ms(c, kStampStart, kStampEnd);  // of a graph the whole step is reported
       } else {
-        timing->tree_build_ms = elapsed(c->ev[0], c->ev[2]);
-        timing->traversal_ms = walk ? elapsed(c->ev[2], c->ev[5]) : 0.0;
+        timing->tree_build_ms = phase_ms(c, kStampStart, walk ? kStampTargets : kStampEnd);
+        timing->traversal_ms = walk ? phase_ms(c, kStampTargets, kStampEnd) : 0.0;
       }
       timing->exchange_ms = 0.0;
     }
@@ -1119,11 +1113,13 @@ int bh_ctx_create(bh_ctx** out, int device) {
   // pinned staging sized so that a one-system table of the allocation-free
   // step never has to grow
   const size_t table0 = 64 << 10;
+  int khz = 0;
   if (hipSetDevice(device) != hipSuccess || hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess ||
-      hipHostMalloc(reinterpret_cast<void**>(&c->host_misc), (kMiscWords + 4) * sizeof(uint32_t), hipHostMallocDefault) !=
+      hipHostMalloc(reinterpret_cast<void**>(&c->host_misc), kReportWords * sizeof(uint32_t), hipHostMallocDefault) !=
           hipSuccess ||
       hipHostMalloc(reinterpret_cast<void**>(&c->host_tables), table0, hipHostMallocDefault) != hipSuccess ||
-      scratch_address(device, &c->arena) != hipSuccess) {
+      scratch_address(device, &c->arena) != hipSuccess ||
+      hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device) != hipSuccess || khz <= 0) {
     (void)hipGetLastError();
     if (c->host_tables) (void)hipHostFree(c->host_tables);
     if (c->host_misc) (void)hipHostFree(c->host_misc);
@@ -1132,18 +1128,7 @@ int bh_ctx_create(bh_ctx** out, int device) {
     return BH_ERR_HIP;
   }
   c->host_tables_cap = table0;
-  for (auto& e : c->ev) {
-    if (hipEventCreate(&e) != hipSuccess) {
-      (void)hipGetLastError();
-      for (auto& f : c->ev)
-        if (f) (void)hipEventDestroy(f);
-      (void)hipHostFree(c->host_tables);
-      (void)hipHostFree(c->host_misc);
-      (void)hipStreamDestroy(c->stream);
-      delete c;
-      return BH_ERR_HIP;
-    }
-  }
+  c->clock_khz = khz;
   *out = reinterpret_cast<bh_ctx*>(c);
   return BH_OK;
 }
@@ -1169,7 +1154,6 @@ void bh_ctx_destroy(bh_ctx* h) {
   release(c->lohi);
   release(c->partial);
   release(c->misc);
-  release(c->totals);
   release(c->posm);
   release(c->L);
   release(c->H);
@@ -1211,8 +1195,6 @@ void bh_ctx_destroy(bh_ctx* h) {
   release(c->dpart);
   release(c->dacc);
   if (c->host_tables) (void)hipHostFree(c->host_tables);
-  for (auto& e : c->ev)
-    if (e) (void)hipEventDestroy(e);
   if (c->host_misc) (void)hipHostFree(c->host_misc);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
@@ -1339,10 +1321,10 @@ int bh_step_device_noalloc(bh_ctx* h, const bh_particle* d_in, bh_particle* d_ou
   c->have_stats = false;
   c->reruns = 0;
   Sorted sd;
-  HIP_OK(c, hipEventRecord(c->ev[0], c->stream));
-  TRY(enqueue_build(c, p, b, d_in, d_out, true, &sd, true));
-  TRY(enqueue_walk(c, p, b, d_out, nullptr, nullptr, nullptr, true, d_in, sd.perm));
-  TRY(finish(c, b));
+  TRY(enqueue_build(c, p, b, d_in, d_out, &sd, true));
+  TRY(enqueue_walk(c, p, b, d_out, nullptr, nullptr, nullptr, d_in, sd.perm));
+  TRY(enqueue_report(c, b));
+  TRY(finish(c));
   const uint32_t* m = c->host_misc;
   if (m[kMiscNonfinite]) {
     set_err(c, "non-finite position, velocity or mass in the input");
@@ -1365,8 +1347,8 @@ int bh_step_device_noalloc(bh_ctx* h, const bh_particle* d_in, bh_particle* d_ou
   c->have_stats = true;
   c->last_graph = false;
   if (timing) {
-    timing->tree_build_ms = elapsed(c->ev[0], c->ev[2]);
-    timing->traversal_ms = elapsed(c->ev[2], c->ev[5]);
+    timing->tree_build_ms = phase_ms(c, kStampStart, kStampTargets);
+    timing->traversal_ms = phase_ms(c, kStampTargets, kStampEnd);
   }
   if (m[kMiscIncomplete]) {
     set_err(c, "incomplete tree: the walk met an interior node it could not open");
@@ -1683,11 +1665,23 @@ int bh_accel(bh_ctx* h, const bh_force_params* fp, uint32_t target_size, double*
   HIP_OK(c, hipMemcpyAsync(b.tables, c->host_tables, sizeof(SysDev), hipMemcpyHostToDevice, c->stream));
   c->have_stats = false;
   c->reruns = 0;
-  HIP_OK(c, hipEventRecord(c->ev[0], c->stream));
-  HIP_OK(c, hipEventRecord(c->ev[1], c->stream));
-  HIP_OK(c, hipEventRecord(c->ev[2], c->stream));
-  TRY(enqueue_walk(c, p, b, nullptr, c->dacc.p, c->dcnt.p, c->dcnt.p + n, true));
-  TRY(finish(c, b));
+  // what the build, or an earlier walk, left
+  ZeroRanges z;
+  z.p[0] = b.misc + kMiscIncomplete;
+  z.n[0] = 1;
+  z.p[1] = b.misc + kMiscTargets;
+  z.n[1] = kMiscStamps - kMiscTargets;  // target and unit counts, queue heads, totals
+  z.p[2] = b.mark;
+  z.n[2] = n;
+  z.p[3] = b.gmark;
+  z.n[3] = n;
+  z.p[4] = b.unit_lb;
+  z.n[4] = unit_list_words(n);
+  HIP_OK(c, launch_zero(z, c->stream));
+  TRY(enqueue_walk(c, p, b, nullptr, c->dacc.p, c->dcnt.p, c->dcnt.p + n));
+  TRY(enqueue_report(c, b));
+  TRY(finish(c));
+  c->stamps[kStampStart] = c->stamps[kStampTree] = c->stamps[kStampTargets];
   const uint32_t* m = c->host_misc;
   c->n_targets = m[kMiscTargets];
   c->n_groups = m[kMiscGroups];
@@ -1719,12 +1713,12 @@ int bh_last_step_stats(bh_ctx* h, bh_step_stats* st) {
   if (c->last_graph) {
     st->sort_ms = st->tree_ms = st->targets_ms = st->walk_ms = 0.0;
   } else {
-    st->sort_ms = elapsed(c->ev[0], c->ev[1]);
-    st->tree_ms = elapsed(c->ev[1], c->ev[2]);
-    st->targets_ms = elapsed(c->ev[2], c->ev[3]);
-    st->walk_ms = elapsed(c->ev[4], c->ev[5]);
+    st->sort_ms = phase_ms(c, kStampStart, kStampTree);
+    st->tree_ms = phase_ms(c, kStampTree, kStampTargets);
+    st->targets_ms = phase_ms(c, kStampTargets, kStampWalk);
+    st->walk_ms = phase_ms(c, kStampWalk, kStampEnd);
   }
-  st->step_ms = elapsed(c->ev[0], c->ev[5]);
+  st->step_ms = phase_ms(c, kStampStart, kStampEnd);
   st->n_pp = c->last_totals[0];
   st->n_pc = c->last_totals[1];
   st->n_nodes = c->n_nodes;

@@ -41,7 +41,7 @@ struct SysDev {
 };
 static_assert(sizeof(SysDev) == 64, "SysDev layout");
 
-constexpr uint32_t kChunk = 4096;    // particles per bounds block
+constexpr uint32_t kChunk = 4096;    // particles per bounds block, at most
 constexpr uint32_t kMaxSystems = 65535;
 constexpr uint64_t kMaxN = (1ull << 30) - 1;  // particles per step (all systems)
 constexpr uint32_t kGroupCap = 128;  // largest walk tile: a walk unit's particles fill at most two slots per lane
@@ -64,6 +64,14 @@ constexpr int kMiscTargets = 40;    // walk targets
 constexpr int kMiscGroups = 41;     // walk units
 constexpr int kMiscQueue = 48;      // [48, 56): walk-unit queue heads, one per XCD
 constexpr int kMiscWords = 64;
+// Behind them the two 64-bit interaction totals and the times (of the GPU's
+// constant-rate clock) at which the step's phases began: start, tree, targets,
+// walk, and the report that ends the step.
+constexpr int kMiscTotals = kMiscWords;
+constexpr int kMiscStamps = kMiscTotals + 4;
+constexpr int kStamps = 5;
+enum Stamp { kStampStart, kStampTree, kStampTargets, kStampWalk, kStampEnd };
+constexpr int kReportWords = kMiscStamps + 2 * kStamps;
 constexpr uint32_t kAbortNodes = 1;  // more nodes or leaves than the node arrays hold
 constexpr uint32_t kAbortDepth = 2;  // deeper than the levels the upward pass launched
 constexpr uint32_t kAbortSort = 4;   // too many keys share the sort's leading bits
@@ -141,28 +149,56 @@ struct WalkArgs {
 // ---- bh_sort.hip
 // Up to kMax device ranges of 32-bit words to zero (unused: n = 0).
 struct ZeroRanges {
-  static constexpr int kMax = 8;
+  static constexpr int kMax = 6;
   uint32_t* p[kMax] = {};
   uint64_t n[kMax] = {};
 };
 hipError_t launch_zero(const ZeroRanges& r, hipStream_t s);
+__device__ inline void zero_ranges(const ZeroRanges& r, uint64_t t, uint64_t threads) {
+#pragma unroll
+  for (int k = 0; k < ZeroRanges::kMax; ++k) {
+    // 16 bytes at a time where the range allows it
+    uint32_t* p = r.p[k];
+    const uint64_t quads = (reinterpret_cast<uintptr_t>(p) & 15u) ? 0 : r.n[k] / 4;
+    for (uint64_t i = t; i < quads; i += threads) reinterpret_cast<uint4*>(p)[i] = make_uint4(0u, 0u, 0u, 0u);
+    for (uint64_t i = 4 * quads + t; i < r.n[k]; i += threads) p[i] = 0u;
+  }
+}
+// The time at which a phase's first workgroup begins, into the report.
+__device__ inline void stamp(uint32_t* misc, Stamp which) {
+  if (blockIdx.x == 0 && threadIdx.x == 0)
+    reinterpret_cast<unsigned long long*>(misc + kMiscStamps)[which] = wall_clock64();
+}
 
-// chunks[c] = {system, begin, end, 0}: blocks of <= kChunk particles of one
-// system; chunk_first[s] = first chunk of system s (chunk_first[S] = total).
-hipError_t launch_fill_u32(uint32_t* p, uint32_t value, uint64_t n, hipStream_t s);
-hipError_t launch_fill_sid(const uint4* chunks, uint32_t n_chunks, uint16_t* sid, hipStream_t s);
-hipError_t launch_bounds(const bh_particle* p, const uint4* chunks, uint32_t n_chunks, const uint32_t* chunk_first,
-                         uint32_t n_sys, double* partial, uint32_t* nonfinite, double* lohi, hipStream_t s);
+// The step's first launches: the system table read from the host, everything
+// that a step needs zeroed, every particle's system, and the bounds.
+struct StartArgs {
+  const uint4* host_table;   // pinned host memory: the system table ...
+  uint4* table;              // ... and where the device keeps it
+  uint32_t table_quads;
+  const uint4* host_hist;    // pinned: digit counts of the system ids (null: one system)
+  uint4* hist;
+  ZeroRanges zero;
+  const uint4* host_chunks;  // [n_chunks] in the host's table: {system, begin, end, 0}, particles of one system
+  const uint32_t* chunk_first;  // [n_sys + 1] in the device's table: first chunk of each system, then n_chunks
+  uint32_t n_chunks, n_sys;
+  uint32_t n, chunk;         // one system: chunk c is [c * chunk, min(n, (c + 1) * chunk)), not read from the host
+  uint16_t* sid;             // [n]
+  double* partial;           // [6 n_chunks]
+  double* lohi;              // [6 n_sys]
+  uint32_t* misc;
+};
+hipError_t launch_start(const bh_particle* p, const StartArgs& a, hipStream_t s);
+// The step's last: the report (misc, totals, stamps) to pinned host memory.
+hipError_t launch_report(uint32_t* misc, uint32_t* host, hipStream_t s);
 // Keys, and the histograms of their `passes` leading 8-bit digits.
 hipError_t launch_keys_hist(const bh_particle* p, uint32_t n, int passes, const uint16_t* sid, const double* lohi,
                             uint64_t* keys, uint32_t* hist, hipStream_t s);
 // The same from the compact copy a resident step's walk wrote for its
 // output (the next step's input): blocks of n x, y, z and m, of which these
 // read x, y, z (24 of the records' 64 bytes). carried_bad: that walk's
-// non-finite flag, added to nonfinite.
-hipError_t launch_bounds(const double* pos, uint32_t n, const uint32_t* carried_bad, const uint4* chunks,
-                         uint32_t n_chunks, const uint32_t* chunk_first, uint32_t n_sys, double* partial,
-                         uint32_t* nonfinite, double* lohi, hipStream_t s);
+// non-finite flag, added to misc[kMiscNonfinite].
+hipError_t launch_start(const double* pos, const uint32_t* carried_bad, const StartArgs& a, hipStream_t s);
 hipError_t launch_keys_hist(const double* pos, uint32_t n, int passes, const uint16_t* sid, const double* lohi,
                             uint64_t* keys, uint32_t* hist, hipStream_t s);
 // key_passes passes over the keys' leading bits, sid_passes (0-2) over the
@@ -185,7 +221,8 @@ uint64_t radix_lookback_words(uint32_t n);  // 10 passes of look-back words + 10
 
 // ---- bh_tree.hip
 hipError_t launch_tree_count(const uint64_t* keys, uint32_t n, const uint16_t* sid, const SysDev* sys,
-                             uint32_t max_leaf_max, uint8_t* L, uint8_t* H, uint32_t* tile_counts, hipStream_t s);
+                             uint32_t max_leaf_max, uint8_t* L, uint8_t* H, uint32_t* tile_counts, uint32_t* misc,
+                             hipStream_t s);
 hipError_t launch_tree_scan(const uint32_t* tile_counts, uint32_t tiles, uint32_t* tile_prefix, uint32_t* totals,
                             hipStream_t s);
 // Numbers the nodes and writes their topology; when the tree has more nodes
@@ -196,9 +233,9 @@ hipError_t launch_tree_emit(const uint8_t* L, const uint8_t* H, uint32_t n, cons
 // Links, geometry and the upward pass: every leaf in one launch, then the
 // interior nodes of levels depth_plan - 1..0 (one launch per level, each
 // grid-striding over the level's range read on the device; n_sys systems
-// bound a level's node count by n_sys * 8^d).
+// bound a level's node count by n_sys * 8^d). The first also zeroes `zero`.
 hipError_t launch_tree_finish(const uint64_t* keys, const double4* posm, uint32_t n, const uint16_t* sid, uint32_t n_sys,
-                              const double* lohi, uint32_t depth_plan, TreeDev t, hipStream_t s);
+                              const double* lohi, uint32_t depth_plan, const ZeroRanges& zero, TreeDev t, hipStream_t s);
 // Marks the walk targets (node + 1 at the first particle in tmark; their
 // number is added to misc[kMiscTargets]) and lists the walk units (their
 // number to misc[kMiscGroups]). Targets: topmost nodes with leaf || count <=

@@ -71,18 +71,9 @@ __device__ inline uint32_t quantize(double v, double lo, double scale) {
   return static_cast<uint32_t>(t);
 }
 
-__global__ __launch_bounds__(kBlock) void k_fill_u32(uint32_t* p, uint32_t v, uint64_t n) {
-  for (uint64_t i = blockIdx.x * uint64_t(kBlock) + threadIdx.x; i < n; i += uint64_t(gridDim.x) * kBlock) p[i] = v;
-}
-
-// Zeroes several ranges in one launch (a step's flag words, totals, digit
-// histograms and look-back words).
+// Zeroes several ranges in one launch.
 __global__ __launch_bounds__(kBlock) void k_zero_ranges(ZeroRanges r) {
-  const uint64_t stride = uint64_t(gridDim.x) * kBlock;
-  const uint64_t t = blockIdx.x * uint64_t(kBlock) + threadIdx.x;
-#pragma unroll
-  for (int k = 0; k < ZeroRanges::kMax; ++k)
-    for (uint64_t i = t; i < r.n[k]; i += stride) r.p[k][i] = 0u;
+  zero_ranges(r, blockIdx.x * uint64_t(kBlock) + threadIdx.x, gridDim.x * uint64_t(kBlock));
 }
 
 __device__ inline double wave_min(double v) {
@@ -92,12 +83,6 @@ __device__ inline double wave_min(double v) {
 __device__ inline double wave_max(double v) {
   for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o));
   return v;
-}
-
-// System id of every particle, one block per chunk.
-__global__ __launch_bounds__(kBlock) void k_fill_sid(const uint4* __restrict__ chunks, uint16_t* __restrict__ sid) {
-  const uint4 c = chunks[blockIdx.x];
-  for (uint32_t i = c.y + threadIdx.x; i < c.z; i += kBlock) sid[i] = static_cast<uint16_t>(c.x);
 }
 
 // Where the build reads a particle's position: its record, or the compact
@@ -127,18 +112,34 @@ __device__ inline void pos_of(const CompactSrc& s, uint32_t i, double* x, double
   *finite = isfinite(*x) && isfinite(*y) && isfinite(*z);
 }
 
-// Min/max of the positions of one chunk (flat_build_ttg.h:93-113; min/max
-// is exact, so the chunking does not matter); flags any non-finite
-// position, velocity or mass (and, from a compact copy, its writer's flag).
+// A step's first kernel. Small systems wait for each of a step's launches in
+// turn (5 us each), so one takes all that needs nothing but the input: the
+// system table, read from pinned host memory, the zeroing, each particle's
+// system, and block b < n_chunks the min/max of the positions of chunk b
+// (flat_build_ttg.h:93-113; min/max is exact, so the chunking does not matter).
+// A chunk with a non-finite position, velocity or mass leaves NaN in place of
+// its lower x. (With copies and launches of their own for these, and events and
+// copies in place of the report below, a step of 1,000 particles took 252 us,
+// now 217; of 65,536 in FP64 800 and 760; of 1M 1,710 and 1,688.)
 template <typename Src>
-__global__ __launch_bounds__(kBlock) void k_bounds_partial(Src src, const uint32_t* __restrict__ carried_bad,
-                                                           const uint4* __restrict__ chunks, double* __restrict__ partial,
-                                                           uint32_t* __restrict__ nonfinite) {
+__global__ __launch_bounds__(kBlock) void k_start(Src src, StartArgs a) {
+  stamp(a.misc, kStampStart);
+  const uint64_t t = blockIdx.x * uint64_t(kBlock) + threadIdx.x, threads = gridDim.x * uint64_t(kBlock);
+  const bool mine = blockIdx.x < a.n_chunks;
+  uint4 c = make_uint4(0u, blockIdx.x * a.chunk, 0u, 0u);
+  if (a.n_sys == 1)
+    c.z = a.n - c.y < a.chunk ? a.n : c.y + a.chunk;
+  else if (mine)
+    c = a.host_chunks[blockIdx.x];
+  for (uint64_t i = t; i < a.table_quads; i += threads) a.table[i] = a.host_table[i];
+  if (a.host_hist)
+    for (uint64_t i = t; i < 2 * 256 / 4; i += threads) a.hist[i] = a.host_hist[i];
+  zero_ranges(a.zero, t, threads);
+  if (!mine) return;
+  for (uint32_t i = c.y + threadIdx.x; i < c.z; i += kBlock) a.sid[i] = static_cast<uint16_t>(c.x);
   const double inf = __builtin_huge_val();
   double lo[3] = {inf, inf, inf}, hi[3] = {-inf, -inf, -inf};
   bool bad = false;
-  if (carried_bad && blockIdx.x == 0 && threadIdx.x == 0 && *carried_bad) atomicOr(nonfinite, 1u);
-  const uint4 c = chunks[blockIdx.x];
   // kB elements per lane and round, all loads issued before the first use
   // (indices clamped into the chunk, extra elements dropped after the load)
   constexpr int kB = 4;
@@ -165,30 +166,34 @@ __global__ __launch_bounds__(kBlock) void k_bounds_partial(Src src, const uint32
   __shared__ double s[4][6];
   const int w = threadIdx.x >> 6, lane = __lane_id();
   double r[6];
-  for (int a = 0; a < 3; ++a) {
-    r[a] = wave_min(lo[a]);
-    r[3 + a] = wave_max(hi[a]);
+  for (int k = 0; k < 3; ++k) {
+    r[k] = wave_min(lo[k]);
+    r[3 + k] = wave_max(hi[k]);
   }
   if (lane == 0)
-    for (int a = 0; a < 6; ++a) s[w][a] = r[a];
-  if (__ballot(bad) != 0 && lane == 0) atomicOr(nonfinite, 1u);
-  __syncthreads();
+    for (int k = 0; k < 6; ++k) s[w][k] = r[k];
+  bad = __syncthreads_or(bad);
   if (threadIdx.x < 6) {
-    const int a = threadIdx.x;
-    double v = s[0][a];
-    for (int k = 1; k < 4; ++k) v = a < 3 ? fmin(v, s[k][a]) : fmax(v, s[k][a]);
-    partial[blockIdx.x * 6 + a] = v;
+    const int k = threadIdx.x;
+    double v = s[0][k];
+    for (int j = 1; j < 4; ++j) v = k < 3 ? fmin(v, s[j][k]) : fmax(v, s[j][k]);
+    a.partial[blockIdx.x * 6 + k] = bad && k == 0 ? __builtin_nan("") : v;
   }
 }
 
-// Per system: reduce its chunks' partials to lohi[6 s .. 6 s + 6).
+// Per system: reduce its chunks' partials to lohi[6 s .. 6 s + 6), and flag a
+// chunk with a non-finite value (and, from a compact copy, its writer's flag).
 __global__ __launch_bounds__(kBlock) void k_bounds_final(const double* __restrict__ partial,
-                                                         const uint32_t* __restrict__ chunk_first, double* __restrict__ lohi) {
+                                                         const uint32_t* __restrict__ chunk_first,
+                                                         const uint32_t* __restrict__ carried_bad, double* __restrict__ lohi,
+                                                         uint32_t* __restrict__ nonfinite) {
   const double inf = __builtin_huge_val();
   __shared__ double s[4][6];
   double r[6] = {inf, inf, inf, -inf, -inf, -inf};
   const uint32_t b0 = chunk_first[blockIdx.x], b1 = chunk_first[blockIdx.x + 1];
+  bool bad = carried_bad && *carried_bad;
   for (uint32_t b = b0 + threadIdx.x; b < b1; b += kBlock) {
+    bad |= partial[b * 6] != partial[b * 6];
     for (int a = 0; a < 3; ++a) {
       r[a] = fmin(r[a], partial[b * 6 + a]);
       r[3 + a] = fmax(r[3 + a], partial[b * 6 + 3 + a]);
@@ -201,7 +206,8 @@ __global__ __launch_bounds__(kBlock) void k_bounds_final(const double* __restric
   }
   if (lane == 0)
     for (int a = 0; a < 6; ++a) s[w][a] = r[a];
-  __syncthreads();
+  bad = __syncthreads_or(bad);
+  if (bad && threadIdx.x == 0) atomicOr(nonfinite, 1u);
   if (threadIdx.x < 6) {
     const int a = threadIdx.x;
     double v = s[0][a];
@@ -598,6 +604,16 @@ __global__ __launch_bounds__(kBlock) void k_gather_pos(const double* __restrict_
   reinterpret_cast<double2*>(posm + k)[half] = make_double2(pos[b0], pos[b0 + n]);
 }
 
+// The report, written to pinned host memory by the step itself (no copies
+// back, and the phases' times come with it: no events between them).
+__global__ __launch_bounds__(128) void k_report(uint32_t* __restrict__ misc, uint32_t* __restrict__ host) {
+  static_assert(kReportWords <= 128, "one thread per word");
+  stamp(misc, kStampEnd);
+  __syncthreads();
+  if (threadIdx.x < kReportWords)
+    __hip_atomic_store(&host[threadIdx.x], misc[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 inline uint32_t grid_for(uint64_t n, uint32_t cap) {
   uint64_t g = (n + kBlock - 1) / kBlock;
   if (g < 1) g = 1;
@@ -605,12 +621,6 @@ inline uint32_t grid_for(uint64_t n, uint32_t cap) {
 }
 
 }  // namespace
-
-hipError_t launch_fill_u32(uint32_t* p, uint32_t value, uint64_t n, hipStream_t s) {
-  if (n == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_fill_u32, dim3(grid_for(n, 4096)), dim3(kBlock), 0, s, p, value, n);
-  return hipGetLastError();
-}
 
 hipError_t launch_zero(const ZeroRanges& r, hipStream_t s) {
   uint64_t most = 0;
@@ -620,26 +630,31 @@ hipError_t launch_zero(const ZeroRanges& r, hipStream_t s) {
   return hipGetLastError();
 }
 
-hipError_t launch_fill_sid(const uint4* chunks, uint32_t n_chunks, uint16_t* sid, hipStream_t s) {
-  if (n_chunks == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_fill_sid, dim3(n_chunks), dim3(kBlock), 0, s, chunks, sid);
+namespace {
+template <typename Src>
+hipError_t start(Src src, const uint32_t* carried_bad, const StartArgs& a, hipStream_t s) {
+  // blocks beyond the chunks only zero: 16 KB a block
+  uint64_t words = 0;
+  for (int k = 0; k < ZeroRanges::kMax; ++k) words += a.zero.n[k];
+  const uint64_t zeroing = words / 4096 + 1 < 2048 ? words / 4096 + 1 : 2048;
+  const uint32_t blocks = a.n_chunks > zeroing ? a.n_chunks : static_cast<uint32_t>(zeroing);
+  hipLaunchKernelGGL(k_start<Src>, dim3(blocks), dim3(kBlock), 0, s, src, a);
+  hipLaunchKernelGGL(k_bounds_final, dim3(a.n_sys), dim3(kBlock), 0, s, a.partial, a.chunk_first, carried_bad, a.lohi,
+                     a.misc + kMiscNonfinite);
   return hipGetLastError();
 }
+}  // namespace
 
-hipError_t launch_bounds(const bh_particle* p, const uint4* chunks, uint32_t n_chunks, const uint32_t* chunk_first,
-                         uint32_t n_sys, double* partial, uint32_t* nonfinite, double* lohi, hipStream_t s) {
-  hipLaunchKernelGGL(k_bounds_partial<RecordSrc>, dim3(n_chunks), dim3(kBlock), 0, s, RecordSrc{p}, nullptr, chunks,
-                     partial, nonfinite);
-  hipLaunchKernelGGL(k_bounds_final, dim3(n_sys), dim3(kBlock), 0, s, partial, chunk_first, lohi);
-  return hipGetLastError();
+hipError_t launch_start(const bh_particle* p, const StartArgs& a, hipStream_t s) {
+  return start(RecordSrc{p}, nullptr, a, s);
 }
 
-hipError_t launch_bounds(const double* pos, uint32_t n, const uint32_t* carried_bad, const uint4* chunks,
-                         uint32_t n_chunks, const uint32_t* chunk_first, uint32_t n_sys, double* partial,
-                         uint32_t* nonfinite, double* lohi, hipStream_t s) {
-  hipLaunchKernelGGL(k_bounds_partial<CompactSrc>, dim3(n_chunks), dim3(kBlock), 0, s, CompactSrc{pos, n}, carried_bad,
-                     chunks, partial, nonfinite);
-  hipLaunchKernelGGL(k_bounds_final, dim3(n_sys), dim3(kBlock), 0, s, partial, chunk_first, lohi);
+hipError_t launch_start(const double* pos, const uint32_t* carried_bad, const StartArgs& a, hipStream_t s) {
+  return start(CompactSrc{pos, a.n}, carried_bad, a, s);
+}
+
+hipError_t launch_report(uint32_t* misc, uint32_t* host, hipStream_t s) {
+  hipLaunchKernelGGL(k_report, dim3(1), dim3(128), 0, s, misc, host);
   return hipGetLastError();
 }
 

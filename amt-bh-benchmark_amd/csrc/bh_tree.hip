@@ -100,7 +100,8 @@ __global__ __launch_bounds__(kTileThreads) void k_tree_count(const uint64_t* __r
                                                              const uint16_t* __restrict__ sid,
                                                              const SysDev* __restrict__ sys, uint32_t mlx,
                                                              uint8_t* __restrict__ L, uint8_t* __restrict__ H,
-                                                             uint32_t* __restrict__ tile_counts) {
+                                                             uint32_t* __restrict__ tile_counts, uint32_t* misc) {
+  stamp(misc, kStampTree);
   // dynamic LDS sized by the batch's largest max_leaf (mlx): keys of
   // [base - mlx - 1, base + tile + mlx), then P of [base - mlx, base + tile)
   extern __shared__ __align__(8) unsigned char s_dyn[];
@@ -387,7 +388,9 @@ __global__ __launch_bounds__(kTileThreads) void k_tree_emit(const uint8_t* __res
 // Children, parents, leaf counts and cell geometry of every node.
 __global__ __launch_bounds__(kBlock) void k_tree_links(const uint64_t* __restrict__ keys, uint32_t n,
                                                        const uint16_t* __restrict__ sid, const double* __restrict__ lohi,
-                                                       TreeDev t) {
+                                                       ZeroRanges zero, TreeDev t) {
+  // also when the step is given up: the unit list's look-back relies on it
+  zero_ranges(zero, blockIdx.x * uint64_t(kBlock) + threadIdx.x, gridDim.x * uint64_t(kBlock));
   if (t.misc[kMiscAbort]) return;
   const uint32_t n_nodes = t.level_off[kLevels], n_leaves = t.misc[kMiscLevels + kLevels];
   for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n_nodes; i += gridDim.x * kBlock) {
@@ -696,6 +699,7 @@ __global__ __launch_bounds__(kBlock) void k_units_mark(TreeDev t, const uint16_t
                                                        uint32_t* __restrict__ tmark, uint32_t* __restrict__ gmark,
                                                        uint32_t* __restrict__ unit_n) {
   __shared__ uint32_t s_targets;
+  stamp(t.misc, kStampTargets);
   if (t.misc[kMiscAbort]) return;
   if (threadIdx.x == 0) s_targets = 0;
   __syncthreads();
@@ -778,10 +782,11 @@ __global__ __launch_bounds__(kBlock) void k_units_mark(TreeDev t, const uint16_t
 // tile's place comes from decoupled look-back over the tiles before it (64 at
 // a time), tiles taken in the order of a counter.
 __global__ __launch_bounds__(kBlock) void k_units_list(const uint32_t* __restrict__ mark, uint32_t n, uint32_t tiles,
-                                                       uint32_t* __restrict__ lookback, uint32_t* __restrict__ n_units,
+                                                       uint32_t* __restrict__ lookback, uint32_t* __restrict__ misc,
                                                        uint2* __restrict__ out) {
   __shared__ uint32_t s_wc[4];
   __shared__ uint32_t s_tile, s_excl;
+  if (misc[kMiscAbort]) return;
   if (threadIdx.x == 0) s_tile = atomicAdd(&lookback[tiles], 1u);
   __syncthreads();
   const uint32_t tile = s_tile, base = tile * kTreeTile;
@@ -823,7 +828,7 @@ __global__ __launch_bounds__(kBlock) void k_units_list(const uint32_t* __restric
     if (lane == 0) {
       __hip_atomic_store(&lookback[tile], kLbPre | (excl + total), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       s_excl = excl;
-      if (tile + 1 == tiles) *n_units = excl + total;
+      if (tile + 1 == tiles) misc[kMiscGroups] = excl + total;
     }
   }
   __syncthreads();
@@ -847,10 +852,12 @@ inline uint32_t grid_for(uint64_t n, uint32_t cap) {
 }  // namespace
 
 hipError_t launch_tree_count(const uint64_t* keys, uint32_t n, const uint16_t* sid, const SysDev* sys,
-                             uint32_t max_leaf_max, uint8_t* L, uint8_t* H, uint32_t* tile_counts, hipStream_t s) {
+                             uint32_t max_leaf_max, uint8_t* L, uint8_t* H, uint32_t* tile_counts, uint32_t* misc,
+                             hipStream_t s) {
   const uint32_t tiles = (n + kTreeTile - 1) / kTreeTile;
   const size_t lds = (kTreeTile + 2 * size_t(max_leaf_max) + 1) * sizeof(uint64_t) + kTreeTile + max_leaf_max;
-  hipLaunchKernelGGL(k_tree_count, dim3(tiles), dim3(kTileThreads), lds, s, keys, n, sid, sys, max_leaf_max, L, H, tile_counts);
+  hipLaunchKernelGGL(k_tree_count, dim3(tiles), dim3(kTileThreads), lds, s, keys, n, sid, sys, max_leaf_max, L, H,
+                     tile_counts, misc);
   return hipGetLastError();
 }
 
@@ -869,9 +876,9 @@ hipError_t launch_tree_emit(const uint8_t* L, const uint8_t* H, uint32_t n, cons
 }
 
 hipError_t launch_tree_finish(const uint64_t* keys, const double4* posm, uint32_t n, const uint16_t* sid, uint32_t n_sys,
-                              const double* lohi, uint32_t depth_plan, TreeDev t, hipStream_t s) {
+                              const double* lohi, uint32_t depth_plan, const ZeroRanges& zero, TreeDev t, hipStream_t s) {
   // grid-stride loops over the node count read on the device
-  hipLaunchKernelGGL(k_tree_links, dim3(grid_for(t.cap, 4096)), dim3(kBlock), 0, s, keys, n, sid, lohi, t);
+  hipLaunchKernelGGL(k_tree_links, dim3(grid_for(t.cap, 4096)), dim3(kBlock), 0, s, keys, n, sid, lohi, zero, t);
   // every leaf, then the interior nodes bottom-up: one launch per level
   // below the planned depth (the deepest level holds leaves only), each
   // reading its level's range on the device and grid-striding over it.
@@ -896,7 +903,7 @@ hipError_t launch_units(TreeDev t, uint32_t n, const uint16_t* sid, const SysDev
   const uint32_t tiles = (n + kTreeTile - 1) / kTreeTile;
   hipLaunchKernelGGL(k_units_mark, dim3(grid_for(t.cap, 4096)), dim3(kBlock), 0, s, t, sid, sys, grouped, tmark, gmark,
                      unit_n);
-  hipLaunchKernelGGL(k_units_list, dim3(tiles), dim3(kBlock), 0, s, gmark, n, tiles, lookback, t.misc + kMiscGroups,
+  hipLaunchKernelGGL(k_units_list, dim3(tiles), dim3(kBlock), 0, s, gmark, n, tiles, lookback, t.misc,
                      units);
   return hipGetLastError();
 }

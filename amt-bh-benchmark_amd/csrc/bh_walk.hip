@@ -1090,6 +1090,7 @@ template <typename Real, int kWaves, bool kMask, bool kDeep>
 __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(4))) void k_walk(WalkArgs a) {
   __shared__ WaveLds<Real, kShallowFrames, kDeep> lds[kWaves];
   static_assert(kWaves == 1, "one wavefront per workgroup: the queues hand out units per workgroup");
+  stamp(a.misc, kStampWalk);
   if (a.misc[kMiscNonfinite] | a.misc[kMiscAbort]) return;
   const uint32_t units = a.misc[kMiscGroups];
   const uint32_t x = blockIdx.x & 7u;

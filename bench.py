@@ -16,7 +16,7 @@ warm-up step; the K timed steps are full kick+drift steps.
 
 Prints one JSON line. `roofline` is for the walk kernel (the dominant one):
 algorithmic FP32 flops per launch (19 per particle interaction, 55 per
-quadrupole-cell interaction) over its average duration from HIP events on
+quadrupole-cell interaction) over its average duration by the GPU's clock on
 the library's stream. `cpu_baseline` times the FP64 oracle (a C++
 restatement of the reference's grouped path) on the host's usable cores over
 a bounded sample of the same workload.

@@ -291,8 +291,8 @@ int bh_tree_export(bh_ctx* ctx, int layout, uint64_t* keys, uint32_t* perm, bh_p
 int bh_accel(bh_ctx* ctx, const bh_force_params* fp, uint32_t target_size, double* acc, uint32_t* n_pp, uint32_t* n_pc,
              uint64_t* totals);
 
-/* Per-phase device times of the last step or bh_accel call, from HIP events
- * recorded on the context's stream (the reference's StepTiming split,
+/* Per-phase device times of the last step or bh_accel call, from the GPU's
+ * constant-rate clock as each phase begins (the reference's StepTiming split,
  * integrate_ttg.h:24-28, refined), and the work the walk did. Has no
  * reference counterpart beyond StepTiming; it exists for measurement. */
 typedef struct bh_step_stats {
