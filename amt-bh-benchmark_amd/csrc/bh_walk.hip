@@ -135,21 +135,13 @@ __device__ inline uint32_t wave_incl_add(uint32_t v) {
   x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);  // row_bcast:31
   return static_cast<uint32_t>(x);
 }
-// Inclusive max-scan of non-negative values.
-__device__ inline uint32_t wave_incl_max(uint32_t v) {
-  int x = static_cast<int>(v);
-  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, false));
-  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, false));
-  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, false));
-  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, false));
-  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false));
-  x = max(x, __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false));
-  return static_cast<uint32_t>(x);
-}
-
-__device__ inline uint64_t lanemask_lt() {
-  const int lane = __lane_id();
-  return lane == 0 ? 0ull : (~0ull >> (64 - lane));
+// The lanes where p holds: a comparison's mask as it is (__ballot makes it a
+// value per lane first and compares again).
+__device__ inline uint64_t ballot(bool p) { return __builtin_amdgcn_ballot_w64(p); }
+// Set bits of mask below this lane.
+__device__ inline uint32_t rank_of(uint64_t mask) {
+  return __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(mask >> 32),
+                                   __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(mask), 0u));
 }
 
 __device__ inline uint32_t uniform(uint32_t v) { return __builtin_amdgcn_readfirstlane(v); }
@@ -473,7 +465,6 @@ __device__ bool traverse(const WalkArgs& a, Lds& L, uint32_t* gfr, const Box6& b
   constexpr int F = Lds::kFrames;
   constexpr int kStack = Lds::kDeepFrames ? kLevels : F;
   const int lane = __lane_id();
-  const uint64_t lt = lanemask_lt();
   const uint32_t last_node = a.n_nodes - 1, last_part = a.n_parts - 1;
   const double blo0 = uniform_d(box.v[0]), blo1 = uniform_d(box.v[1]), blo2 = uniform_d(box.v[2]);
   const double bhi0 = uniform_d(box.v[3]), bhi1 = uniform_d(box.v[4]), bhi2 = uniform_d(box.v[5]);
@@ -533,10 +524,10 @@ __device__ bool traverse(const WalkArgs& a, Lds& L, uint32_t* gfr, const Box6& b
       continue;
     }
     // Pop whole child ranges, up to 64 nodes. Range j covers slots
-    // [excl_j, excl_j + count_j); its index j, placed at its first slot,
-    // is non-decreasing over the slots, so a prefix max gives every slot its
-    // range: node = first_j + (slot - excl_j). (The ranges themselves need
-    // not be ascending: children of deferred nodes come in walk order.)
+    // [excl_j, excl_j + count_j) and flags its first slot, so a slot's range
+    // is the number of flags up to it less one: node = first_j + (slot -
+    // excl_j). (The ranges themselves need not be ascending: children of
+    // deferred nodes come in walk order.)
     const uint32_t rr = cur + lane;
     const bool rv = rr < nr;
     uint32_t node, total;
@@ -556,14 +547,13 @@ __device__ bool traverse(const WalkArgs& a, Lds& L, uint32_t* gfr, const Box6& b
       const uint32_t rfirst = packed >> 3;
       const uint32_t incl = wave_incl_add(rcnt);
       const bool taken = rv && incl <= kWave;
-      const int k = __popcll(__ballot(taken));
+      const int k = __popcll(ballot(taken));
       total = uniform(__builtin_amdgcn_readlane(incl, k - 1));
       const uint32_t excl = incl - rcnt;
-      // each taken range sends its index to its first slot; the other lanes
-      // send range 0's, 0, to slot 0
-      const int own = __builtin_amdgcn_ds_permute(taken ? static_cast<int>(excl << 2) : 0, taken ? lane : 0);
+      // the other lanes flag slot 0, where range 0 starts
+      const int own = __builtin_amdgcn_ds_permute(taken ? static_cast<int>(excl << 2) : 0, 1);
       if (lane == depth) fr_cur = cur + k;
-      const int j = static_cast<int>(wave_incl_max(static_cast<uint32_t>(own)));
+      const int j = static_cast<int>(rank_of(ballot(own != 0))) + own - 1;
       node = static_cast<uint32_t>(__shfl(static_cast<int>(rfirst - excl), j)) + static_cast<uint32_t>(lane);
     }
     const bool nv = static_cast<uint32_t>(lane) < total;
@@ -611,25 +601,25 @@ __device__ bool traverse(const WalkArgs& a, Lds& L, uint32_t* gfr, const Box6& b
     // integrate_ttg.h:104-106).
     const bool openable = !isleaf && lcnt != 0u && depth + 1 < kStack && static_cast<uint32_t>(depth) + 1 < a.stack_limit;
     const bool openf = nv && !accept && !defer && !isleaf && openable;
-    if (__ballot(nv && !accept && !defer && !isleaf && !openable)) {
+    if (ballot(nv && !accept && !defer && !isleaf && !openable)) {
       if (lane == 0) atomicOr(&a.misc[kMiscIncomplete], 1u);
     }
     if constexpr (kGroup) {
-      const uint64_t dm = __ballot(deff);
+      const uint64_t dm = ballot(deff);
       if (dm) {
         const uint32_t nd_new = __popcll(dm);
         if (n_def + nd_new > kDefer) {
           ok = false;
           break;
         }
-        if (deff) dl[n_def + __popcll(dm & lt)] = nd << 3;
+        if (deff) dl[n_def + rank_of(dm)] = nd << 3;
         n_def += nd_new;
       }
     }
     // children of opened interior nodes -> frame depth + 1
-    const uint64_t om = __ballot(openf);
+    const uint64_t om = ballot(openf);
     if (om) {
-      const uint32_t pos = __popcll(om & lt);
+      const uint32_t pos = rank_of(om);
       if constexpr (Lds::kDeepFrames) {
         if (depth + 1 < F) {
           if (openf) L.fr[depth + 1][pos] = (lfirst << 3) | (lcnt - 1u);
@@ -646,10 +636,10 @@ __device__ bool traverse(const WalkArgs& a, Lds& L, uint32_t* gfr, const Box6& b
       }
     }
     // accepted nodes
-    const uint64_t cm = __ballot(cellf);
+    const uint64_t cm = ballot(cellf);
     if (cm) {
       const uint32_t nc = __popcll(cm);
-      const uint32_t pos = __popcll(cm & lt);
+      const uint32_t pos = rank_of(cm);
       if (use_quad) {
         if (cellf) {
           const uint32_t slot = pc_cnt + pos;
@@ -678,25 +668,27 @@ __device__ bool traverse(const WalkArgs& a, Lds& L, uint32_t* gfr, const Box6& b
         if (pp_cnt >= kBatch) flush_pp(Eval::take(pp_cnt));
       }
     }
-    // particles of opened leaves, mapped to slots like the nodes: the lane
-    // of the leaf covering each slot by a prefix max of lane indices
-    const uint64_t lm = __ballot(leaff);
+    // particles of opened leaves, mapped to slots like the nodes: the leaves'
+    // offsets move to the first lanes, where a slot's count of flags finds them
+    const uint64_t lm = ballot(leaff);
     if (lm) {
       const uint32_t lc = leaff ? lcnt : 0u;
       const uint32_t lincl = wave_incl_add(lc);
       const uint32_t lexcl = lincl - lc;
       const uint32_t ltot = uniform(__builtin_amdgcn_readlane(lincl, 63));
+      // (lanes without a leaf write the last lane, which then holds none)
+      const int from = __builtin_amdgcn_ds_permute(static_cast<int>((leaff ? rank_of(lm) : 63u) << 2),
+                                                   static_cast<int>(lfirst - lexcl));
       for (uint32_t b = 0; b < ltot; b += kWave) {
-        // the leaf holding slot b: the last leaf lane starting at or before it
-        const uint64_t before = __ballot(leaff && lexcl <= b);
-        const int j0 = 63 - __clzll(static_cast<long long>(before));
+        // leaves that start at or before slot b
+        const int before = __popcll(ballot(leaff && lexcl <= b));
         const uint32_t e = b + lane;
-        // each leaf that starts in this chunk sends its lane to its first
-        // slot; the other lanes send j0 to slot 0
+        // each leaf that starts later in this chunk flags its first slot; the
+        // other lanes clear slot 0
         const bool here = leaff && lexcl > b && lexcl < b + kWave;
-        const int own = __builtin_amdgcn_ds_permute(here ? static_cast<int>((lexcl - b) << 2) : 0, here ? lane : j0);
-        const int jj = static_cast<int>(wave_incl_max(static_cast<uint32_t>(own)));
-        uint32_t q = static_cast<uint32_t>(__shfl(static_cast<int>(lfirst - lexcl), jj)) + e;
+        const int own = __builtin_amdgcn_ds_permute(here ? static_cast<int>((lexcl - b) << 2) : 0, here ? 1 : 0);
+        const int jj = before - 1 + static_cast<int>(rank_of(ballot(own != 0))) + own;
+        uint32_t q = static_cast<uint32_t>(__shfl(from, jj)) + e;
         q = q < last_part ? q : last_part;
         const uint32_t chunk = ltot - b < kWave ? ltot - b : kWave;
         if (e < ltot) {
@@ -879,7 +871,7 @@ __device__ inline uint32_t covering_target(const WalkArgs& a, uint32_t gb, uint3
   for (uint32_t back = 0;; back += kWave) {
     const uint32_t d = back + __lane_id();
     const uint32_t m = d <= p - gb ? a.tmark[p - d] : 0u;
-    const uint64_t have = __ballot(m != 0);
+    const uint64_t have = ballot(m != 0);
     if (have) return uniform(__builtin_amdgcn_readlane(m, __ffsll(static_cast<long long>(have)) - 1)) - 1u;
     if (back + kWave > p - gb) return 0u;  // not reached: a unit's first particle begins a target
   }
@@ -968,7 +960,7 @@ __device__ void walk_group(const WalkArgs& a, Lds& L, uint32_t slot, uint32_t g,
         while (!bits && c < r1) {
           const uint32_t i = c + lane;
           m = i < r1 ? a.tmark[i] : 0u;
-          bits = __ballot(m != 0);
+          bits = ballot(m != 0);
           c += kWave;
         }
         if (!bits) break;  // not reached: targets fill the unit
