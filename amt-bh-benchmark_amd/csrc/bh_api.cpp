@@ -88,6 +88,10 @@ struct Scratch {
   double* gacc = nullptr;
 };
 
+// The walk's queue heads lie over the sort's look-back words (at least 2,560),
+// which are free by then.
+uint32_t* walk_queue(const Scratch& b) { return b.lookback; }
+
 // What the host decides before a step is enqueued.
 struct Plan {
   uint32_t n = 0;         // particles of all systems
@@ -725,15 +729,18 @@ int enqueue_build(Ctx* c, const Plan& p, const Scratch& b, const bh_particle* d_
   HIP_OK(c, launch_tree_scan(b.tcounts, tiles, b.tprefix, b.misc + kMiscLevels, s));
   HIP_OK(c, launch_tree_emit(b.L, b.H, n, b.tprefix, b.t, p.depth_plan, s));
   // what the walk needs zeroed and could not be before: unit_lb may lie over
-  // tcounts, and the carried flag has been read
+  // tcounts, the queue heads over the look-back words, and the carried flag
+  // has been read
   ZeroRanges z;
   if (p.walk) {
     z.p[0] = b.unit_lb;
     z.n[0] = unit_list_words(n);
+    z.p[1] = walk_queue(b);
+    z.n[1] = kQueueWords;
   }
   if (p.walk && p.carry_out) {
-    z.p[1] = c->carry_flag.p;
-    z.n[1] = 1;
+    z.p[2] = c->carry_flag.p;
+    z.n[2] = 1;
   }
   HIP_OK(c, launch_tree_finish(out->keys, b.posm, n, b.sid, p.S, b.lohi, p.depth_plan, z, b.t, s));
   return BH_OK;
@@ -767,6 +774,7 @@ int enqueue_walk(Ctx* c, const Plan& p, const Scratch& b, bh_particle* parts, do
   a.defer = b.defer;
   a.deep_frames = p.deep ? b.deep_frames : nullptr;
   a.misc = b.misc;
+  a.queue = walk_queue(b);
   a.n_nodes = p.cap_nodes;
   a.n_parts = n;
   a.stack_limit = c->stack_limit;
@@ -1670,13 +1678,15 @@ int bh_accel(bh_ctx* h, const bh_force_params* fp, uint32_t target_size, double*
   z.p[0] = b.misc + kMiscIncomplete;
   z.n[0] = 1;
   z.p[1] = b.misc + kMiscTargets;
-  z.n[1] = kMiscStamps - kMiscTargets;  // target and unit counts, queue heads, totals
+  z.n[1] = kMiscStamps - kMiscTargets;  // target and unit counts, totals
   z.p[2] = b.mark;
   z.n[2] = n;
   z.p[3] = b.gmark;
   z.n[3] = n;
   z.p[4] = b.unit_lb;
   z.n[4] = unit_list_words(n);
+  z.p[5] = walk_queue(b);
+  z.n[5] = kQueueWords;
   HIP_OK(c, launch_zero(z, c->stream));
   TRY(enqueue_walk(c, p, b, nullptr, c->dacc.p, c->dcnt.p, c->dcnt.p + n));
   TRY(enqueue_report(c, b));

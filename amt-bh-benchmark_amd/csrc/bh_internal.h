@@ -48,6 +48,8 @@ constexpr uint32_t kGroupCap = 128;  // largest walk tile: a walk unit's particl
 constexpr uint32_t kMinTile = 16;    // smallest walk tile
 constexpr uint32_t kDefer = 512;     // deferred nodes a group may hand its targets
 constexpr uint32_t kShallowFrames = 12;  // walk stack of trees with at most this many levels
+constexpr uint32_t kQueueStride = 32;    // words from one walk-unit queue head to the next: a cache line
+constexpr uint32_t kQueueWords = 8 * kQueueStride;
 constexpr uint32_t kWalkSlots = 4096;    // walk workgroups at most: 256 CUs x 4 SIMDs x 4 waves
 
 // The step's flag and count words (`misc`), cleared when a step starts and
@@ -62,7 +64,6 @@ constexpr int kMiscMaxDepth = 3;    // deepest level of the tree
 constexpr int kMiscLevels = 8;      // [8, 8 + kLevels): nodes per level; [8 + kLevels]: leaves
 constexpr int kMiscTargets = 40;    // walk targets
 constexpr int kMiscGroups = 41;     // walk units
-constexpr int kMiscQueue = 48;      // [48, 56): walk-unit queue heads, one per XCD
 constexpr int kMiscWords = 64;
 // Behind them the two 64-bit interaction totals and the times (of the GPU's
 // constant-rate clock) at which the step's phases began: start, tree, targets,
@@ -131,7 +132,8 @@ struct WalkArgs {
   double* gacc;            // [3n] scratch: a group's shared-list sums per particle
   uint32_t* defer;         // [slots * kDefer] scratch: deferred nodes, per walk workgroup
   uint32_t* deep_frames;   // [slots * (kLevels - kShallowFrames) * 64] stack frames below the LDS ones
-  uint32_t* misc;          // the step's flags; unit count and queue heads
+  uint32_t* misc;          // the step's flags and the unit count
+  uint32_t* queue;         // [kQueueWords] walk-unit queue heads, one per XCD and cache line, zero at the start
   uint32_t n_nodes;        // index clamps (the node capacity): a node or particle
   uint32_t n_parts;        // index never leaves its array, whatever the tree holds
   uint32_t stack_limit;    // frames the walk may use (kLevels; lower only to test the incomplete-walk report)

@@ -1066,9 +1066,15 @@ __device__ void walk_group(const WalkArgs& a, Lds& L, uint32_t slot, uint32_t g,
 // b % 8, which holds the eighth [x U / 8, (x + 1) U / 8) of the U units
 // (Morton order): each XCD walks a contiguous run, so neighbouring units
 // share its L2, and within an XCD the units go to whichever wavefront is
-// free. A wavefront leaves once its queue is past its end, so every
-// wavefront exits. The unit count and the queue heads are on the device
-// (counted and cleared by the step), so the launch needs no host read.
+// free. A wavefront whose queue is past its end goes on with the queue that
+// has most units left, and leaves once none has any; a head only grows, so
+// every wavefront exits. Equal shares of the units are not equal shares of the
+// work: of 64 systems of different sizes the XCDs needed 16 to 39 ms, now all
+// 26.4; 16M 38.7 -> 38.2, 4M 10.2 -> 10.0. The heads lie a cache line apart and
+// are looked at before a claim: next to each other, and claimed to find out
+// that a queue is empty, they took 0.3 ms more at 1M. The unit count and the
+// heads are on the device (counted and cleared by the step), so the launch
+// needs no host read.
 //
 // Device-scope atomics on one address from many wavefronts queue up behind
 // each other (measured inside this kernel at 65,536 particles: a claim 27,000
@@ -1085,23 +1091,47 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(4))
   stamp(a.misc, kStampWalk);
   if (a.misc[kMiscNonfinite] | a.misc[kMiscAbort]) return;
   const uint32_t units = a.misc[kMiscGroups];
-  const uint32_t x = blockIdx.x & 7u;
-  const uint32_t lo = static_cast<uint32_t>(uint64_t(units) * x / 8);
-  const uint32_t hi = static_cast<uint32_t>(uint64_t(units) * (x + 1) / 8);
   auto& L = lds[0];
   if (__lane_id() == 0) L.tot[0] = L.tot[1] = 0ull;
   __builtin_amdgcn_wave_barrier();
   const uint32_t first = gridDim.x >> 3;
-  for (uint32_t k = blockIdx.x >> 3; k < hi - lo;) {
+  // queue q's units: [lo, lo + len)
+  uint32_t q = blockIdx.x & 7u, lo, len;
+  const auto part = [&](uint32_t p) { return static_cast<uint32_t>(uint64_t(units) * p / 8); };
+  lo = part(q);
+  len = part(q + 1) - lo;
+  // Every lane takes part in the claim (adding 1 for lane 0, 0 for the
+  // others) and the unit is read from lane 0's result: no branch on the
+  // lane id inside the loop, so all 64 lanes stay together in it (a
+  // lane-0-only claim lets the compiler keep the other lanes looping on
+  // their own, with a stale claim).
+  const auto claim = [&]() {
+    const uint32_t mine = atomicAdd(&a.queue[kQueueStride * q], __lane_id() == 0 ? 1u : 0u);
+    return first + uniform(__builtin_amdgcn_readlane(mine, 0));
+  };
+  uint32_t k = blockIdx.x >> 3;
+  for (;;) {
+    while (k >= len) {
+      // the queue with most units left, if any is: lane p looks at queue p
+      const uint32_t p = __lane_id() & 7u, n = part(p + 1) - part(p);
+      uint32_t left = 0;
+      if (n > first) {
+        const uint32_t h = __hip_atomic_load(&a.queue[kQueueStride * p], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        left = h < n - first ? n - first - h : 0u;
+      }
+      uint32_t most = left << 3 | p;
+      for (int o = 4; o > 0; o >>= 1) most = max(most, static_cast<uint32_t>(__shfl_xor(static_cast<int>(most), o)));
+      most = uniform(most);
+      if (most < 8u) break;
+      q = most & 7u;
+      lo = part(q);
+      len = part(q + 1) - lo;
+      k = claim();
+    }
+    if (k >= len) break;
     const uint2 u = a.units[lo + k];
     walk_group<Real, kMask>(a, L, blockIdx.x, uniform(u.x), uniform(u.y));
-    // Every lane takes part in the claim (adding 1 for lane 0, 0 for the
-    // others) and the unit is read from lane 0's result: no branch on the
-    // lane id inside the loop, so all 64 lanes stay together in it (a
-    // lane-0-only claim lets the compiler keep the other lanes looping on
-    // their own, with a stale claim).
-    const uint32_t mine = atomicAdd(&a.misc[kMiscQueue + x], __lane_id() == 0 ? 1u : 0u);
-    k = first + uniform(__builtin_amdgcn_readlane(mine, 0));
+    k = claim();
   }
   if (__lane_id() == 0 && (L.tot[0] | L.tot[1]) != 0ull) {
     atomicAdd(&a.totals[0], L.tot[0]);
