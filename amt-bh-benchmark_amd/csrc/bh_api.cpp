@@ -317,7 +317,9 @@ int check_args(Ctx* c, uint64_t n, const bh_force_params* fp, uint32_t max_leaf,
 //   16,384 (32/96)   0.536 -> 0.326       200 systems 5.56 -> 5.53
 //   65,536 (16/32)   0.732 -> 0.329        64 systems 9.40 -> 9.22
 //   65,536 (32/96)   0.668 -> 0.456        64 systems 8.48 -> 8.45
+//   131,072 (32/96)  0.750 -> 0.591        32 systems 8.76 -> 8.67
 //   250,007 (32/64)  1.229 -> 0.837        16 systems 9.33 -> 9.09
+//   500,000 (16/32)  1.665 -> 1.429        16 systems 18.75 -> 17.62
 //   500,000 (32/96)  1.531 -> 1.466        16 systems 9.39 -> 9.31
 //   1M (32/96) 3.06 -> 2.87; 1M uniform (8/32) 1.43 -> 1.33
 // Above 2M whole units are the fastest (4M: 10.25 against 10.50 at 64).
@@ -329,7 +331,8 @@ Pieces walk_pieces(uint64_t n, uint32_t tsm) {
   if (n <= 4096) return narrow ? Pieces{16, 32} : Pieces{24, 32};
   if (n <= 16384) return narrow ? Pieces{16, 32} : Pieces{32, 48};
   if (n <= 65536) return narrow ? Pieces{24, 32} : Pieces{32, 48};
-  if (n <= (512u << 10) && tsm <= 64) return Pieces{32, 64};
+  if (n <= (256u << 10)) return Pieces{32, 64};
+  if (n <= (512u << 10) && !narrow && tsm <= 64) return Pieces{32, 64};
   if (n <= (2u << 20)) return Pieces{64, 64};
   return Pieces{kGroupCap, kGroupCap};
 }
