@@ -52,8 +52,15 @@ namespace bhk {
 
 namespace {
 
-constexpr int kBatch = 48;  // staged entries that make a batch (a batch takes all that are staged)
-constexpr int kBuf = 112;   // staging capacity: kBatch - 1 left over + 64 staged at once
+// Staged entries that make a batch, and staging capacity: kBatch - 1 left over
+// + 64 staged at once. FP64 entries take twice the LDS; with 48 only 10
+// wavefronts fitted a CU, with 22 the 12 that the registers allow do (walk of
+// 65,536 particles 0.575 -> 0.54 ms, 131,072 1.65 -> 1.52, 1M 5.73 -> 5.55; 16:
+// 0.62, 1.60, 5.78).
+template <typename Real>
+constexpr int kBatch = sizeof(Real) == 4 ? 48 : 22;
+template <typename Real>
+constexpr int kBuf = kBatch<Real> + 64;
 constexpr int kGroupChunks = kGroupCap / kWave;  // a group's particle slots per lane
 
 template <typename Real>
@@ -81,9 +88,9 @@ struct Vec2T<double> {
 // {Qxz, Qyz} c[i] (40 bytes in FP32).
 template <typename Real>
 struct PcRing {
-  typename Vec4T<Real>::T a[kBuf];
-  typename Vec4T<Real>::T b[kBuf];
-  typename Vec2T<Real>::T c[kBuf];
+  typename Vec4T<Real>::T a[kBuf<Real>];
+  typename Vec4T<Real>::T b[kBuf<Real>];
+  typename Vec2T<Real>::T c[kBuf<Real>];
 };
 
 // The walk's stack: frame d holds the child ranges d levels below the
@@ -96,7 +103,7 @@ struct WaveLds {
   using V4 = typename Vec4T<Real>::T;
   uint32_t fr[F][kWave];  // child ranges: (first << 3) | (count - 1)
   unsigned long long tot[2];    // interactions of the wavefront's units so far
-  V4 pp[kBuf];                  // x, y, z (relative to the target centre), m
+  V4 pp[kBuf<Real>];                  // x, y, z (relative to the target centre), m
   PcRing<Real> pc;
 };
 
@@ -263,7 +270,7 @@ __device__ inline void eval_pc(const PcRing<Real>& r, int j0, int n, const Real*
 template <typename Real, bool kMask>
 struct TargetEval {
   using V4 = typename Vec4T<Real>::T;
-  static constexpr int kFoldEntries = 2 * kBatch;
+  static constexpr int kFoldEntries = 2 * kBatch<Real>;
   // a batch takes all that is staged
   static constexpr bool kTakesAll = true;
   __device__ static inline uint32_t take(uint32_t n) { return n; }
@@ -327,7 +334,7 @@ struct GroupEval {
   using V4 = typename Vec4T<Real>::T;
   // a batch takes whole folds
   static constexpr bool kTakesAll = false;
-  __device__ static inline uint32_t take(uint32_t n) { return n / kBatch * kBatch; }
+  __device__ static inline uint32_t take(uint32_t n) { return n / kBatch<Real> * kBatch<Real>; }
   Real gx[kGroupChunks], gy[kGroupChunks], gz[kGroupChunks], eps2;
   int nc;          // slots in the fused loop (1 or 2)
   bool tail;       // slot 1 has a loop of its own
@@ -382,7 +389,7 @@ struct GroupEval {
     sh.of(n, &q, &j0, &more);
     Real bx[NC], by[NC], bz[NC];
     for (;;) {
-      const int c = q < kBatch ? q : kBatch;
+      const int c = q < kBatch<Real> ? q : kBatch<Real>;
 #pragma unroll
       for (int k = 0; k < NC; ++k) bx[k] = by[k] = bz[k] = 0;
       eval_pp<Real, kMask, NC>(ring + j0, c, gx + K0, gy + K0, gz + K0, eps2, bx, by, bz);
@@ -408,7 +415,7 @@ struct GroupEval {
     sh.of(n, &q, &j0, &more);
     Real bx[NC], by[NC], bz[NC];
     for (;;) {
-      const int c = q < kBatch ? q : kBatch;
+      const int c = q < kBatch<Real> ? q : kBatch<Real>;
 #pragma unroll
       for (int k = 0; k < NC; ++k) bx[k] = by[k] = bz[k] = 0;
       eval_pc<Real, NC>(r, j0, c, gx + K0, gy + K0, gz + K0, eps2, bx, by, bz);
@@ -657,7 +664,7 @@ __device__ bool traverse(const WalkArgs& a, Lds& L, uint32_t* gfr, const Box6& b
         }
         pc_cnt += nc;
         n_pc += nc;
-        if (pc_cnt >= kBatch) flush_pc(Eval::take(pc_cnt));
+        if (pc_cnt >= kBatch<Real>) flush_pc(Eval::take(pc_cnt));
       } else {
         if (cellf) {
           const double m = sizeof(Real) == 4 ? static_cast<double>(__uint_as_float(rw2.z)) : a.q64[8 * nd];
@@ -665,7 +672,7 @@ __device__ bool traverse(const WalkArgs& a, Lds& L, uint32_t* gfr, const Box6& b
         }
         pp_cnt += nc;
         n_pp += nc;
-        if (pp_cnt >= kBatch) flush_pp(Eval::take(pp_cnt));
+        if (pp_cnt >= kBatch<Real>) flush_pp(Eval::take(pp_cnt));
       }
     }
     // particles of opened leaves, mapped to slots like the nodes: the leaves'
@@ -697,7 +704,7 @@ __device__ bool traverse(const WalkArgs& a, Lds& L, uint32_t* gfr, const Box6& b
         }
         pp_cnt += chunk;
         n_pp += chunk;
-        if (pp_cnt >= kBatch) flush_pp(Eval::take(pp_cnt));
+        if (pp_cnt >= kBatch<Real>) flush_pp(Eval::take(pp_cnt));
       }
     }
     __builtin_amdgcn_wave_barrier();
