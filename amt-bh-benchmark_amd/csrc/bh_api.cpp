@@ -114,6 +114,9 @@ struct Plan {
   bool carried_in = false; // the input is the last resident step's output: build from its compact positions
 };
 
+// One workgroup sorts the system.
+bool small(const Plan& p) { return p.S == 1 && p.n <= kSmallSort; }
+
 // One captured step, keyed by everything its launches depend on.
 struct GraphKey {
   const void* in;
@@ -695,15 +698,17 @@ int enqueue_build(Ctx* c, const Plan& p, const Scratch& b, const bh_particle* d_
   // words, and the walk's marks
   a.zero.p[0] = b.misc;
   a.zero.n[0] = kMiscStamps;
-  a.zero.p[1] = b.hist;
-  a.zero.n[1] = 8 * 256;
-  a.zero.p[2] = b.lookback;
-  a.zero.n[2] = lb_words;
   if (p.walk) {
-    a.zero.p[3] = b.mark;
-    a.zero.n[3] = n;
-    a.zero.p[4] = b.gmark;
-    a.zero.n[4] = n;
+    a.zero.p[1] = b.mark;
+    a.zero.n[1] = n;
+    a.zero.p[2] = b.gmark;
+    a.zero.n[2] = n;
+  }
+  if (!small(p)) {
+    a.zero.p[3] = b.hist;
+    a.zero.n[3] = 8 * 256;
+    a.zero.p[4] = b.lookback;
+    a.zero.n[4] = lb_words;
   }
   a.host_chunks = reinterpret_cast<const uint4*>(c->host_tables + p.off_chunks);
   a.chunk_first = reinterpret_cast<const uint32_t*>(b.tables + p.off_first);
@@ -715,19 +720,31 @@ int enqueue_build(Ctx* c, const Plan& p, const Scratch& b, const bh_particle* d_
   a.partial = b.partial;
   a.lohi = b.lohi;
   a.misc = b.misc;
-  if (p.carried_in) {
-    HIP_OK(c, launch_start(c->carry.p, c->carry_flag.p, a, s));
-    HIP_OK(c, launch_keys_hist(c->carry.p, n, p.key_passes, b.sid, b.lohi, b.keys_a, b.hist, s));
+  if (small(p)) {
+    out->keys = b.keys_a;
+    out->perm = b.vals_a;
+    double4* posm = walk_writes_out ? b.posm : nullptr;
+    if (p.carried_in)
+      HIP_OK(c, launch_small_sort(c->carry.p, c->carry_flag.p, a, out->keys, out->perm, b.keys_b, b.vals_b, posm, s));
+    else
+      HIP_OK(c, launch_small_sort(d_in, a, out->keys, out->perm, b.keys_b, b.vals_b, posm, s));
+    if (!walk_writes_out) HIP_OK(c, launch_gather(d_in, d_out, out->perm, b.posm, n, s));
   } else {
-    HIP_OK(c, launch_start(d_in, a, s));
-    HIP_OK(c, launch_keys_hist(d_in, n, p.key_passes, b.sid, b.lohi, b.keys_a, b.hist, s));
+    if (p.carried_in) {
+      HIP_OK(c, launch_start(c->carry.p, c->carry_flag.p, a, s));
+      HIP_OK(c, launch_keys_hist(c->carry.p, n, p.key_passes, b.sid, b.lohi, b.keys_a, b.hist, s));
+    } else {
+      HIP_OK(c, launch_start(d_in, a, s));
+      HIP_OK(c, launch_keys_hist(d_in, n, p.key_passes, b.sid, b.lohi, b.keys_a, b.hist, s));
+    }
+    HIP_OK(c, launch_radix_sort(b.keys_a, b.vals_a, b.keys_b, b.vals_b, n, p.key_passes, p.sid_passes, b.sid, b.hist,
+                                b.lookback, b.lookback + (lb_words - 10), b.misc + kMiscAbort, &out->keys, &out->perm,
+                                s));
+    if (p.carried_in && walk_writes_out)
+      HIP_OK(c, launch_gather(c->carry.p, out->perm, b.posm, n, s));
+    else
+      HIP_OK(c, launch_gather(d_in, walk_writes_out ? nullptr : d_out, out->perm, b.posm, n, s));
   }
-  HIP_OK(c, launch_radix_sort(b.keys_a, b.vals_a, b.keys_b, b.vals_b, n, p.key_passes, p.sid_passes, b.sid, b.hist,
-                              b.lookback, b.lookback + (lb_words - 10), b.misc + kMiscAbort, &out->keys, &out->perm, s));
-  if (p.carried_in && walk_writes_out)
-    HIP_OK(c, launch_gather(c->carry.p, out->perm, b.posm, n, s));
-  else
-    HIP_OK(c, launch_gather(d_in, walk_writes_out ? nullptr : d_out, out->perm, b.posm, n, s));
   HIP_OK(c, launch_tree_count(out->keys, n, b.sid, sys, p.mlx, b.L, b.H, b.tcounts, b.misc, s));
   HIP_OK(c, launch_tree_scan(b.tcounts, tiles, b.tprefix, b.misc + kMiscLevels, s));
   HIP_OK(c, launch_tree_emit(b.L, b.H, n, b.tprefix, b.t, p.depth_plan, s));
@@ -849,7 +866,7 @@ int launch_graph(Ctx* c, const Plan& p, const Scratch& b, const bh_particle* d_i
   for (auto& g : c->graphs)
     if (g.key == key) hit = &g;
   // the sort's output buffers follow from the pass count alone
-  const int passes = p.key_passes + p.sid_passes;
+  const int passes = small(p) ? 0 : p.key_passes + p.sid_passes;
   sorted->keys = (passes % 2 == 0) ? b.keys_a : b.keys_b;
   sorted->perm = (passes % 2 == 0) ? b.vals_a : b.vals_b;
   if (!hit) {

@@ -191,6 +191,14 @@ struct StartArgs {
   uint32_t* misc;
 };
 hipError_t launch_start(const bh_particle* p, const StartArgs& a, hipStream_t s);
+// One system of at most kSmallSort particles: all of that (a.zero's range 0 is
+// misc), its keys, their sort and (posm not null) the walk copy in one launch or,
+// above 1,024 particles, two, with bkeys and bperm between; a.hist, the chunks
+// and a.partial are not used. It orders whole keys, so there is nothing to give
+// up.
+constexpr uint32_t kSmallSort = 12288;
+hipError_t launch_small_sort(const bh_particle* p, const StartArgs& a, uint64_t* keys, uint32_t* perm, uint64_t* bkeys,
+                             uint32_t* bperm, double4* posm, hipStream_t s);
 // The step's last: the report (misc, totals, stamps) to pinned host memory.
 hipError_t launch_report(uint32_t* misc, uint32_t* host, hipStream_t s);
 // Keys, and the histograms of their `passes` leading 8-bit digits.
@@ -201,6 +209,8 @@ hipError_t launch_keys_hist(const bh_particle* p, uint32_t n, int passes, const 
 // read x, y, z (24 of the records' 64 bytes). carried_bad: that walk's
 // non-finite flag, added to misc[kMiscNonfinite].
 hipError_t launch_start(const double* pos, const uint32_t* carried_bad, const StartArgs& a, hipStream_t s);
+hipError_t launch_small_sort(const double* pos, const uint32_t* carried_bad, const StartArgs& a, uint64_t* keys,
+                             uint32_t* perm, uint64_t* bkeys, uint32_t* bperm, double4* posm, hipStream_t s);
 hipError_t launch_keys_hist(const double* pos, uint32_t n, int passes, const uint16_t* sid, const double* lohi,
                             uint64_t* keys, uint32_t* hist, hipStream_t s);
 // key_passes passes over the keys' leading bits, sid_passes (0-2) over the

@@ -111,6 +111,21 @@ __device__ inline void pos_of(const CompactSrc& s, uint32_t i, double* x, double
   *z = s.p[2 * s.n + i];
   *finite = isfinite(*x) && isfinite(*y) && isfinite(*z);
 }
+// x, y, z and mass
+__device__ inline double4 posm_of(const RecordSrc& s, uint32_t i) {
+  const bh_particle& q = s.p[i];
+  return make_double4(q.pos[0], q.pos[1], q.pos[2], q.mass);
+}
+__device__ inline double4 posm_of(const CompactSrc& s, uint32_t i) {
+  return make_double4(s.p[i], s.p[s.n + i], s.p[2 * s.n + i], s.p[3 * s.n + i]);
+}
+
+// The Morton key of a position in the domain whose lowest corner is (lx, ly,
+// lz); scale = cells per unit length.
+__device__ inline uint64_t morton_key(double x, double y, double z, double lx, double ly, double lz, double scale) {
+  return spread_bits3(quantize(x, lx, scale)) | (spread_bits3(quantize(y, ly, scale)) << 1) |
+         (spread_bits3(quantize(z, lz, scale)) << 2);
+}
 
 // A step's first kernel. Small systems wait for each of a step's launches in
 // turn (5 us each), so one takes all that needs nothing but the input: the
@@ -267,8 +282,7 @@ __global__ __launch_bounds__(kBlock) void k_keys_hist(Src src, uint32_t n,
         lz = c[2] - hw;
         have = sys_i;
       }
-      key = spread_bits3(quantize(x, lx, scale)) | (spread_bits3(quantize(y, ly, scale)) << 1) |
-            (spread_bits3(quantize(z, lz, scale)) << 2);
+      key = morton_key(x, y, z, lx, ly, lz, scale);
       keys[i] = key;
     }
     // Input in (or near) Morton order, as a resident step's is, gives long
@@ -604,6 +618,190 @@ __global__ __launch_bounds__(kBlock) void k_gather_pos(const double* __restrict_
   reinterpret_cast<double2*>(posm + k)[half] = make_double2(pos[b0], pos[b0 + n]);
 }
 
+// What k_start, k_bounds_final, the keys, the sort and the gather do, for one
+// system of at most kSmallSort particles: nine launches that each wait for the
+// one before take 5 us apiece, whatever they hold. Block b orders particles
+// [1024 b, 1024 b + 1024) by (key, index), each block from bounds of its own over
+// all particles, and k_small_merge merges the blocks (a single block writes
+// the result itself). The sort is bitonic, on the key's leading 54 bits (18
+// levels) with the index in the block below them, one element per thread, with
+// shuffles inside a wavefront and LDS, two buffers in turn so that a step needs
+// one barrier, beyond. Runs that share the 54 bits are then ordered by the rest
+// of the key (a count over the run).
+//
+// The code runs once a step, from cold instruction caches: loops stay rolled
+// where no load waits in them. (All 4,096 in one workgroup: 48 us, with an
+// unrolled body 53.) Sort phase, nine launches -> here: 1,000 particles 45 -> 20
+// us, 4,096 53 -> 29, 8,192 58 -> 38, 12,000 59 -> 48; 16,384 57 -> 56: the line
+// is at 12,288.
+constexpr int kSmallThreads = 1024;
+constexpr int kSmallBits = 54;  // 64 - 10 for the index in the block
+
+template <typename Src>
+__global__ __launch_bounds__(kSmallThreads) void k_small_sort(Src src, const uint32_t* __restrict__ carried_bad, StartArgs a,
+                                                              uint64_t* __restrict__ keys, uint32_t* __restrict__ perm,
+                                                              double4* __restrict__ posm) {
+  constexpr int kWaves = kSmallThreads / 64;
+  constexpr int kLoads = 4;
+  __shared__ uint64_t s_x[2][kSmallThreads], s_key[kSmallThreads];
+  __shared__ double s_red[6][kWaves];
+  __shared__ double s_lohi[6];
+  stamp(a.misc, kStampStart);
+  const uint32_t t = threadIdx.x, base = blockIdx.x * kSmallThreads;
+  const uint32_t cnt = a.n - base < kSmallThreads ? a.n - base : kSmallThreads;
+  const double inf = __builtin_huge_val();
+  double b[6] = {inf, inf, inf, inf, inf, inf};  // lo, and -hi
+  bool bad = t == 0 && carried_bad && *carried_bad != 0;
+  double mx, my, mz;  // this thread's particle
+  {
+    bool fin;
+    pos_of(src, base + (t < cnt ? t : cnt - 1), &mx, &my, &mz, &fin);
+  }
+#pragma unroll 1
+  for (uint32_t i0 = 0; i0 < a.n; i0 += kLoads * kSmallThreads) {
+    double x[kLoads], y[kLoads], z[kLoads];
+#pragma unroll
+    for (int j = 0; j < kLoads; ++j) {
+      // past the end the last particle again
+      const uint32_t i = i0 + t + j * kSmallThreads;
+      bool fin;
+      if (j > 0 && i0 + j * kSmallThreads >= a.n) {
+        x[j] = x[0];
+        y[j] = y[0];
+        z[j] = z[0];
+        continue;
+      }
+      pos_of(src, i < a.n ? i : a.n - 1, &x[j], &y[j], &z[j], &fin);
+      bad |= !fin;
+    }
+#pragma unroll
+    for (int j = 0; j < kLoads; ++j) {
+      b[0] = fmin(b[0], x[j]);
+      b[1] = fmin(b[1], y[j]);
+      b[2] = fmin(b[2], z[j]);
+      b[3] = fmin(b[3], -x[j]);
+      b[4] = fmin(b[4], -y[j]);
+      b[5] = fmin(b[5], -z[j]);
+    }
+  }
+#pragma unroll 1
+  for (uint32_t i = base + t; i < a.table_quads; i += gridDim.x * kSmallThreads) a.table[i] = a.host_table[i];
+  // misc (range 0) is the first block's, which also writes to it
+#pragma unroll 1
+  for (int k = blockIdx.x ? 1 : 0; k < ZeroRanges::kMax; ++k) {
+    uint32_t* p = a.zero.p[k];
+#pragma unroll 1
+    for (uint64_t i = k ? base + t : t; i < a.zero.n[k]; i += k ? gridDim.x * kSmallThreads : kSmallThreads) p[i] = 0u;
+  }
+  if (t < cnt) a.sid[base + t] = 0;
+#pragma unroll 1
+  for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+    for (int k = 0; k < 6; ++k) b[k] = fmin(b[k], __shfl_xor(b[k], o));
+  if (__lane_id() == 0)
+#pragma unroll
+    for (int k = 0; k < 6; ++k) s_red[k][t >> 6] = b[k];
+  bad = __syncthreads_or(bad);  // and misc is zero
+  if (bad && t == 0 && blockIdx.x == 0) a.misc[kMiscNonfinite] = 1u;
+  if (t < 6) {
+    double v = s_red[t][0];
+#pragma unroll 1
+    for (int q = 1; q < kWaves; ++q) v = fmin(v, s_red[t][q]);
+    if (t >= 3) v = -v;
+    s_lohi[t] = v;
+    if (blockIdx.x == 0) a.lohi[t] = v;
+  }
+  __syncthreads();
+  uint64_t v;
+  {
+    double c[3], hw;
+    domain_from_lohi(s_lohi, c, &hw);
+    const uint64_t key = morton_key(mx, my, mz, c[0] - hw, c[1] - hw, c[2] - hw, 2097152.0 / (2.0 * hw));
+    s_key[t] = key;
+    v = t < cnt ? (key >> (63 - kSmallBits)) << (64 - kSmallBits) | t : ~0ull;
+  }
+  uint32_t turn = 0;
+#pragma unroll 1
+  for (uint32_t k = 2; k <= kSmallThreads; k <<= 1)
+#pragma unroll 1
+    for (uint32_t m = k >> 1; m > 0; m >>= 1) {
+      // the smaller element stays here in the lower half of an ascending
+      // block and in the upper half of a descending one
+      const bool keep_min = ((t & m) == 0) == ((t & k) == 0);
+      uint64_t o;
+      if (m < 64) {
+        o = __shfl_xor(static_cast<unsigned long long>(v), static_cast<int>(m));
+      } else {
+        s_x[turn][t] = v;
+        __syncthreads();
+        o = s_x[turn][t ^ m];
+        turn ^= 1;
+      }
+      v = (v < o) == keep_min ? v : o;
+    }
+  __syncthreads();
+  // the whole key at place t
+  const uint32_t i = static_cast<uint32_t>(v) & (kSmallThreads - 1);
+  const uint64_t key = s_key[i], lead = key >> (63 - kSmallBits);
+  s_x[0][t] = key;
+  __syncthreads();
+  if (t >= cnt) return;
+  uint32_t at = t;
+  if ((t > 0 && s_x[0][t - 1] >> (63 - kSmallBits) == lead) || (t + 1 < cnt && s_x[0][t + 1] >> (63 - kSmallBits) == lead)) {
+    // the run of these leading bits, in input order, starts at r0
+    uint32_t r0 = 0;
+    for (uint32_t q = t; r0 < q;) {
+      const uint32_t mid = (r0 + q) / 2;
+      if (s_x[0][mid] >> (63 - kSmallBits) < lead)
+        r0 = mid + 1;
+      else
+        q = mid;
+    }
+    at = r0;
+    for (uint32_t q = r0; q < cnt && s_x[0][q] >> (63 - kSmallBits) == lead; ++q)
+      at += s_x[0][q] < key || (s_x[0][q] == key && q < t);
+  }
+  keys[base + at] = key;
+  perm[base + at] = base + i;
+  if (posm) posm[base + at] = posm_of(src, base + i);
+}
+
+// Merges the ordered blocks of k_small_sort: an element's place is its own in
+// its block, and in every other block the number of elements that go before it
+// (of equal keys those of earlier blocks).
+template <typename Src>
+__global__ __launch_bounds__(kBlock) void k_small_merge(Src src, uint32_t n, const uint64_t* __restrict__ bkeys,
+                                                        const uint32_t* __restrict__ bperm, uint64_t* __restrict__ keys,
+                                                        uint32_t* __restrict__ perm, double4* __restrict__ posm) {
+  extern __shared__ uint64_t s_k[];  // n
+#pragma unroll 8
+  for (uint32_t i = threadIdx.x; i < n; i += kBlock) s_k[i] = bkeys[i];
+  const uint32_t e = blockIdx.x * kBlock + threadIdx.x, mine = e / kSmallThreads;
+  const uint32_t i = e < n ? bperm[e] : 0u;
+  const double4 q = posm_of(src, i);
+  __syncthreads();
+  if (e >= n) return;
+  const uint64_t key = s_k[e];
+  uint32_t at = e - mine * kSmallThreads;
+#pragma unroll 1
+  for (uint32_t b = 0; b * kSmallThreads < n; ++b) {
+    if (b == mine) continue;
+    uint32_t lo = b * kSmallThreads, hi = n - lo < kSmallThreads ? n : lo + kSmallThreads;
+    const uint32_t first = lo;
+    while (lo < hi) {
+      const uint32_t mid = (lo + hi) / 2;
+      if (s_k[mid] < key || (s_k[mid] == key && b < mine))
+        lo = mid + 1;
+      else
+        hi = mid;
+    }
+    at += lo - first;
+  }
+  keys[at] = key;
+  perm[at] = i;
+  if (posm) posm[at] = q;
+}
+
 // The report, written to pinned host memory by the step itself (no copies
 // back, and the phases' times come with it: no events between them).
 __global__ __launch_bounds__(128) void k_report(uint32_t* __restrict__ misc, uint32_t* __restrict__ host) {
@@ -651,6 +849,33 @@ hipError_t launch_start(const bh_particle* p, const StartArgs& a, hipStream_t s)
 
 hipError_t launch_start(const double* pos, const uint32_t* carried_bad, const StartArgs& a, hipStream_t s) {
   return start(CompactSrc{pos, a.n}, carried_bad, a, s);
+}
+
+namespace {
+template <typename Src>
+hipError_t small_sort(Src src, const uint32_t* carried_bad, const StartArgs& a, uint64_t* keys, uint32_t* perm,
+                      uint64_t* bkeys, uint32_t* bperm, double4* posm, hipStream_t s) {
+  if (a.n == 0 || a.n > kSmallSort || a.n_sys != 1) return hipErrorInvalidValue;
+  const uint32_t blocks = (a.n + kSmallThreads - 1) / kSmallThreads;
+  const bool one = blocks == 1;
+  hipLaunchKernelGGL(k_small_sort<Src>, dim3(blocks), dim3(kSmallThreads), 0, s, src, carried_bad, a, one ? keys : bkeys,
+                     one ? perm : bperm, one ? posm : nullptr);
+  if (!one)
+    hipLaunchKernelGGL(k_small_merge<Src>, dim3((a.n + kBlock - 1) / kBlock), dim3(kBlock), a.n * sizeof(uint64_t), s,
+                       src, a.n, bkeys, bperm,
+                       keys, perm, posm);
+  return hipGetLastError();
+}
+}  // namespace
+
+hipError_t launch_small_sort(const bh_particle* p, const StartArgs& a, uint64_t* keys, uint32_t* perm, uint64_t* bkeys,
+                             uint32_t* bperm, double4* posm, hipStream_t s) {
+  return small_sort(RecordSrc{p}, nullptr, a, keys, perm, bkeys, bperm, posm, s);
+}
+
+hipError_t launch_small_sort(const double* pos, const uint32_t* carried_bad, const StartArgs& a, uint64_t* keys,
+                             uint32_t* perm, uint64_t* bkeys, uint32_t* bperm, double4* posm, hipStream_t s) {
+  return small_sort(CompactSrc{pos, a.n}, carried_bad, a, keys, perm, bkeys, bperm, posm, s);
 }
 
 hipError_t launch_report(uint32_t* misc, uint32_t* host, hipStream_t s) {
