@@ -685,7 +685,6 @@ int enqueue_build(Ctx* c, const Plan& p, const Scratch& b, const bh_particle* d_
                   bool walk_writes_out) {
   hipStream_t s = c->stream;
   const uint32_t n = p.n;
-  const uint32_t tiles = (n + kTreeTile - 1) / kTreeTile;
   const SysDev* sys = reinterpret_cast<const SysDev*>(b.tables);
   const uint64_t lb_words = radix_lookback_words(n);
   StartArgs a{};
@@ -746,8 +745,7 @@ int enqueue_build(Ctx* c, const Plan& p, const Scratch& b, const bh_particle* d_
       HIP_OK(c, launch_gather(d_in, walk_writes_out ? nullptr : d_out, out->perm, b.posm, n, s));
   }
   HIP_OK(c, launch_tree_count(out->keys, n, b.sid, sys, p.mlx, b.L, b.H, b.tcounts, b.misc, s));
-  HIP_OK(c, launch_tree_scan(b.tcounts, tiles, b.tprefix, b.misc + kMiscLevels, s));
-  HIP_OK(c, launch_tree_emit(b.L, b.H, n, b.tprefix, b.t, p.depth_plan, s));
+  HIP_OK(c, launch_tree_emit(b.L, b.H, n, b.tcounts, b.tprefix, b.t, p.depth_plan, s));
   // what the walk needs zeroed and could not be before: unit_lb may lie over
   // tcounts, the queue heads over the look-back words, and the carried flag
   // has been read

@@ -235,13 +235,12 @@ uint64_t radix_lookback_words(uint32_t n);  // 10 passes of look-back words + 10
 hipError_t launch_tree_count(const uint64_t* keys, uint32_t n, const uint16_t* sid, const SysDev* sys,
                              uint32_t max_leaf_max, uint8_t* L, uint8_t* H, uint32_t* tile_counts, uint32_t* misc,
                              hipStream_t s);
-hipError_t launch_tree_scan(const uint32_t* tile_counts, uint32_t tiles, uint32_t* tile_prefix, uint32_t* totals,
-                            hipStream_t s);
 // Numbers the nodes and writes their topology; when the tree has more nodes
 // or leaves than t.cap it writes nothing and sets kAbortNodes, when it is
 // deeper than depth_plan it sets kAbortDepth.
-hipError_t launch_tree_emit(const uint8_t* L, const uint8_t* H, uint32_t n, const uint32_t* tile_prefix, TreeDev t,
-                            uint32_t depth_plan, hipStream_t s);
+// The levels' and the leaves' totals go to misc.
+hipError_t launch_tree_emit(const uint8_t* L, const uint8_t* H, uint32_t n, const uint32_t* tile_counts,
+                            uint32_t* tile_prefix, TreeDev t, uint32_t depth_plan, hipStream_t s);
 // Links, geometry and the upward pass: every leaf in one launch, then the
 // interior nodes of levels depth_plan - 1..0 (one launch per level, each
 // grid-striding over the level's range read on the device; n_sys systems

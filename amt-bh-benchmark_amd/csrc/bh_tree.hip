@@ -264,25 +264,55 @@ __global__ __launch_bounds__(1024) void k_col_scan(const uint32_t* __restrict__ 
 // nodes or leaves than the arrays hold (kAbortNodes; the host grows them and
 // runs the step again); a tree deeper than the upward launches planned is
 // numbered but flagged (kAbortDepth), so the kernels after this one skip it.
+//
+// kScan: cols holds the tiles' counts, and each tile adds them up for itself
+// (the first also for the report); else it holds k_col_scan's prefixes, and the
+// totals are in misc.
+template <bool kScan>
 __global__ __launch_bounds__(kTileThreads) void k_tree_emit(const uint8_t* __restrict__ L, const uint8_t* __restrict__ H,
-                                                            uint32_t n, const uint32_t* __restrict__ tile_prefix,
+                                                            uint32_t n, const uint32_t* __restrict__ cols, uint32_t tiles,
                                                             TreeDev t, uint32_t depth_plan) {
   __shared__ uint32_t s_loff[kLevels + 2];
+  __shared__ uint32_t s_tot[32], s_pre[32];
   __shared__ uint32_t s_wc[kTileWaves][kTreeCols];
   __shared__ uint32_t s_over;
   const uint32_t tile = blockIdx.x, base = tile * kTreeTile;
   const int w = threadIdx.x >> 6, lane = __lane_id();
+  if constexpr (kScan) {
+    constexpr uint32_t kParts = kTileThreads / 32;
+    __shared__ uint32_t s_part[2][kParts][33];
+    const uint32_t col = threadIdx.x & 31u, part = threadIdx.x >> 5;
+    uint32_t all = 0, before = 0;
+    if (col < kTreeCols)
+      for (uint32_t k = part; k < tiles; k += kParts) {
+        const uint32_t v = cols[uint64_t(k) * kTreeCols + col];
+        all += v;
+        before += k < tile ? v : 0u;
+      }
+    s_part[0][part][col] = all;
+    s_part[1][part][col] = before;
+    __syncthreads();
+    if (threadIdx.x < 64) {
+      uint32_t sum = 0;
+      for (uint32_t k = 0; k < kParts; ++k) sum += s_part[part][k][col];
+      (part ? s_pre : s_tot)[col] = sum;
+      if (tile == 0 && part == 0 && col <= kLevels) t.misc[kMiscLevels + col] = sum;
+    }
+  } else if (threadIdx.x <= kLevels) {
+    s_tot[threadIdx.x] = t.misc[kMiscLevels + threadIdx.x];
+    s_pre[threadIdx.x] = cols[uint64_t(tile) * kTreeCols + threadIdx.x];
+  }
+  __syncthreads();
   if (threadIdx.x == 0) {
-    const uint32_t* totals = t.misc + kMiscLevels;
     uint32_t off = 0, deepest = 0;
     for (int d = 0; d < kLevels; ++d) {
       s_loff[d] = off;
-      off += totals[d];
-      if (totals[d]) deepest = static_cast<uint32_t>(d);
+      off += s_tot[d];
+      if (s_tot[d]) deepest = static_cast<uint32_t>(d);
     }
     s_loff[kLevels] = off;
     s_loff[kLevels + 1] = off;
-    const bool over = off > t.cap || totals[kLevels] > t.cap;
+    const bool over = off > t.cap || s_tot[kLevels] > t.cap;
     s_over = over ? 1u : 0u;
     if (tile == 0) {
       t.misc[kMiscMaxDepth] = deepest;
@@ -334,8 +364,8 @@ __global__ __launch_bounds__(kTileThreads) void k_tree_emit(const uint8_t* __res
   // phase 2: global ranks
   uint32_t run[kLevels + 1];
 #pragma unroll
-  for (int d = 0; d < kLevels; ++d) run[d] = s_loff[d] + tile_prefix[uint64_t(tile) * kTreeCols + d] + s_wc[w][d];
-  run[kLevels] = tile_prefix[uint64_t(tile) * kTreeCols + kLevels] + s_wc[w][kLevels];
+  for (int d = 0; d < kLevels; ++d) run[d] = s_loff[d] + s_pre[d] + s_wc[w][d];
+  run[kLevels] = s_pre[kLevels] + s_wc[w][kLevels];
   const uint32_t total_nodes = s_loff[kLevels];
   const uint64_t lt = lanemask_lt();
   nlh = load_lh(0);
@@ -861,17 +891,22 @@ hipError_t launch_tree_count(const uint64_t* keys, uint32_t n, const uint16_t* s
   return hipGetLastError();
 }
 
-hipError_t launch_tree_scan(const uint32_t* tile_counts, uint32_t tiles, uint32_t* tile_prefix, uint32_t* totals,
-                            hipStream_t s) {
-  hipLaunchKernelGGL(k_col_scan, dim3(kLevels + 1), dim3(1024), 0, s, tile_counts, tiles, static_cast<uint32_t>(kTreeCols),
-                     tile_prefix, totals);
-  return hipGetLastError();
-}
+// Up to this many tiles each tile adds up the others' counts itself, a launch
+// less: @@EMIT@@
+constexpr uint32_t kScanTiles = 256;
 
-hipError_t launch_tree_emit(const uint8_t* L, const uint8_t* H, uint32_t n, const uint32_t* tile_prefix, TreeDev t,
-                            uint32_t depth_plan, hipStream_t s) {
+hipError_t launch_tree_emit(const uint8_t* L, const uint8_t* H, uint32_t n, const uint32_t* tile_counts,
+                            uint32_t* tile_prefix, TreeDev t, uint32_t depth_plan, hipStream_t s) {
   const uint32_t tiles = (n + kTreeTile - 1) / kTreeTile;
-  hipLaunchKernelGGL(k_tree_emit, dim3(tiles), dim3(kTileThreads), 0, s, L, H, n, tile_prefix, t, depth_plan);
+  if (tiles <= kScanTiles) {
+    hipLaunchKernelGGL(k_tree_emit<true>, dim3(tiles), dim3(kTileThreads), 0, s, L, H, n, tile_counts, tiles, t,
+                       depth_plan);
+  } else {
+    hipLaunchKernelGGL(k_col_scan, dim3(kLevels + 1), dim3(1024), 0, s, tile_counts, tiles,
+                       static_cast<uint32_t>(kTreeCols), tile_prefix, t.misc + kMiscLevels);
+    hipLaunchKernelGGL(k_tree_emit<false>, dim3(tiles), dim3(kTileThreads), 0, s, L, H, n, tile_prefix, tiles, t,
+                       depth_plan);
+  }
   return hipGetLastError();
 }
 
