@@ -324,10 +324,13 @@ __global__ __launch_bounds__(kTileThreads) void k_tree_emit(const uint8_t* __res
   }
   __syncthreads();
   if (s_over) return;
+  // Lane d holds level d's count (lane kLevels the leaves'), later its running
+  // rank; the levels of an item are gone through bit by bit. (Unrolled over all
+  // 22 levels the kernel was 9.8 KB, fetched from cold caches: tree
+  // phase at 1,000 particles 48.7 -> 44.6 us, 262,144 84.9 -> 79.8.)
+  //
   // phase 1: per-wave counts of level begins and leaf begins
-  uint32_t c[kLevels + 1];
-#pragma unroll
-  for (int d = 0; d <= kLevels; ++d) c[d] = 0;
+  uint32_t cnt = 0;
   // an item's L and H, packed (255 = no particle); the next item's load is
   // issued before the current item's levels are counted
   auto load_lh = [&](int j) -> uint32_t {
@@ -341,16 +344,16 @@ __global__ __launch_bounds__(kTileThreads) void k_tree_emit(const uint8_t* __res
     if (j + 1 < kTileItems) nlh = load_lh(j + 1);
     const int lj = static_cast<int>(lh & 255u), hj = static_cast<int>(lh >> 8);
     // only the levels where some lane begins a node
-    const uint32_t wm = wave_or(level_bits(lj, hj));
-#pragma unroll
-    for (int d = 0; d < kLevels; ++d)
-      if ((wm >> d) & 1u) c[d] += __popcll(__ballot(lj <= d && d <= hj));
-    c[kLevels] += __popcll(__ballot(lj <= hj));
+#pragma unroll 1
+    for (uint32_t wm = wave_or(level_bits(lj, hj)); wm; wm &= wm - 1) {
+      const int d = __ffs(static_cast<int>(wm)) - 1;
+      const uint32_t begins = __popcll(__builtin_amdgcn_ballot_w64(lj <= d && d <= hj));
+      if (lane == d) cnt += begins;
+    }
+    const uint32_t leaves = __popcll(__builtin_amdgcn_ballot_w64(lj <= hj));
+    if (lane == kLevels) cnt += leaves;
   }
-  if (lane == 0) {
-#pragma unroll
-    for (int d = 0; d <= kLevels; ++d) s_wc[w][d] = c[d];
-  }
+  if (lane <= kLevels) s_wc[w][lane] = cnt;
   __syncthreads();
   if (threadIdx.x <= kLevels) {
     uint32_t a = 0;
@@ -362,10 +365,8 @@ __global__ __launch_bounds__(kTileThreads) void k_tree_emit(const uint8_t* __res
   }
   __syncthreads();
   // phase 2: global ranks
-  uint32_t run[kLevels + 1];
-#pragma unroll
-  for (int d = 0; d < kLevels; ++d) run[d] = s_loff[d] + s_pre[d] + s_wc[w][d];
-  run[kLevels] = s_pre[kLevels] + s_wc[w][kLevels];
+  uint32_t run = 0;
+  if (lane <= kLevels) run = (lane < kLevels ? s_loff[lane] : 0u) + s_pre[lane] + s_wc[w][lane];
   const uint32_t total_nodes = s_loff[kLevels];
   const uint64_t lt = lanemask_lt();
   nlh = load_lh(0);
@@ -375,29 +376,24 @@ __global__ __launch_bounds__(kTileThreads) void k_tree_emit(const uint8_t* __res
     const uint32_t lh = nlh;
     if (j + 1 < kTileItems) nlh = load_lh(j + 1);
     const int lj = static_cast<int>(lh & 255u), hj = static_cast<int>(lh >> 8);
-    const uint64_t lm = __ballot(lj <= hj);
-    const uint32_t lr = run[kLevels] + __popcll(lm & lt);
-    run[kLevels] += __popcll(lm);
+    const uint64_t lm = __builtin_amdgcn_ballot_w64(lj <= hj);
+    const uint32_t lr = __builtin_amdgcn_readlane(run, kLevels) + __popcll(lm & lt);
+    if (lane == kLevels) run += __popcll(lm);
     // levels with begins in this wave, and the levels just below them (the
-    // children's start ranks); elsewhere no lane begins a node and a rank is
-    // the running count
+    // children's start ranks): a node of level d - 1 is written with level
+    // d's rank, right after level d - 1's
     const uint32_t wm = wave_or(level_bits(lj, hj));
-    const uint32_t need = wm | (wm << 1);
     uint32_t prev = 0;
-#pragma unroll
-    for (int d = 0; d <= kLevels; ++d) {
-      uint32_t rank;
+#pragma unroll 1
+    for (uint32_t need = wm | (wm << 1); need; need &= need - 1) {
+      const int d = __ffs(static_cast<int>(need)) - 1;
+      uint32_t rank = total_nodes;
       if (d < kLevels) {
-        rank = run[d];
-        if ((need >> d) & 1u) {
-          const uint64_t m = __ballot(lj <= d && d <= hj);
-          rank += __popcll(m & lt);
-          run[d] += __popcll(m);
-        }
-      } else {
-        rank = total_nodes;
+        const uint64_t m = __builtin_amdgcn_ballot_w64(lj <= d && d <= hj);
+        rank = __builtin_amdgcn_readlane(run, d) + __popcll(m & lt);
+        if (lane == d) run += __popcll(m);
       }
-      if (d >= 1 && lj <= d - 1 && d - 1 <= hj) {
+      if (lj <= d - 1 && d - 1 <= hj) {
         const uint32_t node = prev;
         t.begin[node] = idx;
         t.depth[node] = static_cast<uint8_t>(d - 1);
@@ -728,6 +724,8 @@ __global__ __launch_bounds__(kBlock) void k_units_mark(TreeDev t, const uint16_t
                                                        const SysDev* __restrict__ sys, bool grouped,
                                                        uint32_t* __restrict__ tmark, uint32_t* __restrict__ gmark,
                                                        uint32_t* __restrict__ unit_n) {
+  // the children of each thread's node: particles | leaf << 31, first particle
+  __shared__ uint2 s_kid[8][kBlock];
   __shared__ uint32_t s_targets;
   stamp(t.misc, kStampTargets);
   if (t.misc[kMiscAbort]) return;
@@ -741,66 +739,60 @@ __global__ __launch_bounds__(kBlock) void k_units_mark(TreeDev t, const uint16_t
     const uint32_t tsm = q.tsm, tile = q.tile, upiece = q.unit_piece, tpiece = q.target_piece;
     const bool leaf = t.leaf[i] != 0, root = t.depth[i] == 0;
     const bool single = leaf || cnt <= tsm;
-    if (single && (root || t.count[t.parent[i]] > tsm)) {
+    const bool target = single && (root || t.count[t.parent[i]] > tsm);
+    if (target) {
       tmark[b] = i + 1;
       ++mine;
-      if (!grouped) mark_unit(gmark, i, b, cnt, tpiece);
     }
-    if (!grouped) continue;
     const uint32_t thr = max(tsm, tile);
-    if (leaf || cnt <= thr) {
-      if (root) {  // a system that is one walk group
-        unit_n[i] = 0u;
-        mark_unit(gmark, i, b, cnt, single ? tpiece : upiece);
-      }
-      continue;
-    }
-    const uint32_t fc = t.first_child[i], k = t.nchild[i];
-    uint32_t run = 0, run_b = 0, run_len = 0, run_n = 0;
-    auto end_run = [&]() {  // a run is the first child of a unit and what is packed behind it
-      if (run_len == 0) return;
-      unit_n[run] = run_len > 1 ? run_n | 0x80000000u : 0u;
-      mark_unit(gmark, run, run_b, run_n, run_len == 1 ? tpiece : upiece);
-      run_len = 0;
-    };
-    // every child's fields loaded before the first is looked at
-    uint32_t kid_n[8], kid_b[8];
-    uint8_t kid_leaf[8];
+    // the unit being put together: a child and what is packed behind it
+    uint32_t run = i, run_b = b, run_n = cnt, run_len = 0, run_piece = 0, fc = 0, k = 0;
+    bool open = false;  // more may be packed
+    if (!grouped) {
+      run_len = target ? 1 : 0;
+      run_piece = tpiece;
+    } else if (leaf || cnt <= thr) {
+      run_len = root ? 1 : 0;  // a system that is one walk group
+      run_piece = single ? tpiece : upiece;
+    } else {
+      fc = t.first_child[i];
+      k = t.nchild[i];
+      // every child's fields loaded before the first is looked at
+      uint2 kid[8];
 #pragma unroll
-    for (uint32_t j = 0; j < 8; ++j) {
-      const uint32_t c = fc + (j < k ? j : 0u);
-      kid_n[j] = t.count[c];
-      kid_b[j] = t.begin[c];
-      kid_leaf[j] = t.leaf[c];
-    }
-#pragma unroll
-    for (uint32_t j = 0; j < 8; ++j) {
-      if (j >= k) break;
-      const uint32_t c = fc + j, cn = kid_n[j];
-      const bool cleaf = kid_leaf[j] != 0;
-      if (!cleaf && cn > thr) {
-        end_run();
-        continue;
+      for (uint32_t j = 0; j < 8; ++j) {
+        const uint32_t c = fc + (j < k ? j : 0u);
+        kid[j] = make_uint2(t.count[c] | (t.leaf[c] != 0 ? 1u << 31 : 0u), t.begin[c]);
       }
+#pragma unroll
+      for (uint32_t j = 0; j < 8; ++j) s_kid[j][threadIdx.x] = kid[j];
+    }
+    // The last turn only writes the unit in hand. (One place that writes units,
+    // not one per child: with the children's loop unrolled the kernel was 15.8
+    // KB, most of it fetched from cold caches: targets phase at 1,000 particles 12.4 ->
+    // 10.6 us, 262,144 19.5 -> 15.4, 1M 33 -> 30.)
+#pragma unroll 1
+    for (uint32_t j = 0; j <= k; ++j) {
+      const uint2 kid = j < k ? s_kid[j][threadIdx.x] : make_uint2(0u, 0u);
+      const uint32_t c = fc + j, cn = kid.x & 0x7fffffffu;
+      const bool cleaf = (kid.x >> 31) != 0;
       const bool csingle = cleaf || cn <= tsm;
-      if (csingle && cn <= tile && run_len > 0 && run_n + cn <= tile) {
+      if (j < k && open && csingle && run_n + cn <= tile) {
         ++run_len;
         run_n += cn;
         continue;
       }
-      end_run();
-      if (csingle) {
-        run = c;
-        run_b = kid_b[j];
-        run_n = cn;
-        run_len = 1;
-        if (cn > tile) end_run();
-      } else {
-        unit_n[c] = 0u;
-        mark_unit(gmark, c, kid_b[j], cn, upiece);
+      if (run_len > 0) {
+        unit_n[run] = run_len > 1 ? run_n | 0x80000000u : 0u;
+        mark_unit(gmark, run, run_b, run_n, run_len > 1 ? upiece : run_piece);
       }
+      run_len = j < k && (cleaf || cn <= thr) ? 1 : 0;
+      open = csingle && run_len > 0;
+      run = c;
+      run_b = kid.y;
+      run_n = cn;
+      run_piece = csingle ? tpiece : upiece;
     }
-    end_run();
   }
   for (int o = 32; o > 0; o >>= 1) mine += __shfl_xor(mine, o);
   if (__lane_id() == 0 && mine) atomicAdd(&s_targets, mine);
@@ -892,7 +884,8 @@ hipError_t launch_tree_count(const uint64_t* keys, uint32_t n, const uint16_t* s
 }
 
 // Up to this many tiles each tile adds up the others' counts itself, a launch
-// less: @@EMIT@@
+// less (tree phase at 1,000 particles 51.3 -> 48.8 us, 65,536 73.0 -> 70.8, 1M
+// 161.3 -> 159.9; beyond, the tiles' reads of all counts grow with their square).
 constexpr uint32_t kScanTiles = 256;
 
 hipError_t launch_tree_emit(const uint8_t* L, const uint8_t* H, uint32_t n, const uint32_t* tile_counts,
