@@ -160,6 +160,19 @@ __device__ inline double uniform_d(double v) {
   return __builtin_bit_cast(double, (static_cast<uint64_t>(hi) << 32) | lo);
 }
 
+// k_walk's arguments, read again from the kernel's argument segment (its first
+// argument). A field used here and there costs two scalar registers from the
+// kernel's start to its last use, and what does not fit is moved to and from
+// vector registers in the traversal's loop: all but the loop's own fields are
+// read where they are used (spilled scalar registers 112 -> 44; walk of 65,536
+// particles in FP64 0.525 -> 0.515 ms, 250,007 0.88 -> 0.865, 1M 1.325 -> 1.305).
+using LateArgs = const __attribute__((address_space(4))) WalkArgs;
+__device__ inline LateArgs& late_args() {
+  LateArgs* p = (LateArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *p;
+}
+
 // A walk box (FP64): lo x, y, z, hi x, y, z.
 struct Box6 {
   double v[6];
@@ -751,8 +764,8 @@ __device__ inline Box6 particle_box(const WalkArgs& a, uint32_t b, uint32_t n) {
 }
 
 // A node's particle box as computed by the upward pass.
-__device__ inline Box6 node_box(const WalkArgs& a, uint32_t node) {
-  const double* p = a.nbox + 6 * uint64_t(node);
+__device__ inline Box6 node_box(uint32_t node) {
+  const double* p = late_args().nbox + 6 * uint64_t(node);
   Box6 box;
 #pragma unroll
   for (int k = 0; k < 6; ++k) box.v[k] = p[k];
@@ -762,9 +775,10 @@ __device__ inline Box6 node_box(const WalkArgs& a, uint32_t node) {
 // The end of one target particle's walk: its FP64 sums plus the group's
 // share (gacc, when given), times G, to the outputs (grouped_ttg.h:63-66,
 // the update callback) and the fused kick/drift.
-__device__ inline void finish_particle(const WalkArgs& a, uint32_t k3, double ax, double ay, double az,
+__device__ inline void finish_particle(uint32_t k3, double ax, double ay, double az,
                                        const double* gacc, double sys_G, double kick_dt, double drift_dt,
                                        uint32_t n_pp, uint32_t n_pc) {
+  const LateArgs& a = late_args();
   if (gacc) {
     ax += gacc[3 * uint64_t(k3) + 0];
     ay += gacc[3 * uint64_t(k3) + 1];
@@ -824,12 +838,13 @@ __device__ void walk_target(const WalkArgs& a, Lds& L, uint32_t* gfr, uint32_t t
                             const uint32_t* start, uint32_t n_start, const double* gacc, uint32_t g_pp, uint32_t g_pc,
                             unsigned long long& tot_pp, unsigned long long& tot_pc) {
   const int lane = __lane_id();
-  const uint32_t sys_id = uniform(a.sid[tb]);
-  const SysDev& sp = a.sys[sys_id];
+  const LateArgs& la = late_args();
+  const uint32_t sys_id = uniform(la.sid[tb]);
+  const SysDev& sp = la.sys[sys_id];
   const bool use_quad = sp.use_quad != 0;
-  const double4 tcv = a.ctr[tnode];
+  const double4 tcv = la.ctr[tnode];
   const double tcx = tcv.x, tcy = tcv.y, tcz = tcv.z;
-  const Box6 box = node_box(a, tnode);
+  const Box6 box = node_box(tnode);
 
   const int S = kWave / static_cast<int>(T);
   TargetEval<Real, kMask> ev;
@@ -864,7 +879,7 @@ __device__ void walk_target(const WalkArgs& a, Lds& L, uint32_t* gfr, uint32_t t
       ay += red[3 * src + 1];
       az += red[3 * src + 2];
     }
-    finish_particle(a, tb + lane, ax, ay, az, gacc, sp.G, sp.kick_dt, sp.drift_dt, n_pp, n_pc);
+    finish_particle(tb + lane, ax, ay, az, gacc, sp.G, sp.kick_dt, sp.drift_dt, n_pp, n_pc);
   }
   tot_pp += static_cast<unsigned long long>(n_pp) * T;
   tot_pc += static_cast<unsigned long long>(n_pc) * T;
@@ -874,10 +889,10 @@ __device__ void walk_target(const WalkArgs& a, Lds& L, uint32_t* gfr, uint32_t t
 // The target that holds particle p of a unit that starts at particle gb: the
 // last mark at or before p (a unit of several targets spans at most kGroupCap
 // particles).
-__device__ inline uint32_t covering_target(const WalkArgs& a, uint32_t gb, uint32_t p) {
+__device__ inline uint32_t covering_target(uint32_t gb, uint32_t p) {
   for (uint32_t back = 0;; back += kWave) {
     const uint32_t d = back + __lane_id();
-    const uint32_t m = d <= p - gb ? a.tmark[p - d] : 0u;
+    const uint32_t m = d <= p - gb ? late_args().tmark[p - d] : 0u;
     const uint64_t have = ballot(m != 0);
     if (have) return uniform(__builtin_amdgcn_readlane(m, __ffsll(static_cast<long long>(have)) - 1)) - 1u;
     if (back + kWave > p - gb) return 0u;  // not reached: a unit's first particle begins a target
@@ -885,9 +900,9 @@ __device__ inline uint32_t covering_target(const WalkArgs& a, uint32_t gb, uint3
 }
 
 // Where the cut at particle p of such a unit lies.
-__device__ inline uint32_t cut_place(const WalkArgs& a, uint32_t gb, uint32_t p, uint32_t target_piece) {
-  const uint32_t node = covering_target(a, gb, p);
-  const uint32_t b = uniform(a.begin[node]), n = uniform(a.count[node]);
+__device__ inline uint32_t cut_place(uint32_t gb, uint32_t p, uint32_t target_piece) {
+  const uint32_t node = covering_target(gb, p);
+  const uint32_t b = uniform(late_args().begin[node]), n = uniform(late_args().count[node]);
   return b == p || n > target_piece ? p : b + n;
 }
 
@@ -917,17 +932,17 @@ __device__ inline uint32_t cut_place(const WalkArgs& a, uint32_t gb, uint32_t p,
 template <typename Real, bool kMask, typename Lds>
 __device__ void walk_group(const WalkArgs& a, Lds& L, uint32_t slot, uint32_t g, uint32_t p0) {
   const int lane = __lane_id();
-  const uint32_t gb = uniform(a.begin[g]);
+  const uint32_t gb = uniform(late_args().begin[g]);
   // a unit packed from sibling single-target groups spans several nodes
-  const uint32_t un = a.unit_n ? uniform(a.unit_n[g]) : 0u;
+  const uint32_t un = late_args().unit_n ? uniform(late_args().unit_n[g]) : 0u;
   const bool packed = (un >> 31) != 0;
-  const uint32_t G = packed ? un & 0x7fffffffu : uniform(a.count[g]);
-  const uint32_t sys_id = uniform(a.sid[gb]);
-  const SysDev& sp = a.sys[sys_id];
+  const uint32_t G = packed ? un & 0x7fffffffu : uniform(late_args().count[g]);
+  const uint32_t sys_id = uniform(late_args().sid[gb]);
+  const SysDev& sp = late_args().sys[sys_id];
   const bool gleaf = (a.rec[g].count >> 31) != 0;
-  uint32_t* gfr = Lds::kDeepFrames ? a.deep_frames + uint64_t(slot) * (kLevels - Lds::kFrames) * kWave : nullptr;
+  uint32_t* gfr = Lds::kDeepFrames ? late_args().deep_frames + uint64_t(slot) * (kLevels - Lds::kFrames) * kWave : nullptr;
   const bool single = !packed && (gleaf || G <= sp.tsm || G > kGroupCap);
-  uint32_t* dl = a.defer + uint64_t(slot) * kDefer;
+  uint32_t* dl = late_args().defer + uint64_t(slot) * kDefer;
   uint32_t g_pp = 0, g_pc = 0, n_def = 0;
   bool ok = false;  // the group's shared walk kept all its deferred nodes
   unsigned long long tot_pp = 0, tot_pc = 0;
@@ -937,8 +952,8 @@ __device__ void walk_group(const WalkArgs& a, Lds& L, uint32_t slot, uint32_t g,
     const uint32_t len = piece_size(G, single ? sp.target_piece : sp.unit_piece), left = gb + G - p0;
     r1 = p0 + (len < left ? len : left);
     if (!single) {
-      if (r0 > gb) r0 = cut_place(a, gb, r0, sp.target_piece);
-      if (r1 < gb + G) r1 = cut_place(a, gb, r1, sp.target_piece);
+      if (r0 > gb) r0 = cut_place(gb, r0, sp.target_piece);
+      if (r1 < gb + G) r1 = cut_place(gb, r1, sp.target_piece);
       if (r0 >= r1) return;
     }
   }
@@ -961,12 +976,12 @@ __device__ void walk_group(const WalkArgs& a, Lds& L, uint32_t slot, uint32_t g,
       b0 = r1;
     } else {
       if (b0 == r0) {
-        tnode = covering_target(a, gb, r0);
+        tnode = covering_target(gb, r0);
         c = r0 + 1;
       } else {
         while (!bits && c < r1) {
           const uint32_t i = c + lane;
-          m = i < r1 ? a.tmark[i] : 0u;
+          m = i < r1 ? late_args().tmark[i] : 0u;
           bits = ballot(m != 0);
           c += kWave;
         }
@@ -976,13 +991,13 @@ __device__ void walk_group(const WalkArgs& a, Lds& L, uint32_t slot, uint32_t g,
         tnode = uniform(__builtin_amdgcn_readlane(m, j)) - 1u;
       }
       jb = b0;
-      const uint32_t e = uniform(a.begin[tnode]) + uniform(a.count[tnode]);
+      const uint32_t e = uniform(late_args().begin[tnode]) + uniform(late_args().count[tnode]);
       b0 = e < r1 ? e : r1;
       size = b0 - jb;
     }
     const uint32_t* start = ok ? dl : nullptr;
     const uint32_t n_start = ok ? n_def : 0u;
-    const double* gacc = ok ? a.gacc : nullptr;
+    const double* gacc = ok ? late_args().gacc : nullptr;
     const uint32_t jpp = ok ? g_pp : 0u, jpc = ok ? g_pc : 0u;
     if (!is_group && size < kWideMin) {
       walk_target<Real, kMask>(a, L, gfr, tnode, jb, size, start, n_start, gacc, jpp, jpc, tot_pp, tot_pc);
@@ -992,10 +1007,10 @@ __device__ void walk_group(const WalkArgs& a, Lds& L, uint32_t slot, uint32_t g,
     // a packed unit's box and the origin of its relative coordinates (the
     // box centre); a group's or target's: its node box and centre
     const bool pbox = is_group && packed;
-    const Box6 box = pbox ? particle_box(a, gb, G) : node_box(a, tnode);
+    const Box6 box = pbox ? particle_box(a, gb, G) : node_box(tnode);
     const double4 ccv = pbox ? make_double4(0.5 * (box.v[0] + box.v[3]), 0.5 * (box.v[1] + box.v[4]),
                                             0.5 * (box.v[2] + box.v[5]), 0.0)
-                             : a.ctr[tnode];
+                             : late_args().ctr[tnode];
     GroupEval<Real, kMask> ev;
     ev.setup(size, lane);
     ev.eps2 = static_cast<Real>(sp.eps2);
@@ -1044,11 +1059,11 @@ __device__ void walk_group(const WalkArgs& a, Lds& L, uint32_t slot, uint32_t g,
             az += red[3 * src + 2];
           }
           if (is_group) {
-            a.gacc[3 * uint64_t(jb + i) + 0] = ax;
-            a.gacc[3 * uint64_t(jb + i) + 1] = ay;
-            a.gacc[3 * uint64_t(jb + i) + 2] = az;
+            late_args().gacc[3 * uint64_t(jb + i) + 0] = ax;
+            late_args().gacc[3 * uint64_t(jb + i) + 1] = ay;
+            late_args().gacc[3 * uint64_t(jb + i) + 2] = az;
           } else {
-            finish_particle(a, jb + i, ax, ay, az, gacc, sp.G, sp.kick_dt, sp.drift_dt, n_pp, n_pc);
+            finish_particle(jb + i, ax, ay, az, gacc, sp.G, sp.kick_dt, sp.drift_dt, n_pp, n_pc);
           }
         }
         __builtin_amdgcn_wave_barrier();
@@ -1113,7 +1128,7 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(4))
   // lane-0-only claim lets the compiler keep the other lanes looping on
   // their own, with a stale claim).
   const auto claim = [&]() {
-    const uint32_t mine = atomicAdd(&a.queue[kQueueStride * q], __lane_id() == 0 ? 1u : 0u);
+    const uint32_t mine = atomicAdd(&late_args().queue[kQueueStride * q], __lane_id() == 0 ? 1u : 0u);
     return first + uniform(__builtin_amdgcn_readlane(mine, 0));
   };
   uint32_t k = blockIdx.x >> 3;
@@ -1123,7 +1138,7 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(4))
       const uint32_t p = __lane_id() & 7u, n = part(p + 1) - part(p);
       uint32_t left = 0;
       if (n > first) {
-        const uint32_t h = __hip_atomic_load(&a.queue[kQueueStride * p], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const uint32_t h = __hip_atomic_load(&late_args().queue[kQueueStride * p], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         left = h < n - first ? n - first - h : 0u;
       }
       uint32_t most = left << 3 | p;
@@ -1136,13 +1151,13 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(4))
       k = claim();
     }
     if (k >= len) break;
-    const uint2 u = a.units[lo + k];
+    const uint2 u = late_args().units[lo + k];
     walk_group<Real, kMask>(a, L, blockIdx.x, uniform(u.x), uniform(u.y));
     k = claim();
   }
   if (__lane_id() == 0 && (L.tot[0] | L.tot[1]) != 0ull) {
-    atomicAdd(&a.totals[0], L.tot[0]);
-    atomicAdd(&a.totals[1], L.tot[1]);
+    atomicAdd(&late_args().totals[0], L.tot[0]);
+    atomicAdd(&late_args().totals[1], L.tot[1]);
   }
 }
 
