@@ -671,12 +671,15 @@ __global__ __launch_bounds__(kBlock) void k_upward(int level, TreeDev t) {
                gridDim.x * kPer);
 }
 
-// Levels top, top - 1, ... 0 of a single system in one workgroup, one round
-// of teams each: a launch less for every level but one (65,536 particles: tree
-// phase 79 -> 76 us with levels 0-2; with level 3 too, whose 512 nodes take
-// several rounds here and one in a launch of its own, 80).
-constexpr int kTopLevel = 2;  // at most 8^2 = 64 nodes
-constexpr int kTopThreads = 64 * kKids;
+// Levels top, top - 1, ... 0 of a single system in one workgroup: a launch less
+// for every level but one, as long as a level takes few rounds of teams. For all
+// sizes levels 0-2 (at most 64 nodes; 65,536 particles: tree phase 79 -> 76 us,
+// with level 3's 512 nodes too 80), up to 2,048 particles every level (500 and
+// 1,000: 40 -> 35 and 44.5 -> 39.7 us, 2,000: 49.4 -> 45.6; 4,096 would be slower
+// with small leaves: 57 -> 65).
+constexpr int kTopLevel = 2;
+constexpr uint32_t kTopParticles = 2048;
+constexpr int kTopThreads = 1024;
 
 __global__ __launch_bounds__(kTopThreads) void k_upward_top(int top, TreeDev t) {
   constexpr uint32_t kPer = kTopThreads / kKids;
@@ -914,8 +917,8 @@ hipError_t launch_tree_finish(const uint64_t* keys, const double4* posm, uint32_
   hipLaunchKernelGGL(k_upward_leaves, dim3(grid_for(uint64_t(n) * kBlock / kLeafThreads, 8192)), dim3(kLeafThreads), 0, s,
                      posm, n, t);
   const int top = static_cast<int>(depth_plan < kDepthCap ? depth_plan : kDepthCap);
-  // a single system's upper levels (at most 8^kTopLevel nodes) in one launch
-  const int single = n_sys == 1 ? (top - 1 < kTopLevel ? top - 1 : kTopLevel) : -1;
+  const int in_one = n <= kTopParticles || top - 1 < kTopLevel ? top - 1 : kTopLevel;
+  const int single = n_sys == 1 ? in_one : -1;
   for (int d = top - 1; d > single; --d) {
     uint64_t bound = n_sys;
     for (int e = 0; e < d && bound < n; ++e) bound *= 8;
