@@ -98,6 +98,7 @@ struct Plan {
   uint32_t S = 0;         // non-empty systems
   uint32_t n_chunks = 0;  // bounds blocks ...
   uint32_t chunk = kChunk;  // ... of at most this many particles
+  uint32_t sort_tile = kSortTile;  // keys of a radix workgroup
   uint32_t mlx = 0;       // largest max_leaf
   int sid_passes = 0;     // radix passes over the system id
   int key_passes = 8;     // radix passes over the keys' leading bits (8: all of them)
@@ -407,6 +408,8 @@ int plan_systems(Ctx* c, const HostSys* sys, uint32_t S, bool no_grow, Plan* p) 
   *p = Plan{};
   p->n = static_cast<uint32_t>(n);
   p->chunk = chunk;
+  // (the allocation-free step's scratch has room for the larger tiles' words)
+  if (!no_grow) p->sort_tile = sort_tile(p->n);
   p->largest = largest;
   if (n == 0) return BH_OK;
   p->S = live;
@@ -499,7 +502,7 @@ int provision(Ctx* c, const Plan& p, Scratch* b) {
   TRY(ensure(c, c->vals_a, n, "indices"));
   TRY(ensure(c, c->vals_b, n, "indices"));
   TRY(ensure(c, c->hist, 10 * 256, "histograms"));
-  TRY(ensure(c, c->lookback, radix_lookback_words(n), "look-back"));
+  TRY(ensure(c, c->lookback, radix_lookback_words(n, p.sort_tile, 10), "look-back"));
   TRY(ensure(c, c->lohi, 6ull * p.S, "bounds"));
   TRY(ensure(c, c->partial, 6ull * p.n_chunks, "bounds"));
   TRY(ensure(c, c->misc, kReportWords, "flags"));
@@ -619,7 +622,7 @@ bool carve(uint8_t* base, size_t bytes, Plan* p, Scratch* b) {
   s.vals_a = reinterpret_cast<uint32_t*>(take(4ull * n));
   s.vals_b = reinterpret_cast<uint32_t*>(take(4ull * n));
   s.hist = reinterpret_cast<uint32_t*>(take(4 * 10 * 256));
-  s.lookback = reinterpret_cast<uint32_t*>(take(4 * radix_lookback_words(n)));
+  s.lookback = reinterpret_cast<uint32_t*>(take(4 * radix_lookback_words(n, p->sort_tile, 10)));
   s.lohi = reinterpret_cast<double*>(take(48ull * p->S));
   s.partial = reinterpret_cast<double*>(take(48ull * p->n_chunks));
   s.misc = reinterpret_cast<uint32_t*>(take(4 * kReportWords));
@@ -686,7 +689,6 @@ int enqueue_build(Ctx* c, const Plan& p, const Scratch& b, const bh_particle* d_
   hipStream_t s = c->stream;
   const uint32_t n = p.n;
   const SysDev* sys = reinterpret_cast<const SysDev*>(b.tables);
-  const uint64_t lb_words = radix_lookback_words(n);
   StartArgs a{};
   a.host_table = reinterpret_cast<const uint4*>(c->host_tables);
   a.table = reinterpret_cast<uint4*>(b.tables);
@@ -707,7 +709,7 @@ int enqueue_build(Ctx* c, const Plan& p, const Scratch& b, const bh_particle* d_
     a.zero.p[3] = b.hist;
     a.zero.n[3] = 8 * 256;
     a.zero.p[4] = b.lookback;
-    a.zero.n[4] = lb_words;
+    a.zero.n[4] = radix_lookback_words(n, p.sort_tile, p.key_passes + p.sid_passes);
   }
   a.host_chunks = reinterpret_cast<const uint4*>(c->host_tables + p.off_chunks);
   a.chunk_first = reinterpret_cast<const uint32_t*>(b.tables + p.off_first);
@@ -736,9 +738,8 @@ int enqueue_build(Ctx* c, const Plan& p, const Scratch& b, const bh_particle* d_
       HIP_OK(c, launch_start(d_in, a, s));
       HIP_OK(c, launch_keys_hist(d_in, n, p.key_passes, b.sid, b.lohi, b.keys_a, b.hist, s));
     }
-    HIP_OK(c, launch_radix_sort(b.keys_a, b.vals_a, b.keys_b, b.vals_b, n, p.key_passes, p.sid_passes, b.sid, b.hist,
-                                b.lookback, b.lookback + (lb_words - 10), b.misc + kMiscAbort, &out->keys, &out->perm,
-                                s));
+    HIP_OK(c, launch_radix_sort(b.keys_a, b.vals_a, b.keys_b, b.vals_b, n, p.sort_tile, p.key_passes, p.sid_passes, b.sid,
+                                b.hist, b.lookback, b.misc + kMiscAbort, &out->keys, &out->perm, s));
     if (p.carried_in && walk_writes_out)
       HIP_OK(c, launch_gather(c->carry.p, out->perm, b.posm, n, s));
     else

@@ -13,7 +13,7 @@ constexpr int kWave = 64;
 constexpr int kDepthCap = 21;           // flat_tree.h:102 (21 octal digits)
 constexpr int kLevels = kDepthCap + 1;  // depths 0..21
 constexpr uint32_t kMaxLeafCap = 1024;  // halo of the tree-build tile
-constexpr uint32_t kSortTile = 4096;    // keys per onesweep workgroup
+constexpr uint32_t kSortTile = 4096;    // keys per onesweep workgroup, at most
 constexpr uint32_t kTreeTile = 4096;    // particles per tree-build workgroup
 constexpr int kTreeCols = 24;           // per tile: 22 level counts, leaf count, pad
 
@@ -219,9 +219,9 @@ hipError_t launch_keys_hist(const double* pos, uint32_t n, int passes, const uin
 // (key, index) pairs in place. hist: 10 x 256 digit counts (8-9: the
 // systems). abort: gets kAbortSort when such a run is too long.
 hipError_t launch_radix_sort(uint64_t* keys_a, uint32_t* vals_a, uint64_t* keys_b, uint32_t* vals_b, uint32_t n,
-                             int key_passes, int sid_passes, const uint16_t* sid, const uint32_t* hist,
-                             uint32_t* lookback, uint32_t* tile_counters, uint32_t* abort, uint64_t** keys_out,
-                             uint32_t** vals_out, hipStream_t s);
+                             uint32_t tile, int key_passes, int sid_passes, const uint16_t* sid, const uint32_t* hist,
+                             uint32_t* lookback, uint32_t* abort, uint64_t** keys_out, uint32_t** vals_out,
+                             hipStream_t s);
 // The FP64 walk copy (x, y, z, m) in Morton order; with out, also the
 // Morton-ordered particles (a step's walk writes those itself).
 hipError_t launch_gather(const bh_particle* in, bh_particle* out, const uint32_t* perm, double4* posm, uint32_t n,
@@ -229,7 +229,18 @@ hipError_t launch_gather(const bh_particle* in, bh_particle* out, const uint32_t
 // The same walk copy from a carried compact copy (blocks of n x, y, z and
 // m) in the order perm indexes.
 hipError_t launch_gather(const double* pos, const uint32_t* perm, double4* posm, uint32_t n, hipStream_t s);
-uint64_t radix_lookback_words(uint32_t n);  // 10 passes of look-back words + 10 tile counters
+// A pass's workgroups take `tile` keys, kSortTile or half of it: with few tiles a
+// pass is a chain of latencies, and half the keys shorten it, with many it is
+// bound by memory and a tile's 256 look-back words are overhead (sort phase,
+// 4,096 -> 2,048 keys: 65,536 particles 75.5 -> 67.7 us, 131,072 82 -> 75, 262,144
+// 94 -> 90, 400,000 equal, 1M 171 -> 193).
+inline uint32_t sort_tile(uint32_t n) { return n <= 64 * kSortTile ? kSortTile / 2 : kSortTile; }
+// Tile counters (10 of 64 words, so that rows of look-back words stay aligned),
+// then up to 10 passes' look-back words.
+constexpr uint32_t kSortCounters = 64;
+inline uint64_t radix_lookback_words(uint32_t n, uint32_t tile, int passes) {
+  return kSortCounters + uint64_t(passes) * ((uint64_t(n) + tile - 1) / tile) * 256;
+}
 
 // ---- bh_tree.hip
 hipError_t launch_tree_count(const uint64_t* keys, uint32_t n, const uint16_t* sid, const SysDev* sys,

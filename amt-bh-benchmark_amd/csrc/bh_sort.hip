@@ -334,7 +334,7 @@ __device__ inline uint32_t block_excl_scan(uint32_t v, uint32_t* s_wsum) {
 // (one by one it was most of the pass when all tiles publish together). For
 // large ones the same tile has twice the wavefronts to hide its loads. A pass
 // at 65,536 particles 12 -> 10 us, 1M 22 -> 19, 16M 146 -> 134.
-template <int kMode>
+template <int kMode, uint32_t kTile>
 __global__ __launch_bounds__(kSortThreads) void k_onesweep(const uint64_t* __restrict__ kin,
                                                            const uint32_t* __restrict__ vin, uint64_t* __restrict__ kout,
                                                            uint32_t* __restrict__ vout, uint32_t n, uint32_t shift,
@@ -343,14 +343,14 @@ __global__ __launch_bounds__(kSortThreads) void k_onesweep(const uint64_t* __res
                                                            uint32_t* __restrict__ lookback,
                                                            uint32_t* __restrict__ tile_counter) {
   constexpr int kW = kSortThreads / 64;
-  constexpr int kI = static_cast<int>(kSortTile) / kSortThreads;
-  constexpr uint32_t kPerWave = kSortTile / kW;
+  constexpr int kI = static_cast<int>(kTile) / kSortThreads;
+  constexpr uint32_t kPerWave = kTile / kW;
   constexpr int kWindow = 8;
   __shared__ uint32_t s_hist[kW][256];  // per-wave digit counters, then per-wave exclusive bases
   __shared__ uint32_t s_lexcl[256];     // tile-local exclusive digit offsets
   __shared__ uint32_t s_adj[256];       // global position - local position, per digit
-  __shared__ uint64_t s_k[kSortTile];   // the tile in digit order: keys, then (reused) payloads
-  __shared__ uint8_t s_d[kSortTile];
+  __shared__ uint64_t s_k[kTile];   // the tile in digit order: keys, then (reused) payloads
+  __shared__ uint8_t s_d[kTile];
   uint32_t* s_v = reinterpret_cast<uint32_t*>(s_k);
   __shared__ uint32_t s_w[kW];
   __shared__ uint32_t s_tile;
@@ -361,7 +361,7 @@ __global__ __launch_bounds__(kSortThreads) void k_onesweep(const uint64_t* __res
   for (int i = tid; i < kW * 256; i += kSortThreads) (&s_hist[0][0])[i] = 0;
   __syncthreads();
   const uint32_t tile = s_tile;
-  const uint32_t base = tile * kSortTile;
+  const uint32_t base = tile * kTile;
 
   uint64_t k[kI];
   uint32_t v[kI];
@@ -462,7 +462,7 @@ __global__ __launch_bounds__(kSortThreads) void k_onesweep(const uint64_t* __res
     }
   }
   __syncthreads();
-  const uint32_t tn = n - base < kSortTile ? n - base : kSortTile;
+  const uint32_t tn = n - base < kTile ? n - base : kTile;
   uint32_t g[kI];
 #pragma unroll
   for (int j = 0; j < kI; ++j) {
@@ -914,32 +914,41 @@ hipError_t launch_keys_hist(const double* pos, uint32_t n, int passes, const uin
   return keys_hist(CompactSrc{pos, n}, n, passes, sid, lohi, keys, hist, s);
 }
 
-uint64_t radix_lookback_words(uint32_t n) {
-  const uint64_t tiles = (uint64_t(n) + kSortTile - 1) / kSortTile;
-  return 10 * tiles * 256 + 10;
+namespace {
+template <int kMode>
+void onesweep(uint32_t tile, uint32_t tiles, const uint64_t* kin, const uint32_t* vin, uint64_t* ko, uint32_t* vo, uint32_t n,
+              uint32_t shift, const uint16_t* sid, const uint32_t* hist, uint32_t* lookback, uint32_t* counter,
+              hipStream_t s) {
+  if (tile == kSortTile)
+    hipLaunchKernelGGL((k_onesweep<kMode, kSortTile>), dim3(tiles), dim3(kSortThreads), 0, s, kin, vin, ko, vo, n, shift,
+                       sid, hist, lookback, counter);
+  else
+    hipLaunchKernelGGL((k_onesweep<kMode, kSortTile / 2>), dim3(tiles), dim3(kSortThreads), 0, s, kin, vin, ko, vo, n,
+                       shift, sid, hist, lookback, counter);
 }
+}  // namespace
 
 hipError_t launch_radix_sort(uint64_t* keys_a, uint32_t* vals_a, uint64_t* keys_b, uint32_t* vals_b, uint32_t n,
-                             int key_passes, int sid_passes, const uint16_t* sid, const uint32_t* hist,
-                             uint32_t* lookback, uint32_t* tile_counters, uint32_t* abort, uint64_t** keys_out,
-                             uint32_t** vals_out, hipStream_t s) {
-  const uint32_t tiles = (n + kSortTile - 1) / kSortTile;
+                             uint32_t tile, int key_passes, int sid_passes, const uint16_t* sid, const uint32_t* hist,
+                             uint32_t* lookback, uint32_t* abort, uint64_t** keys_out, uint32_t** vals_out,
+                             hipStream_t s) {
+  if (tile != kSortTile && tile != kSortTile / 2) return hipErrorInvalidValue;
+  const uint32_t tiles = (n + tile - 1) / tile;
   const uint32_t low = key_passes == 8 ? 0u : 63u - 8u * key_passes;  // bits below the radix digits
   uint64_t* kin = keys_a;
   uint32_t* vin = vals_a;
   uint64_t* ko = keys_b;
   uint32_t* vo = vals_b;
   for (int pass = 0; pass < key_passes + sid_passes; ++pass) {
-    uint32_t* lb = lookback + uint64_t(pass) * tiles * 256;
+    uint32_t* lb = lookback + radix_lookback_words(n, tile, pass);
+    uint32_t* counter = lookback + pass;
     if (pass == 0)
-      hipLaunchKernelGGL(k_onesweep<0>, dim3(tiles), dim3(kSortThreads), 0, s, kin, vin, ko, vo, n, low, sid, hist, lb,
-                         tile_counters + pass);
+      onesweep<0>(tile, tiles, kin, vin, ko, vo, n, low, sid, hist, lb, counter, s);
     else if (pass < key_passes)
-      hipLaunchKernelGGL(k_onesweep<1>, dim3(tiles), dim3(kSortThreads), 0, s, kin, vin, ko, vo, n, low + 8u * pass, sid,
-                         hist + pass * 256, lb, tile_counters + pass);
+      onesweep<1>(tile, tiles, kin, vin, ko, vo, n, low + 8u * pass, sid, hist + pass * 256, lb, counter, s);
     else
-      hipLaunchKernelGGL(k_onesweep<2>, dim3(tiles), dim3(kSortThreads), 0, s, kin, vin, ko, vo, n,
-                         8u * (pass - key_passes), sid, hist + (8 + pass - key_passes) * 256, lb, tile_counters + pass);
+      onesweep<2>(tile, tiles, kin, vin, ko, vo, n, 8u * (pass - key_passes), sid, hist + (8 + pass - key_passes) * 256, lb,
+                  counter, s);
     std::swap(kin, ko);
     std::swap(vin, vo);
   }
