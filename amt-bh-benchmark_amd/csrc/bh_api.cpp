@@ -2,14 +2,16 @@
 // device buffers, and the per-step orchestration of the kernels.
 //
 // One step (step_particles, integrate_ttg.h:88-107, grouped branch):
-//   system table upload -> bounds -> keys + digit histograms -> 8 onesweep
-//   radix passes -> gather (Morton-ordered particles + FP64 walk copy) ->
-//   tree counts -> node emit -> links/centres -> upward pass (per level) ->
-//   targets and walk units -> walk with fused kick/drift.
+//   start (system table, zeroing, chunk bounds) -> bounds -> keys + digit
+//   histograms -> onesweep radix passes over the leading bits -> runs of equal
+//   ones -> gather of the FP64 walk copy (one system of at most kSmallSort
+//   particles: one or two launches for all of these) ->
+//   tree counts -> node emit -> links/centres -> upward pass (leaves, levels) ->
+//   targets and walk units -> walk with fused kick/drift -> report.
 // Everything is ordered on the context's stream and nothing in between
 // needs the host: the kernels read the node, level and unit counts on the
-// device. The host waits once, at the end, and reads back one block of flag
-// and count words. The node arrays and the number of upward levels are
+// device. The host waits once, at the end; the last kernel has by then written
+// the flags, counts and phase times to pinned host memory. The node arrays and the number of upward levels are
 // planned from what the context has seen (and from n); a tree that turns out
 // larger or deeper sets an abort word, every kernel after the node count
 // returns at once, and the step runs again with the arrays grown (its input

@@ -255,7 +255,8 @@ hipError_t launch_tree_emit(const uint8_t* L, const uint8_t* H, uint32_t n, cons
 // Links, geometry and the upward pass: every leaf in one launch, then the
 // interior nodes of levels depth_plan - 1..0 (one launch per level, each
 // grid-striding over the level's range read on the device; n_sys systems
-// bound a level's node count by n_sys * 8^d). The first also zeroes `zero`.
+// bound a level's node count by n_sys * 8^d; a single system's upper levels in
+// one launch, all of them for a small one). The first also zeroes `zero`.
 hipError_t launch_tree_finish(const uint64_t* keys, const double4* posm, uint32_t n, const uint16_t* sid, uint32_t n_sys,
                               const double* lohi, uint32_t depth_plan, const ZeroRanges& zero, TreeDev t, hipStream_t s);
 // Marks the walk targets (node + 1 at the first particle in tmark; their

@@ -18,7 +18,7 @@
 // (sort_passes): 32, 40 or 48 bits hold 10 to 16 octree levels, and the keys
 // below them decide only between particles closer together than that. With
 // all 63 bits (p = 8) there is nothing to fix. Each radix pass is a single
-// "onesweep" kernel: a workgroup ranks a 4096-key tile in LDS with wavefront
+// "onesweep" kernel: a workgroup ranks a tile of 4,096 or 2,048 keys in LDS with wavefront
 // ballots, obtains its global digit offsets by decoupled look-back over the
 // preceding tiles, and writes the tile out digit-sorted so stores coalesce.
 #include <utility>

@@ -1,4 +1,4 @@
-// The grouped force walk on CDNA4: one wavefront per walk group.
+// The grouped force walk on CDNA4: one wavefront per walk unit or piece of one.
 //
 // Reference semantics:
 //   targets           grouped_ttg.h:253 (topmost nodes with leaf || count <= target_size)
@@ -27,7 +27,9 @@
 // and far2 are monotone in the box (also in floating point) and near2 <=
 // far2, so a group's accept / reject-for-all is the decision of every
 // target box inside, and a target opens whatever it does not accept
-// (grouped_ttg.h:42-51).
+// (grouped_ttg.h:42-51). A unit of a system too small to fill the GPU is
+// walked by several wavefronts, each for a piece of its particles (the walk
+// itself with the whole unit's box, so the lists are the same).
 //
 // Per iteration a wavefront pops up to 64 nodes of the top frame of its
 // LDS stack (frame d holds child ranges d levels below the walk's start),
@@ -38,8 +40,8 @@
 // FP64, then rounded to the walk precision, so FP32 arithmetic never sees
 // absolute coordinates. Whenever a ring holds a batch it is evaluated. For a
 // target with T particles, lane = (particle p, slice s): each of the
-// S = 64 / T slices takes every S-th entry, so small leaves still use the
-// whole wavefront. FP32 batch sums are accumulated per lane in FP64;
+// S = 64 / T slices takes its share of the entries, so small leaves still use
+// the whole wavefront. FP32 batch sums are accumulated per lane in FP64;
 // slices, the group's share and the target's own list are combined in
 // FP64.
 //
