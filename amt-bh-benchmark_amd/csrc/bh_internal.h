@@ -286,8 +286,14 @@ __host__ __device__ inline uint32_t piece_size(uint32_t cnt, uint32_t piece) {
 hipError_t launch_walk(const WalkArgs& a, uint32_t slots, bool deep, int fp64, bool any_unsoftened, hipStream_t s);
 // dst[i] = (x, y, z, m) of record i
 hipError_t launch_points(const bh_particle* p, uint32_t n, double4* dst, hipStream_t s);
-hipError_t launch_direct(const double4* src, uint32_t n, const uint32_t* tidx, uint32_t m, double eps2, double G,
-                         double* partial, uint32_t splits, double* acc, hipStream_t s);
+// partial[splits * m]: per split sums over the sources [s0, s1) of src, with more
+// added to what is there. Targets tgt[k], or src[tidx[k]] (src[k]) without tgt;
+// tidx[k] (k) is the source that target k leaves out.
+hipError_t launch_direct(const double4* src, uint32_t s0, uint32_t s1, const double4* tgt, const uint32_t* tidx,
+                         uint32_t m, double eps2, double* partial, uint32_t splits, bool more, hipStream_t s);
+// acc[m] = G times the splits' sums
+hipError_t launch_direct_reduce(const double* partial, uint32_t m, uint32_t splits, double G, double* acc,
+                                hipStream_t s);
 uint32_t direct_splits(uint32_t n, uint32_t m);
 // partial[splits * ceil(n/256)]: per (slice, block) sums of m_i * m_j / r_ij over
 // unordered pairs {i, j} (each counted once, from the i of the block)

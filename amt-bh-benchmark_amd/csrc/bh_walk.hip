@@ -1212,21 +1212,29 @@ __device__ __forceinline__ bool tame(const double4& q) {
 // Bound by FP64 issue: 106 cycles per wavefront and source, of which 16 FP64
 // operations and the reciprocal square root take 85-95 (131,072 particles:
 // 27.5 ms with the general form only -> 11.9; 4,096 targets of 1M: 7.8 -> 3.2).
+// The sources are [s0, s1) of all, cut into the launch's splits; with more, the
+// sums go on from those of the sources before. tgt: the targets themselves, or
+// null for those at their indices in src.
 // A target leaves its own source out; only the tiles that hold a source of
 // the wavefront's targets check for it. Eight wavefronts per SIMD hold the
 // whole grid of a small target set at once.
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_direct(const double4* __restrict__ src, uint32_t n, const uint32_t* __restrict__ tidx,
-                                                uint32_t m, double eps2, double* __restrict__ partial, uint32_t splits) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k_direct(const double4* __restrict__ src, uint32_t s0, uint32_t s1,
+                                                const double4* __restrict__ tgt, const uint32_t* __restrict__ tidx,
+                                                uint32_t m, double eps2, double* __restrict__ partial, uint32_t splits,
+                                                bool more) {
   __shared__ double4 s_src[256];
   const uint32_t k = blockIdx.x * 256 + threadIdx.x;
   const uint32_t split = blockIdx.y;
-  const uint32_t lo = static_cast<uint32_t>(uint64_t(n) * split / splits);
-  const uint32_t hi = static_cast<uint32_t>(uint64_t(n) * (split + 1) / splits);
+  const uint32_t lo = s0 + static_cast<uint32_t>(uint64_t(s1 - s0) * split / splits);
+  const uint32_t hi = s0 + static_cast<uint32_t>(uint64_t(s1 - s0) * (split + 1) / splits);
   const bool ok = k < m;
+  double* o = &partial[(uint64_t(split) * m + k) * 3];
   const uint32_t i = ok ? (tidx ? tidx[k] : k) : 0xffffffffu;
   double4 t = make_double4(0, 0, 0, 0);
-  if (ok) t = src[i];
+  if (ok) t = tgt ? tgt[k] : src[i];
   double a[3] = {0.0, 0.0, 0.0};
+  if (more && ok)
+    for (int c = 0; c < 3; ++c) a[c] = o[c];
   const bool calm = tame(t) && fabs(eps2) < 1e300;
   for (uint32_t b = lo; b < hi; b += 256) {
     const uint32_t e = hi - b < 256 ? hi - b : 256;
@@ -1251,7 +1259,6 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void k
     }
   }
   if (ok) {
-    double* o = &partial[(uint64_t(split) * m + k) * 3];
     o[0] = a[0];
     o[1] = a[1];
     o[2] = a[2];
@@ -1404,10 +1411,17 @@ uint32_t direct_splits(uint32_t n, uint32_t m) {
   return splits;
 }
 
-hipError_t launch_direct(const double4* src, uint32_t n, const uint32_t* tidx, uint32_t m, double eps2, double G,
-                         double* partial, uint32_t splits, double* acc, hipStream_t s) {
+hipError_t launch_direct(const double4* src, uint32_t s0, uint32_t s1, const double4* tgt, const uint32_t* tidx,
+                         uint32_t m, double eps2, double* partial, uint32_t splits, bool more, hipStream_t s) {
   if (m == 0) return hipSuccess;
-  hipLaunchKernelGGL(k_direct, dim3((m + 255) / 256, splits), dim3(256), 0, s, src, n, tidx, m, eps2, partial, splits);
+  hipLaunchKernelGGL(k_direct, dim3((m + 255) / 256, splits), dim3(256), 0, s, src, s0, s1, tgt, tidx, m, eps2, partial,
+                     splits, more);
+  return hipGetLastError();
+}
+
+hipError_t launch_direct_reduce(const double* partial, uint32_t m, uint32_t splits, double G, double* acc,
+                                hipStream_t s) {
+  if (m == 0) return hipSuccess;
   hipLaunchKernelGGL(k_direct_reduce, dim3((m + 255) / 256), dim3(256), 0, s, partial, m, splits, G, acc);
   return hipGetLastError();
 }

@@ -61,3 +61,27 @@ def test_records_loaded_in_pieces(gpu):
     print(f"direct n={n}", flush=True)
     ref, size = reference(p, idx, 1e-6)
     assert (np.abs(gpu.direct_sum(p, idx, 1e-6) - ref) <= (n + 16) * 2.0 ** -52 * size).all()
+
+
+@pytest.mark.parametrize("n,m", [(1 << 19, 1), ((1 << 19) + 3, 7), ((1 << 19) + 3, 4096), ((1 << 19) + 3, 4097), ((1 << 20) + 3, 8193)])
+@pytest.mark.parametrize("wild", ["none", "far", "nan"])
+def test_sources_summed_as_they_arrive(gpu, n, m, wild):
+    """Up to n / 128 targets of at least 2^19 particles are summed piece by
+    piece of 2^18 sources; beside that line all sources come first."""
+    p = ic.uniform_cube(n, 5)
+    last = n - 1 if wild == "far" else n - 2
+    if wild == "far":  # in the last piece
+        p["pos"][last] = (1e160, -2e151, 0.0)
+    elif wild == "nan":
+        p["mass"][last] = np.nan
+    edges = [0, (1 << 18) - 1, 1 << 18, (1 << 19) - 1, n - 1, n - 1, n // 3]
+    idx = np.array((edges * (m // len(edges) + 1))[:m], np.uint32)
+    print(f"direct n={n} m={m} {wild}", flush=True)
+    got = gpu.direct_sum(p, idx, 1e-6)
+    first = min(m, len(edges))
+    ref, size = reference(p, idx[:first], 1e-6)
+    assert np.array_equal(np.isnan(got[:first]), np.isnan(ref))
+    ok = np.isfinite(ref)
+    assert (np.abs(got[:first] - ref)[ok] <= ((n + 16) * 2.0 ** -52 * size)[ok]).all()
+    for k in range(first, m, 997):  # the same target is the same sum
+        assert np.array_equal(got[k], got[k % len(edges)], equal_nan=True)
