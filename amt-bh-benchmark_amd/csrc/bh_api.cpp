@@ -1861,7 +1861,7 @@ int bh_direct_sum(bh_ctx* h, const bh_particle* host, uint64_t n, const uint32_t
       }
   std::unique_ptr<double4[]> xt;
   if (direct_in_pieces(idx, n, m) && side_streams(c)) xt.reset(new (std::nothrow) double4[m]);
-  const uint32_t splits = direct_splits(static_cast<uint32_t>(xt ? kDirectPiece : n), static_cast<uint32_t>(m));
+  const uint32_t splits = pair_splits((m + 255) / 256, xt ? kDirectPiece : n, 64);
   const hipStream_t run = xt ? c->side[0] : c->stream;
   TRY(ensure(c, c->didx, m, "direct sum"));
   TRY(ensure(c, c->dpart, 3ull * m * splits, "direct sum"));
@@ -1896,10 +1896,7 @@ int bh_energies(bh_ctx* h, const bh_particle* host, uint64_t n, double G, double
     return BH_ERR_TOO_LARGE;
   }
   const uint32_t blocks = static_cast<uint32_t>((n + 255) / 256);
-  uint32_t splits = blocks ? 2048 / blocks : 1;
-  if (splits < 1) splits = 1;
-  if (splits > 512) splits = 512;
-  while (splits > 1 && n / splits < 256) splits >>= 1;
+  const uint32_t splits = pair_splits(std::max(blocks, 1u), n / 2, 384);
   if (potential) *potential = 0.0;
   const bool pairs = potential && n >= 2;
   // the GPU sums the pairs while the host sums the kinetic energy

@@ -48,6 +48,8 @@
 // No MFMA: the only GEMM-shaped part, the quadrupole's Q.d, is a K = 4
 // product; on gfx950 the FP32 MFMA does not issue beside the VALU, and a
 // bf16-split form would need more registers than four waves per SIMD leave.
+#include <algorithm>
+
 #include "bh_internal.h"
 
 namespace bhk {
@@ -1402,13 +1404,16 @@ hipError_t launch_potential(const double4* src, uint32_t n, double* partial, uin
   return hipGetLastError();
 }
 
-uint32_t direct_splits(uint32_t n, uint32_t m) {
-  const uint32_t tblocks = (m + 255) / 256;
-  uint32_t splits = 2048 / (tblocks ? tblocks : 1);
-  if (splits < 1) splits = 1;
-  if (splits > 512) splits = 512;
-  while (splits > 1 && n / splits < 256) splits >>= 1;
-  return splits;
+uint32_t pair_splits(uint64_t blocks, uint64_t partners, uint32_t ragged) {
+  // 256 partners a window, down to 64 while there is less than a workgroup per compute unit
+  const uint64_t few = std::min(partners / 64, 256 / blocks);
+  const uint64_t most = std::min<uint64_t>(std::max<uint64_t>({partners / 256, few, 1}), 512);
+  uint64_t best = std::min(std::max<uint64_t>(2048 / blocks, 1), most), cost = ~0ull;
+  for (uint64_t s = best; s <= std::min<uint64_t>(8 * best, most); ++s) {
+    const uint64_t c = (blocks * s + 255) / 256 * ((partners + s - 1) / s + ragged);
+    if (c + c / 64 < cost) best = s, cost = c;
+  }
+  return static_cast<uint32_t>(best);
 }
 
 hipError_t launch_direct(const double4* src, uint32_t s0, uint32_t s1, const double4* tgt, const uint32_t* tidx,

@@ -85,3 +85,22 @@ def test_sources_summed_as_they_arrive(gpu, n, m, wild):
     assert (np.abs(got[:first] - ref)[ok] <= ((n + 16) * 2.0 ** -52 * size)[ok]).all()
     for k in range(first, m, 997):  # the same target is the same sum
         assert np.array_equal(got[k], got[k % len(edges)], equal_nan=True)
+
+
+@pytest.mark.parametrize("n", [2, 3, 63, 64, 65, 127, 128, 129, 500, 1025, 4001, 10001, 20001])
+def test_pair_grids(gpu, n):
+    """The grids of pair sums at sizes where the number of windows changes: the
+    potential energy against numpy's float64 sum and its error bound of n
+    roundings of a sum of terms of one sign, and all targets' accelerations."""
+    p = ic.plummer(n, 7)
+    x, m = p["pos"], p["mass"]
+    pot = 0.0
+    for i in range(n - 1):
+        d = x[i + 1:] - x[i]
+        pot -= m[i] * (m[i + 1:] / np.sqrt((d * d).sum(1))).sum()
+    print(f"pairs n={n}", flush=True)
+    _, got = gpu.energies(p)
+    assert abs(got - pot) <= (n + 16) * 2.0 ** -52 * abs(pot)
+    idx = np.unique([0, n // 2, n - 1])
+    ref, size = reference(p, idx, 1e-4)
+    assert (np.abs(gpu.direct_sum(p, None, 1e-4)[idx] - ref) <= (n + 16) * 2.0 ** -52 * size).all()
