@@ -1111,13 +1111,22 @@ void reference_order(const std::vector<uint32_t>& count, const std::vector<uint8
 // they are, a bounded piece at a time, and the GPU picks the fields: packing
 // them on the host took 9 ns a particle, 7 of 9 ms at 1M.
 constexpr uint64_t kLoadPiece = 1u << 20;
+// A copy of more than 1 MiB from pageable memory takes another path in the
+// runtime, which costs 20 us more than it saves up to 1.5 MiB: two copies there
+// (energies of 17,000 particles 0.280 -> 0.267 ms, 20,000 0.300 -> 0.292; direct
+// sum of 256 over 20,000 0.126 -> 0.112; three copies for 30,000: 0.162 -> 0.186).
+constexpr uint64_t kOneCopy = (1u << 20) / sizeof(bh_particle);
+constexpr uint64_t kTwoCopies = kOneCopy * 3 / 2;
 
 int load_points(Ctx* c, const bh_particle* host, uint64_t n, const char* what) {
   TRY(ensure(c, c->dsrc, n, what));
   TRY(ensure(c, c->drec, std::min(n, kLoadPiece), what));
   for (uint64_t i = 0; i < n; i += kLoadPiece) {
     const uint64_t k = std::min(n - i, kLoadPiece);
-    HIP_OK(c, hipMemcpyAsync(c->drec.p, host + i, k * sizeof(bh_particle), hipMemcpyHostToDevice, c->stream));
+    const uint64_t part = k > kOneCopy && k <= kTwoCopies ? (k + 1) / 2 : k;
+    for (uint64_t j = 0; j < k; j += part)
+      HIP_OK(c, hipMemcpyAsync(c->drec.p + j, host + i + j, std::min(k - j, part) * sizeof(bh_particle),
+                               hipMemcpyHostToDevice, c->stream));
     HIP_OK(c, launch_points(c->drec.p, static_cast<uint32_t>(k), c->dsrc.p + i, c->stream));
   }
   return BH_OK;
@@ -1861,7 +1870,7 @@ int bh_direct_sum(bh_ctx* h, const bh_particle* host, uint64_t n, const uint32_t
       }
   std::unique_ptr<double4[]> xt;
   if (direct_in_pieces(idx, n, m) && side_streams(c)) xt.reset(new (std::nothrow) double4[m]);
-  const uint32_t splits = pair_splits((m + 255) / 256, xt ? kDirectPiece : n, 64);
+  const uint32_t splits = pair_splits((m + 255) / 256, xt ? kDirectPiece : n, 256, 64);
   const hipStream_t run = xt ? c->side[0] : c->stream;
   TRY(ensure(c, c->didx, m, "direct sum"));
   TRY(ensure(c, c->dpart, 3ull * m * splits, "direct sum"));
@@ -1896,7 +1905,7 @@ int bh_energies(bh_ctx* h, const bh_particle* host, uint64_t n, double G, double
     return BH_ERR_TOO_LARGE;
   }
   const uint32_t blocks = static_cast<uint32_t>((n + 255) / 256);
-  const uint32_t splits = pair_splits(std::max(blocks, 1u), n / 2, 384);
+  const uint32_t splits = pair_splits(std::max(blocks, 1u), n / 2, 128, 384);
   if (potential) *potential = 0.0;
   const bool pairs = potential && n >= 2;
   // the GPU sums the pairs while the host sums the kinetic energy

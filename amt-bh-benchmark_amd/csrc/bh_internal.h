@@ -295,16 +295,19 @@ hipError_t launch_direct(const double4* src, uint32_t s0, uint32_t s1, const dou
 hipError_t launch_direct_reduce(const double* partial, uint32_t m, uint32_t splits, double G, double* acc,
                                 hipStream_t s);
 // Into how many windows the partners that each of `blocks` workgroups goes over
-// are split, in the grids of pair sums: up to the 2,048 workgroups that fill
-// the chip's wavefronts or, of up to eight times that, the number with the least
-// work on the compute unit with most (256 share the workgroups; `ragged` partners'
-// time goes with a window's ends; a larger number has to save 1/64, as each split
-// has sums of its own). Only filling the chip left units with a third of the
-// others' work at sizes just over a multiple; ms before -> now:
+// are split, in the grids of pair sums: up to the 2,048 workgroups that fill the
+// chip's wavefronts, with at least `least` partners a window (a quarter of that
+// while no compute unit has two workgroups). Long windows are split further, up
+// to eight times, where that leaves less work on the compute unit with most (256
+// share the workgroups; `ragged` partners' time goes with a window's ends; it has
+// to save 1/64, as each split has sums of its own): only filling the chip left
+// some units a third more than others at sizes just over a multiple. ms:
 //   pairs of (k_potential)   1,000 0.088 -> 0.079   200,000 13.2 -> 11.4   300,001 28.4 -> 24.5
 //                            400,003 49.5 -> 42.5   600,000 100.7 -> 93.4  131,072 equal
 //   all targets (k_direct)   1,000 0.122 -> 0.086   100,003 7.9 -> 7.2     300,000 69.9 -> 59.6
-uint32_t pair_splits(uint64_t blocks, uint64_t partners, uint32_t ragged);
+// (Windows picked that way at 5,000 to 20,000 particles, too, were up to 10%
+// slower: there the ends and the wavefronts a unit has count as much.)
+uint32_t pair_splits(uint64_t blocks, uint64_t partners, uint64_t least, uint32_t ragged);
 // partial[splits * ceil(n/256)]: per (slice, block) sums of m_i * m_j / r_ij over
 // unordered pairs {i, j} (each counted once, from the i of the block)
 hipError_t launch_potential(const double4* src, uint32_t n, double* partial, uint32_t splits, hipStream_t s);

@@ -1404,12 +1404,12 @@ hipError_t launch_potential(const double4* src, uint32_t n, double* partial, uin
   return hipGetLastError();
 }
 
-uint32_t pair_splits(uint64_t blocks, uint64_t partners, uint32_t ragged) {
-  // 256 partners a window, down to 64 while there is less than a workgroup per compute unit
-  const uint64_t few = std::min(partners / 64, 256 / blocks);
-  const uint64_t most = std::min<uint64_t>(std::max<uint64_t>({partners / 256, few, 1}), 512);
-  uint64_t best = std::min(std::max<uint64_t>(2048 / blocks, 1), most), cost = ~0ull;
-  for (uint64_t s = best; s <= std::min<uint64_t>(8 * best, most); ++s) {
+uint32_t pair_splits(uint64_t blocks, uint64_t partners, uint64_t least, uint32_t ragged) {
+  uint64_t best = std::min<uint64_t>(std::max<uint64_t>(2048 / blocks, 1), 512);
+  while (best > 1 && partners / best < (blocks * best > 256 ? least : least / 4)) best >>= 1;
+  uint64_t cost = ~0ull;
+  const uint64_t most = blocks * best < 1024 ? best : std::max(best, std::min(8 * best, partners / 4096));
+  for (uint64_t s = best; s <= most; ++s) {
     const uint64_t c = (blocks * s + 255) / 256 * ((partners + s - 1) / s + ragged);
     if (c + c / 64 < cost) best = s, cost = c;
   }

@@ -87,7 +87,7 @@ def test_sources_summed_as_they_arrive(gpu, n, m, wild):
         assert np.array_equal(got[k], got[k % len(edges)], equal_nan=True)
 
 
-@pytest.mark.parametrize("n", [2, 3, 63, 64, 65, 127, 128, 129, 500, 1025, 4001, 10001, 20001])
+@pytest.mark.parametrize("n", [2, 3, 63, 64, 65, 127, 128, 129, 500, 1025, 4001, 10001, 16384, 16385, 24576, 24577])
 def test_pair_grids(gpu, n):
     """The grids of pair sums at sizes where the number of windows changes: the
     potential energy against numpy's float64 sum and its error bound of n
