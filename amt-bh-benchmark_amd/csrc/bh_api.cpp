@@ -969,6 +969,12 @@ int run(Ctx* c, Plan p, const bh_particle* d_in, bh_particle* d_out, bool walk, 
         set_err(c, "the tree outgrew its planned arrays on every attempt (abort word %u)", abort);
         return BH_ERR_HIP;
       }
+      if (abort & kAbortSort) {
+        // the tree was counted on keys that are not in order: many times the
+        // nodes (1M particles and a far one: 2.9M for 0.2M) and too many levels
+        c->full_sort = true;
+        continue;
+      }
       if (abort & kAbortNodes) {
         uint64_t need = m[kMiscLevels + kLevels];
         uint64_t nodes = 0;
@@ -976,7 +982,6 @@ int run(Ctx* c, Plan p, const bh_particle* d_in, bh_particle* d_out, bool walk, 
         need = std::max(need, nodes);
         c->cap_nodes = static_cast<uint32_t>(std::min<uint64_t>(need + need / 8 + 64, 1ull << 30));
       }
-      if (abort & kAbortSort) c->full_sort = true;
       if (abort & kAbortDepth) {
         c->depth_hint = std::max(c->depth_known ? c->depth_hint : 0u, m[kMiscMaxDepth]);
         c->depth_known = true;
