@@ -489,8 +489,11 @@ __global__ __launch_bounds__(kSortThreads) void k_onesweep(const uint64_t* __res
 // whose keys ascend is done, which equal positions always are. A wavefront
 // takes a run: up to 64 keys are ranked among each other in registers, longer
 // ones key by key against the run in memory, written to the other pair of
-// sort buffers (tk, tv) and copied back. A run of more than kRunCap keys sets
-// kAbortSort: the host runs the step again with full keys.
+// sort buffers (tk, tv) and copied back. A fall in a run of more than kRunCap
+// keys sets kAbortSort: the host runs the step again with full keys.
+// The wavefront looks for one among the run's first kRunCap + 1 keys, each later
+// position's thread at its own (read by one wavefront to its end, a run of
+// 100,000 equal keys among 300,000 took 0.95 of a 1.06 ms sort phase; now 0.12).
 constexpr uint32_t kRunCap = 1024;
 
 __global__ __launch_bounds__(kBlock) void k_fix_runs(uint64_t* keys, uint32_t* vals, uint64_t* tk, uint32_t* tv,
@@ -515,8 +518,14 @@ __global__ __launch_bounds__(kBlock) void k_fix_runs(uint64_t* keys, uint32_t* v
   for (int j = 0; j < kI; ++j) {
     const uint32_t i = base + j * kBlock + threadIdx.x;
     const uint64_t top = k0[j] >> shift;
+    if (i > 0 && i < n && (kp[j] >> shift) == top && sid[i - 1] == sid[i]) {
+      // a fall behind the first kRunCap + 1 keys of a run. (Another workgroup
+      // may be ordering this run, but then it has no key kRunCap places back.)
+      if (kp[j] > k0[j] && i >= kRunCap && (keys[i - kRunCap] >> shift) == top && sid[i - kRunCap] == sid[i])
+        atomicOr(abort, kAbortSort);
+      continue;
+    }
     if (i + 1 >= n || (k1[j] >> shift) != top || sid[i] != sid[i + 1]) continue;
-    if (i > 0 && (kp[j] >> shift) == top && sid[i - 1] == sid[i]) continue;
     s_head[atomicAdd(&s_n, 1u)] = i;  // the first of a run of at least two
   }
   __syncthreads();
@@ -525,10 +534,10 @@ __global__ __launch_bounds__(kBlock) void k_fix_runs(uint64_t* keys, uint32_t* v
     const uint32_t b = s_head[h];
     const uint64_t top = keys[b] >> shift;
     const uint16_t sys = sid[b];
-    // the run's end, and whether it ascends
+    // the run's end, or that it is too long, and whether it ascends
     uint32_t e = b;
     bool sorted = true;
-    for (;;) {
+    while (e - b <= kRunCap) {
       const uint32_t i = e + lane;
       const bool in = i < n && (keys[i] >> shift) == top && sid[i] == sys;
       const uint64_t m = __ballot(!in);

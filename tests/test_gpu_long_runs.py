@@ -1,0 +1,80 @@
+"""Runs of many particles whose keys share the leading bits.
+
+Such a run needs no work where its keys ascend in input order, wherever it is
+that they stop ascending the step has to notice, and neither may cost the time
+of reading the run from one end to the other."""
+import numpy as np
+import pytest
+
+from bhgpu import ic, layout
+from bhgpu import lib as bl
+
+pytestmark = pytest.mark.gpu
+
+FP = layout.force_params(0.7, 1e-2, 1.0, True)
+LOW = 31  # bits below the digits that 12,289 to 32,768 particles are sorted by
+AT = 5000  # where the run's particles lie in the input
+
+
+def line(n, length, swap=()):
+    """n particles of a box of which `length` ascend, two by two, in one cell of
+    the leading bits, with those at the places `swap` changed for each other."""
+    p = ic.random_box(n, 11, 1.0)
+    p["pos"][0], p["pos"][1] = -1.0, 1.0  # the domain: 2^21 cells of 2^-20, 2^11 of them share the bits in x
+    k = np.arange(length) // 2
+    k[list(swap)] = k[list(swap)[::-1]]
+    p["pos"][AT:AT + length] = 0.25 + 2.0 ** -21
+    p["pos"][AT:AT + length, 0] += k * 2.0 ** -20
+    return p
+
+
+def runs(orc, p):
+    """Lengths of the longest run and of the longest that does not ascend, from the oracle's keys."""
+    e = orc.build(p, 16, 256).export()
+    keys = np.zeros(len(p), np.uint64)
+    keys[e["perm"]] = e["keys"]
+    keys = keys[np.argsort(keys >> np.uint64(LOW), kind="stable")]
+    top = keys >> np.uint64(LOW)
+    first = np.r_[True, top[1:] != top[:-1]]
+    length = np.diff(np.r_[np.flatnonzero(first), len(p)])
+    falls = np.add.reduceat(~first & np.r_[False, keys[1:] < keys[:-1]], np.flatnonzero(first)) > 0
+    return length.max(), length[falls].max(initial=0), e
+
+
+def check(orc, p, longest, unsorted, reruns):
+    assert runs(orc, p)[:2] == (longest, unsorted)
+    with bl.Context(0) as gpu:
+        gpu.step(p, FP, 16, 256, 32, 1e-3, 1e-3)
+        assert gpu.last_step_stats().reruns == reruns
+    with bl.Context(0) as gpu:
+        gpu.build_tree(p, 16, 256)
+        ge = gpu.export()
+    oe = runs(orc, p)[2]
+    for k in ("keys", "perm", "particles", "nodes", "center", "iab", "groups"):
+        assert ge[k].tobytes() == oe[k].tobytes(), k
+
+
+# places of the two that fall: at the start, around the 1,024th, behind, at the end
+@pytest.mark.parametrize("swap", [(), (0, 2), (1021, 1023), (1022, 1024), (1023, 1025), (1024, 1026), (1086, 1088),
+                                  (2000, 2500), (2996, 2998)])
+def test_falls_in_a_long_run(orc, swap):
+    print(f"long run, falls at {swap}", flush=True)
+    check(orc, line(20000, 3000, swap), 3000, 3000 if swap else 2, 1 if swap else 0)
+
+
+def test_equal_positions_cost_no_sort_time():
+    # 100,000 of 300,000 at one place: a third of the particles read one after
+    # the other, 64 at a time, takes many times the sort; 3 is room for noise
+    best = {}
+    for same in (0, 100000):
+        p = ic.random_box(300000, 12, 1.0)
+        p["pos"][1000:1000 + same] = 0.3
+        print(f"long run of {same} equal positions", flush=True)
+        with bl.Context(0) as gpu:
+            ms = []
+            for _ in range(4):
+                gpu.step(p, FP, 16, 256, 32, 1e-3, 1e-3)
+                ms.append(gpu.last_step_stats().sort_ms)
+            best[same] = min(ms)
+    print(best, flush=True)
+    assert best[100000] < 3 * best[0], best
