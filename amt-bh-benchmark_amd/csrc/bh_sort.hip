@@ -487,18 +487,19 @@ __global__ __launch_bounds__(kSortThreads) void k_onesweep(const uint64_t* __res
 // Orders the runs of equal leading key bits (key >> shift, within a system)
 // by (key, index). The radix passes left each run in index order, so a run
 // whose keys ascend is done, which equal positions always are. A wavefront
-// takes a run: up to 64 keys are ranked among each other in registers, longer
-// ones key by key against the run in memory, written to the other pair of
-// sort buffers (tk, tv) and copied back. A fall in a run of more than kRunCap
-// keys sets kAbortSort: the host runs the step again with full keys.
-// The wavefront looks for one among the run's first kRunCap + 1 keys, each later
-// position's thread at its own (read by one wavefront to its end, a run of
-// 100,000 equal keys among 300,000 took 0.95 of a 1.06 ms sort phase; now 0.12).
-constexpr uint32_t kRunCap = 1024;
+// takes a run of up to 64 keys and ranks them among each other in registers. A
+// fall in a longer run sets kAbortSort: the host runs the step again with full
+// keys, whose passes take less time than ordering such runs would. (Ranked key
+// by key against the run in memory, up to 1,024 keys: sort phase of 20,000
+// particles in boxes of which runs hold some 600, 743 us; with full keys 73, and
+// 1M 386 against 228.) The wavefront looks for a fall among the run's first 64
+// keys, each later position's thread at its own (read by one wavefront to its
+// end, a run of 100,000 equal keys among 300,000 took 0.95 of a 1.06 ms sort
+// phase; now 0.12).
+constexpr uint32_t kRunCap = kWave;
 
-__global__ __launch_bounds__(kBlock) void k_fix_runs(uint64_t* keys, uint32_t* vals, uint64_t* tk, uint32_t* tv,
-                                                     uint32_t n, uint32_t shift, const uint16_t* __restrict__ sid,
-                                                     uint32_t* __restrict__ abort) {
+__global__ __launch_bounds__(kBlock) void k_fix_runs(uint64_t* keys, uint32_t* vals, uint32_t n, uint32_t shift,
+                                                     const uint16_t* __restrict__ sid, uint32_t* __restrict__ abort) {
   __shared__ uint32_t s_head[kFixTile];
   __shared__ uint32_t s_n;
   const uint32_t base = blockIdx.x * kFixTile;
@@ -519,8 +520,8 @@ __global__ __launch_bounds__(kBlock) void k_fix_runs(uint64_t* keys, uint32_t* v
     const uint32_t i = base + j * kBlock + threadIdx.x;
     const uint64_t top = k0[j] >> shift;
     if (i > 0 && i < n && (kp[j] >> shift) == top && sid[i - 1] == sid[i]) {
-      // a fall behind the first kRunCap + 1 keys of a run. (Another workgroup
-      // may be ordering this run, but then it has no key kRunCap places back.)
+      // a fall behind the first kRunCap keys of a run. (Another workgroup may be
+      // ordering this run, but then it has no key kRunCap places back.)
       if (kp[j] > k0[j] && i >= kRunCap && (keys[i - kRunCap] >> shift) == top && sid[i - kRunCap] == sid[i])
         atomicOr(abort, kAbortSort);
       continue;
@@ -532,56 +533,29 @@ __global__ __launch_bounds__(kBlock) void k_fix_runs(uint64_t* keys, uint32_t* v
   const uint32_t runs = s_n;
   for (uint32_t h = w; h < runs; h += kBlock / 64) {
     const uint32_t b = s_head[h];
-    const uint64_t top = keys[b] >> shift;
     const uint16_t sys = sid[b];
-    // the run's end, or that it is too long, and whether it ascends
-    uint32_t e = b;
-    bool sorted = true;
-    while (e - b <= kRunCap) {
-      const uint32_t i = e + lane;
-      const bool in = i < n && (keys[i] >> shift) == top && sid[i] == sys;
-      const uint64_t m = __ballot(!in);
-      const uint32_t len = m ? static_cast<uint32_t>(__ffsll(static_cast<long long>(m)) - 1) : 64u;
-      const bool falls = in && static_cast<uint32_t>(lane) < len && i > b && keys[i - 1] > keys[i];
-      if (__ballot(falls)) sorted = false;
-      e += len;
-      if (len < 64u) break;
-    }
-    if (sorted) continue;
-    const uint32_t len = e - b;
-    if (len > kRunCap) {
+    // the run's first keys, whether they ascend, and whether there are more
+    const uint32_t i = b + lane;
+    const uint64_t k = i < n ? keys[i] : 0ull;
+    const uint64_t top = __shfl(k, 0) >> shift;
+    const uint64_t out = __ballot(i >= n || (k >> shift) != top || sid[i] != sys);
+    const uint32_t len = out ? static_cast<uint32_t>(__ffsll(static_cast<long long>(out)) - 1) : 64u;
+    const bool in = static_cast<uint32_t>(lane) < len;
+    const uint64_t before = __shfl_up(k, 1);
+    if (!__ballot(in && lane > 0 && before > k)) continue;
+    if (len == kRunCap && b + kRunCap < n && (keys[b + kRunCap] >> shift) == top && sid[b + kRunCap] == sys) {
       if (lane == 0) atomicOr(abort, kAbortSort);
       continue;
     }
-    if (len <= 64u) {
-      const bool in = static_cast<uint32_t>(lane) < len;
-      const uint64_t k = in ? keys[b + lane] : ~0ull;
-      const uint32_t v = in ? vals[b + lane] : ~0u;
-      uint32_t rank = 0;
-      for (uint32_t q = 0; q < len; ++q) {
-        const uint64_t kq = __shfl(k, static_cast<int>(q));
-        rank += kq < k || (kq == k && q < static_cast<uint32_t>(lane)) ? 1u : 0u;
-      }
-      if (in) {
-        keys[b + rank] = k;
-        vals[b + rank] = v;
-      }
-    } else {
-      for (uint32_t c = b + lane; c < e; c += 64) {
-        const uint64_t k = keys[c];
-        uint32_t rank = 0;
-        for (uint32_t q = b; q < e; ++q) {
-          const uint64_t kq = keys[q];
-          rank += kq < k || (kq == k && q < c) ? 1u : 0u;
-        }
-        tk[b + rank] = k;
-        tv[b + rank] = vals[c];
-      }
-      __threadfence_block();
-      for (uint32_t c = b + lane; c < e; c += 64) {
-        keys[c] = tk[c];
-        vals[c] = tv[c];
-      }
+    const uint32_t v = in ? vals[i] : ~0u;
+    uint32_t rank = 0;
+    for (uint32_t q = 0; q < len; ++q) {
+      const uint64_t kq = __shfl(k, static_cast<int>(q));
+      rank += kq < k || (kq == k && q < static_cast<uint32_t>(lane)) ? 1u : 0u;
+    }
+    if (in) {
+      keys[b + rank] = k;
+      vals[b + rank] = v;
     }
   }
 }
@@ -962,8 +936,7 @@ hipError_t launch_radix_sort(uint64_t* keys_a, uint32_t* vals_a, uint64_t* keys_
     std::swap(vin, vo);
   }
   if (low)
-    hipLaunchKernelGGL(k_fix_runs, dim3((n + kFixTile - 1) / kFixTile), dim3(kBlock), 0, s, kin, vin, ko, vo, n, low, sid,
-                       abort);
+    hipLaunchKernelGGL(k_fix_runs, dim3((n + kFixTile - 1) / kFixTile), dim3(kBlock), 0, s, kin, vin, n, low, sid, abort);
   *keys_out = kin;
   *vals_out = vin;
   return hipGetLastError();

@@ -78,3 +78,24 @@ def test_equal_positions_cost_no_sort_time():
             best[same] = min(ms)
     print(best, flush=True)
     assert best[100000] < 3 * best[0], best
+
+
+@pytest.mark.parametrize("n,far", [(20000, 2.0 ** 10), (20000, 2.0 ** 9), (1 << 20, 2.0 ** 10)])
+def test_boxes_of_hundreds_cost_no_sort_time(n, far):
+    # a far particle leaves some hundred keys to each of the sort's boxes;
+    # ordering them by hand took 15 times the sort. Full keys are two to four
+    # more of its six to eight launches
+    best = {}
+    for place in (0.0, far):
+        p = ic.random_box(n, 3, 1.0)
+        if place:
+            p["pos"][-1] = (place, 0.0, 0.0)
+        print(f"boxes n={n} far={place}", flush=True)
+        with bl.Context(0) as gpu:
+            ms = []
+            for _ in range(4):
+                gpu.step(p, FP, 16, 256, 32, 1e-3, 1e-3)
+                ms.append(gpu.last_step_stats().sort_ms)
+            best[place] = min(ms)
+    print(best, flush=True)
+    assert best[far] < 2 * best[0.0], best
