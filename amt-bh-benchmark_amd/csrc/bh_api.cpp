@@ -139,6 +139,12 @@ struct GraphEntry {
 };
 constexpr size_t kGraphCache = 256;
 
+// After a step whose keys shared too many leading bits, so many sort by whole
+// keys before the leading bits are tried again, as a system may lose its far
+// particle and the next one need not have any. A trial that fails costs its
+// sort and tree counts (at 20,000 particles half a step): each doubles the span.
+constexpr uint32_t kFullSteps = 64, kFullStepsMost = 4096;
+
 struct Ctx {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -205,7 +211,8 @@ struct Ctx {
   // plans learnt from earlier steps
   uint32_t cap_nodes = 0;        // node capacity asked for (grow-only)
   bool depth_known = false;
-  bool full_sort = false;        // some step's keys shared too many leading bits
+  uint32_t full_sort = 0;        // steps left that sort by whole keys, as one's shared too many leading bits
+  uint32_t full_span = kFullSteps;  // how many, when the next such step is met
   uint32_t depth_hint = kDepthCap;
 
   std::vector<GraphEntry> graphs;
@@ -494,9 +501,9 @@ uint32_t walk_slots(uint32_t n, uint32_t limit) {
 int sort_passes(uint64_t n) { return n <= 32768 ? 4 : n <= (2u << 20) ? 5 : 6; }
 
 // The plan's sizes that depend on what the context has learnt.
-void plan_shape(Ctx* c, Plan* p, bool walk) {
+void plan_shape(Ctx* c, Plan* p, bool walk, bool full_sort) {
   p->walk = walk;
-  p->key_passes = c->full_sort ? 8 : sort_passes(p->largest);
+  p->key_passes = full_sort ? 8 : sort_passes(p->largest);
   const uint64_t want = std::max<uint64_t>(p->node_estimate, c->cap_nodes);
   p->cap_nodes = static_cast<uint32_t>(std::min<uint64_t>(want, 1ull << 30));
   p->depth_plan = c->depth_known ? c->depth_hint : static_cast<uint32_t>(kDepthCap);
@@ -943,9 +950,11 @@ int run(Ctx* c, Plan p, const bh_particle* d_in, bh_particle* d_out, bool walk, 
   c->have_stats = false;
   c->has_tree = false;
   c->carried_ok = false;
+  bool full_sort = c->full_sort > 0 && !small(p);
+  if (full_sort) --c->full_sort;
   for (int attempt = 0;; ++attempt) {
     c->reruns = static_cast<uint32_t>(attempt);
-    plan_shape(c, &p, walk);
+    plan_shape(c, &p, walk, full_sort);
     Scratch b;
     TRY(provision(c, p, &b));
     Sorted sd;
@@ -972,7 +981,9 @@ int run(Ctx* c, Plan p, const bh_particle* d_in, bh_particle* d_out, bool walk, 
       if (abort & kAbortSort) {
         // the tree was counted on keys that are not in order: many times the
         // nodes (1M particles and a far one: 2.9M for 0.2M) and too many levels
-        c->full_sort = true;
+        full_sort = true;
+        c->full_sort = c->full_span;
+        c->full_span = std::min(2 * c->full_span, kFullStepsMost);
         continue;
       }
       if (abort & kAbortNodes) {
@@ -988,6 +999,7 @@ int run(Ctx* c, Plan p, const bh_particle* d_in, bh_particle* d_out, bool walk, 
       }
       continue;
     }
+    if (!full_sort && !small(p)) c->full_span = kFullSteps;
     // later steps plan for the deepest tree seen
     c->depth_hint = c->depth_known ? std::max(c->depth_hint, m[kMiscMaxDepth]) : m[kMiscMaxDepth];
     c->depth_known = true;
