@@ -49,6 +49,7 @@
 // product; on gfx950 the FP32 MFMA does not issue beside the VALU, and a
 // bf16-split form would need more registers than four waves per SIMD leave.
 #include <algorithm>
+#include <type_traits>
 
 #include "bh_internal.h"
 
@@ -170,8 +171,10 @@ __device__ inline double uniform_d(double v) {
 // vector registers in the traversal's loop: all but the loop's own fields are
 // read where they are used (spilled scalar registers 112 -> 44; walk of 65,536
 // particles in FP64 0.525 -> 0.515 ms, 250,007 0.88 -> 0.865, 1M 1.325 -> 1.305).
+// Only a kernel has the segment's address, so every function on the way from
+// k_walk to here is inlined by force.
 using LateArgs = const __attribute__((address_space(4))) WalkArgs;
-__device__ inline LateArgs& late_args() {
+__device__ __forceinline__ LateArgs& late_args() {
   LateArgs* p = (LateArgs*)__builtin_amdgcn_kernarg_segment_ptr();
   asm volatile("" : "+s"(p));
   return *p;
@@ -768,7 +771,7 @@ __device__ inline Box6 particle_box(const WalkArgs& a, uint32_t b, uint32_t n) {
 }
 
 // A node's particle box as computed by the upward pass.
-__device__ inline Box6 node_box(uint32_t node) {
+__device__ __forceinline__ Box6 node_box(uint32_t node) {
   const double* p = late_args().nbox + 6 * uint64_t(node);
   Box6 box;
 #pragma unroll
@@ -779,7 +782,7 @@ __device__ inline Box6 node_box(uint32_t node) {
 // The end of one target particle's walk: its FP64 sums plus the group's
 // share (gacc, when given), times G, to the outputs (grouped_ttg.h:63-66,
 // the update callback) and the fused kick/drift.
-__device__ inline void finish_particle(uint32_t k3, double ax, double ay, double az,
+__device__ __forceinline__ void finish_particle(uint32_t k3, double ax, double ay, double az,
                                        const double* gacc, double sys_G, double kick_dt, double drift_dt,
                                        uint32_t n_pp, uint32_t n_pc) {
   const LateArgs& a = late_args();
@@ -838,7 +841,7 @@ constexpr uint32_t kWideMin = 33;
 // group's deferred nodes) or from the root with the target's box, then the
 // slices' sums, plus the group's share (gacc, counts g_pp / g_pc) when given.
 template <typename Real, bool kMask, typename Lds>
-__device__ void walk_target(const WalkArgs& a, Lds& L, uint32_t* gfr, uint32_t tnode, uint32_t tb, uint32_t T,
+__device__ __forceinline__ void walk_target(const WalkArgs& a, Lds& L, uint32_t* gfr, uint32_t tnode, uint32_t tb, uint32_t T,
                             const uint32_t* start, uint32_t n_start, const double* gacc, uint32_t g_pp, uint32_t g_pc,
                             unsigned long long& tot_pp, unsigned long long& tot_pc) {
   const int lane = __lane_id();
@@ -893,7 +896,7 @@ __device__ void walk_target(const WalkArgs& a, Lds& L, uint32_t* gfr, uint32_t t
 // The target that holds particle p of a unit that starts at particle gb: the
 // last mark at or before p (a unit of several targets spans at most kGroupCap
 // particles).
-__device__ inline uint32_t covering_target(uint32_t gb, uint32_t p) {
+__device__ __forceinline__ uint32_t covering_target(uint32_t gb, uint32_t p) {
   for (uint32_t back = 0;; back += kWave) {
     const uint32_t d = back + __lane_id();
     const uint32_t m = d <= p - gb ? late_args().tmark[p - d] : 0u;
@@ -904,7 +907,7 @@ __device__ inline uint32_t covering_target(uint32_t gb, uint32_t p) {
 }
 
 // Where the cut at particle p of such a unit lies.
-__device__ inline uint32_t cut_place(uint32_t gb, uint32_t p, uint32_t target_piece) {
+__device__ __forceinline__ uint32_t cut_place(uint32_t gb, uint32_t p, uint32_t target_piece) {
   const uint32_t node = covering_target(gb, p);
   const uint32_t b = uniform(late_args().begin[node]), n = uniform(late_args().count[node]);
   return b == p || n > target_piece ? p : b + n;
@@ -934,7 +937,7 @@ __device__ inline uint32_t cut_place(uint32_t gb, uint32_t p, uint32_t target_pi
 // use the target evaluator. Deferral is off for target jobs (no deferred
 // list): their decisions are accept or open.
 template <typename Real, bool kMask, typename Lds>
-__device__ void walk_group(const WalkArgs& a, Lds& L, uint32_t slot, uint32_t g, uint32_t p0) {
+__device__ __forceinline__ void walk_group(const WalkArgs& a, Lds& L, uint32_t slot, uint32_t g, uint32_t p0) {
   const int lane = __lane_id();
   const uint32_t gb = uniform(late_args().begin[g]);
   // a unit packed from sibling single-target groups spans several nodes
@@ -1131,7 +1134,7 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(4))
   // lane id inside the loop, so all 64 lanes stay together in it (a
   // lane-0-only claim lets the compiler keep the other lanes looping on
   // their own, with a stale claim).
-  const auto claim = [&]() {
+  const auto claim = [&]() __attribute__((always_inline)) {
     const uint32_t mine = atomicAdd(&late_args().queue[kQueueStride * q], __lane_id() == 0 ? 1u : 0u);
     return first + uniform(__builtin_amdgcn_readlane(mine, 0));
   };
@@ -1164,6 +1167,9 @@ __global__ __launch_bounds__(kWaves * 64) __attribute__((amdgpu_waves_per_eu(4))
     atomicAdd(&late_args().totals[1], L.tot[1]);
   }
 }
+
+static_assert(std::is_same<decltype(&k_walk<float, 1, false, false>), void (*)(WalkArgs)>::value,
+              "late_args() reads the kernel's first argument");
 
 __global__ __launch_bounds__(256) void k_points(const bh_particle* __restrict__ p, uint32_t n, double4* __restrict__ dst) {
   const uint32_t i = blockIdx.x * 256 + threadIdx.x;
