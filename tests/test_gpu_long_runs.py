@@ -1,8 +1,9 @@
-"""Runs of many particles whose keys share the leading bits.
+"""Runs of particles whose keys share the leading bits.
 
-Such a run needs no work where its keys ascend in input order, wherever it is
-that they stop ascending the step has to notice, and neither may cost the time
-of reading the run from one end to the other."""
+A run of up to 64 is ordered in registers. A longer one needs no work where its
+keys ascend in input order; wherever it is that they stop ascending, the step
+has to notice and runs again with full keys. Neither may cost the time of
+reading the run from one end to the other."""
 import numpy as np
 import pytest
 
@@ -12,7 +13,6 @@ from bhgpu import lib as bl
 pytestmark = pytest.mark.gpu
 
 FP = layout.force_params(0.7, 1e-2, 1.0, True)
-LOW = 31  # bits below the digits that 12,289 to 32,768 particles are sorted by
 AT = 5000  # where the run's particles lie in the input
 
 
@@ -30,11 +30,12 @@ def line(n, length, swap=()):
 
 def runs(orc, p):
     """Lengths of the longest run and of the longest that does not ascend, from the oracle's keys."""
+    low = np.uint64(31 if len(p) <= 32768 else 23)  # bits below the digits that so many particles are sorted by
     e = orc.build(p, 16, 256).export()
     keys = np.zeros(len(p), np.uint64)
     keys[e["perm"]] = e["keys"]
-    keys = keys[np.argsort(keys >> np.uint64(LOW), kind="stable")]
-    top = keys >> np.uint64(LOW)
+    keys = keys[np.argsort(keys >> low, kind="stable")]
+    top = keys >> low
     first = np.r_[True, top[1:] != top[:-1]]
     length = np.diff(np.r_[np.flatnonzero(first), len(p)])
     falls = np.add.reduceat(~first & np.r_[False, keys[1:] < keys[:-1]], np.flatnonzero(first)) > 0
@@ -99,3 +100,21 @@ def test_boxes_of_hundreds_cost_no_sort_time(n, far):
             best[place] = min(ms)
     print(best, flush=True)
     assert best[far] < 2 * best[0.0], best
+
+
+@pytest.mark.parametrize("n", [13000, 40000])
+@pytest.mark.parametrize("length,reruns", [(40, 0), (63, 0), (64, 0), (65, 1), (66, 1)])
+def test_runs_around_the_limit(orc, n, length, reruns):
+    # 180 runs in falling order, so that many lie across the tiles of 1,024
+    # positions that a workgroup looks at
+    p = ic.random_box(n, 11, 1.0)
+    p["pos"][0], p["pos"][1] = -1.0, 1.0
+    for c in range(180):
+        q = p["pos"][2 + c * length:2 + (c + 1) * length]
+        q[:] = (0.25, -0.75 + c * 2.0 ** -7, 0.25)
+        q += 2.0 ** -21
+        q[:, 0] += np.arange(length)[::-1] // 2 * 2.0 ** -20
+    print(f"run limits n={n} length={length}", flush=True)
+    longest = runs(orc, p)[0]
+    check(orc, p, longest, longest, reruns)
+    assert longest == length
