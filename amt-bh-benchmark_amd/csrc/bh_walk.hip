@@ -279,7 +279,11 @@ __device__ inline void eval_pc(const PcRing<Real>& r, int j0, int n, const Real*
 
 // Evaluator of a target's particles: lane = (particle p, slice s). Batches
 // are summed in walk precision and folded into the lane's FP64 accumulator
-// before it has summed more than kFoldEntries entries.
+// before it has summed more than kFoldEntries entries. (Pieces of targets of
+// 33 to 128 particles come here, too: with twice as many entries a sum, the
+// median error of 4,096 particles at target size 128 was 1.25 times what the
+// group evaluator's sums of one batch gave; now 0.91 times. The walk of 4,096
+// particles at target size 64 takes 143.9 us for it instead of 143.6.)
 //
 // Small targets are bound by latency, not by issue: with 9 particles and 7
 // slices a 48-entry batch is 7 entries per lane, and moving the left-over
@@ -290,7 +294,7 @@ __device__ inline void eval_pc(const PcRing<Real>& r, int j0, int n, const Real*
 template <typename Real, bool kMask>
 struct TargetEval {
   using V4 = typename Vec4T<Real>::T;
-  static constexpr int kFoldEntries = 2 * kBatch<Real>;
+  static constexpr int kFoldEntries = sizeof(Real) == 4 ? kBatch<Real> : 2 * kBatch<Real>;
   // a batch takes all that is staged
   static constexpr bool kTakesAll = true;
   __device__ static inline uint32_t take(uint32_t n) { return n; }
