@@ -119,7 +119,7 @@ struct Plan {
   bool carried_in = false; // the input is the last resident step's output: build from its compact positions
 };
 
-// One workgroup sorts the system.
+// A few workgroups sort the system, one up to 1,024 particles.
 bool small(const Plan& p) { return p.S == 1 && p.n <= kSmallSort; }
 
 // One captured step, keyed by everything its launches depend on.
@@ -330,7 +330,7 @@ int check_args(Ctx* c, uint64_t n, const bh_force_params* fp, uint32_t max_leaf,
 // the rule knows the system alone, not what is stepped with it, so a batch
 // gives each system the bytes of a step alone. The lines lie where a system
 // alone gains most while large batches of such systems, which fill the GPU
-// anyway, take no more than 1% longer than before (walk ms, leaf / target
+// anyway, take no more than 2% longer than before (walk ms, leaf / target
 // size in brackets, one system in whole units -> here; then a batch as it was
 // before the walk's other changes -> here):
 //   1,000 (16/32)    0.294 -> 0.076     2,000 systems 1.94 -> 1.94
@@ -341,10 +341,15 @@ int check_args(Ctx* c, uint64_t n, const bh_force_params* fp, uint32_t max_leaf,
 //   65,536 (32/96)   0.668 -> 0.456        64 systems 8.48 -> 8.45
 //   131,072 (32/96)  0.750 -> 0.591        32 systems 8.76 -> 8.67
 //   250,007 (32/64)  1.229 -> 0.837        16 systems 9.33 -> 9.09
+//   270,000 (32/64)  1.20 -> 0.93          16 systems 9.63 -> 9.51
+//   400,003 (32/64)  1.35 -> 1.21          12 systems 10.59 -> 10.50
+//   500,000 (32/64)  1.58 -> 1.47          16 systems 17.04 -> 17.37
 //   500,000 (16/32)  1.665 -> 1.429        16 systems 18.75 -> 17.62
 //   500,000 (32/96)  1.531 -> 1.466        16 systems 9.39 -> 9.31
 //   1M (32/96) 3.06 -> 2.87; 1M uniform (8/32) 1.43 -> 1.33
-// Above 2M whole units are the fastest (4M: 10.25 against 10.50 at 64).
+// Above 2M whole units are the fastest (4M: 10.25 against 10.50 at 64). With
+// the next class's {64, 64} the three rows of target size 64 would be 1.02, 1.30
+// and 1.56 alone, but 9.29, 10.17 and 16.8 in the batches.
 struct Pieces {
   uint16_t unit, target;
 };

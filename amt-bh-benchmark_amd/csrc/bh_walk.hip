@@ -288,8 +288,8 @@ __device__ inline void eval_pc(const PcRing<Real>& r, int j0, int n, const Real*
 // Small targets are bound by latency, not by issue: with 9 particles and 7
 // slices a 48-entry batch is 7 entries per lane, and moving the left-over
 // entries of the ring to its front took as long as evaluating them. So a
-// batch takes everything that is staged (48 to 111 entries: fewer batches,
-// no move), at any split into slices (Share). 65,536 particles in
+// batch takes everything that is staged (48 to 111 entries, in FP64 22 to 85:
+// fewer batches, no move), at any split into slices (Share). 65,536 particles in
 // 16-particle units, walk 0.282 -> 0.268 ms; 1M uniform 1.58 -> 1.50.
 template <typename Real, bool kMask>
 struct TargetEval {

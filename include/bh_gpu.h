@@ -99,8 +99,8 @@ const char* bh_last_error(const bh_ctx* ctx);
 int bh_set_precision(bh_ctx* ctx, int precision);
 /* Walk schedule (results are the same either way: the interaction lists
  * are identical, sums may round differently): BH_WALK_GROUPED (default) walks
- * once per group of up to 256 particles for the decisions its targets
- * share, then per target; BH_WALK_PER_TARGET walks from the root for
+ * once per unit of up to BH_MAX_WALK_TILE particles for the decisions its
+ * targets share, then per target; BH_WALK_PER_TARGET walks from the root for
  * every target. */
 typedef enum bh_walk_mode { BH_WALK_GROUPED = 0, BH_WALK_PER_TARGET = 1 } bh_walk_mode;
 int bh_set_walk_mode(bh_ctx* ctx, int mode);
@@ -124,7 +124,8 @@ int bh_set_graph_mode(bh_ctx* ctx, int mode);
  * target gets its own walk's interaction list either way; sums may round
  * differently); smaller tiles give small systems more wavefronts, larger
  * ones share more of the walk. (Systems of up to 2M particles are walked in
- * pieces of units too small to be worth a tile, by the system's size alone.)
+ * pieces of units too small to be worth a tile, by the system's size and
+ * min(target_size, group_size) alone.)
  * Applies to the single-system entry points and to batch systems whose
  * walk_tile is 0. */
 #define BH_MIN_WALK_TILE 16u
