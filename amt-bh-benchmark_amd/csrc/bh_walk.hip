@@ -279,7 +279,8 @@ __device__ inline void eval_pc(const PcRing<Real>& r, int j0, int n, const Real*
 
 // Evaluator of a target's particles: lane = (particle p, slice s). Batches
 // are summed in walk precision and folded into the lane's FP64 accumulator
-// before it has summed more than kFoldEntries entries. (Pieces of targets of
+// before it has summed more than kFoldEntries entries (or one batch's, if those
+// are more: 56 of 111 in two slices). (Pieces of targets of
 // 33 to 128 particles come here, too: with twice as many entries a sum, the
 // median error of 4,096 particles at target size 128 was 1.25 times what the
 // group evaluator's sums of one batch gave; now 0.91 times. The walk of 4,096
