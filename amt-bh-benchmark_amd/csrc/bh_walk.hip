@@ -1194,7 +1194,7 @@ __device__ __forceinline__ void direct_term(const double4& t, const double4& q, 
   a[2] += dz * sc;
 }
 
-// The same for a softened distance that cannot overflow: the square root and
+// The same for a softened distance that cannot overflow or underflow: the square root and
 // the division take two thirds of the general form's time, and x^(-3/2) =
 // y^3 (1 - r)^(-3/2), y the hardware reciprocal square root and r = 1 - x y^2,
 // needs eight instructions. The series to r^2 leaves a relative error of order
@@ -1215,10 +1215,15 @@ __device__ __forceinline__ void direct_term_tame(const double4& t, const double4
   a[2] = __builtin_fma(dz, sc, a[2]);
 }
 
-// Coordinates (and softening) whose squared distances stay finite; false for NaN.
-__device__ __forceinline__ bool tame(const double4& q) {
-  return fabs(q.x) < 1e150 && fabs(q.y) < 1e150 && fabs(q.z) < 1e150;
+// Coordinates whose squared distances stay finite and do not underflow either,
+// where the series would make not a number of an infinite pull: of two numbers
+// of 1e-137 or more (or zero) the difference is zero or at least 1e-153. False
+// for NaN.
+__device__ __forceinline__ bool tame(double c) {
+  const double m = fabs(c);
+  return m < 1e150 && (m >= 1e-137 || m == 0.0);
 }
+__device__ __forceinline__ bool tame(const double4& q) { return tame(q.x) && tame(q.y) && tame(q.z); }
 
 // brute_force_accel (brute_force.h:15-28) for targets tidx[0..m) over a
 // slice of the sources; partial sums per slice, reduced in slice order.
